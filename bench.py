@@ -54,21 +54,24 @@ def algorithmic_bytes(m, nblocks, prec_bytes):
 
 def sgs_pass_bytes(m, nsgs, prec_bytes):
     """Bytes the colour passes of one pcfd_sgs call must move, and the pass
-    counts.  A pass over colour c reads its rows' blocks (diagonal + one per
-    neighbour, 25 values each) and moves 15 values per row (b, the
-    neighbours' x, the new x), all in the storage precision.  The library
-    skips a pass that directly follows a pass over the same colour (it would
-    rewrite the same x), so nsgs symmetric sweeps over C colours run
-    2*nsgs*C - (2*nsgs - 1) passes."""
+    counts.  A pass over colour c reads its rows' diagonal blocks and, going
+    forward, their blocks towards lower colours, going backward those towards
+    higher ones (25 values each; the other half's row sums are kept from the
+    pass before), and moves 15 values per row (b, the neighbours' x, the new
+    x), all in the storage precision.  The library skips a pass that directly
+    follows a pass over the same colour (it would rewrite the same x), so nsgs
+    symmetric sweeps over C colours run 2*nsgs*C - (2*nsgs - 1) passes."""
     col, nc = m.colour()
-    deg = np.bincount(np.asarray(m.edges).ravel(), minlength=m.nnode)
-    blocks = np.bincount(col, weights=deg + 1.0, minlength=nc)
+    e = np.asarray(m.edges)
+    a, b = col[e[:, 0]], col[e[:, 1]]
+    lower = np.bincount(np.maximum(a, b), minlength=nc)   # blocks of a colour's rows towards lower colours
+    higher = np.bincount(np.minimum(a, b), minlength=nc)
     rows = np.bincount(col, minlength=nc).astype(float)
     seq = []
     for _ in range(nsgs):
-        seq += list(range(nc)) + list(range(nc - 1, -1, -1))
-    run = [c for k, c in enumerate(seq) if k == 0 or seq[k - 1] != c]
-    nbytes = sum(blocks[c] * 25 * prec_bytes + rows[c] * 15 * prec_bytes for c in run)
+        seq += [(c, lower) for c in range(nc)] + [(c, higher) for c in range(nc - 1, -1, -1)]
+    run = [s for k, s in enumerate(seq) if k == 0 or seq[k - 1][0] != s[0]]
+    nbytes = sum(((half[c] + rows[c]) * 25 + rows[c] * 15) * prec_bytes for c, half in run)
     return float(nbytes), len(run), len(seq)
 
 

@@ -26,11 +26,15 @@ constexpr int kW = 64;       // wavefront width = interleave width of the ELL/SE
 // addresses.
 //
 // SELL (block matrix): rows grouped by colour, within a colour sorted by
-// degree (descending) then id, padded to whole chunks of 64 rows (srow = -1
-// for padding).  Chunk k stores its off-diagonal blocks as
-// [slot][entry 0..24][lane] from sbase[k]*25*64, the diagonal block as
-// [entry][lane] at k*25*64; slot s of a row is its s-th gELL neighbour,
-// scol = -1 for padding.
+// degree, then by the number of neighbours of lower colours (both
+// descending), then id, padded to whole chunks of 64 rows (srow = -1 for
+// padding).  A row's off-diagonal blocks come in two runs of slots: first the
+// blocks towards lower colours (slots 0 .. swidth_lo-1 of the chunk), then
+// those towards higher colours (slots swidth_lo .. swidth-1), each run in
+// gELL order and padded to the chunk's longest; gslot holds the slot of every
+// gELL entry.  Chunk k stores its off-diagonal blocks as [slot][entry
+// 0..24][lane] from sbase[k]*25*64, the diagonal block as [entry][lane] at
+// k*25*64; scol is the neighbour's SELL row, -1 for padding.
 struct Dev {
   // geometry
   double* xyz = nullptr;    // 3 x nnode
@@ -42,6 +46,7 @@ struct Dev {
   int* gbase = nullptr;     // nchunk_g
   int* gcol = nullptr;      // nslot_g*64
   double* gnrm = nullptr;   // 4 x nslot_g*64: canonical (n0->n1) unit normal + |a|
+  int* gslot = nullptr;     // nslot_g*64: SELL slot of the block (node, neighbour) in the node's row
   // half-edges
   int* he_ptr = nullptr;    // nnode+1: half-edges of node i, in half-edge order
   int* he_id = nullptr;     // nbnode
@@ -76,17 +81,21 @@ struct Dev {
   // SELL block matrix
   int* srow = nullptr;      // nrow_pad: node of each padded row (-1 = padding)
   int* swidth = nullptr;    // nchunk_s
+  int* swidth_lo = nullptr; // nchunk_s: slots of the lower-colour run
   int* sbase = nullptr;     // nchunk_s
   int* scol = nullptr;      // nslot_s*64
   double* Md = nullptr;     // nslot_s*64*25 (FP64 mode)
   float* Mf = nullptr;      // nslot_s*64*25 (FP32 mode)
   double* Dd = nullptr;     // nchunk_s*64*25
   float* Df = nullptr;      // nchunk_s*64*25
-  int* piv = nullptr;       // nrow_pad, 3-bit packed row permutation
   double* bsd = nullptr;    // 5 x nrow_pad right-hand side in SELL row order
   float* bsf = nullptr;
-  double* xd = nullptr;     // 5 x nnode AoS correction, FP64 mode
-  float* xf = nullptr;      // 5 x nnode AoS correction, FP32 mode
+  double* xsd = nullptr;    // 5 x nrow_pad AoS correction in SELL row order, the one the sweeps work on
+  float* xsf = nullptr;
+  double* psd = nullptr;    // 5 x nrow_pad partial row sums a pass leaves for the next one over its colour
+  float* psf = nullptr;
+  double* xd = nullptr;     // 5 x nnode AoS correction in node order (a solve's result), FP64 mode
+  float* xf = nullptr;      // the same, FP32 mode
   // reductions
   double* red = nullptr;    // partial sums
   double* red_out = nullptr;
@@ -111,7 +120,7 @@ struct Ctx {
   std::vector<int> color_chunk;  // [ncolor+1] chunk range of each colour
   std::vector<int> h_bc_type;
   // host copies used by downloads
-  std::vector<int> h_row_ptr, h_col, h_srow, h_spos, h_sbase;
+  std::vector<int> h_row_ptr, h_col, h_slot, h_srow, h_spos, h_sbase;
   pcfd_params prm{};
   bool have_params = false;
   int iter = 1;

@@ -32,6 +32,13 @@ void dput(Ctx& c, T** p, const std::vector<T>& h) {
   if (!h.empty()) PCFD_HIP(hipMemcpy(*p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
 }
 
+// zero-filled: the padding rows of a row-order vector stay zero
+template <typename T>
+void dzero(Ctx& c, T** p, size_t n) {
+  dalloc(c, p, n);
+  PCFD_HIP(hipMemset(*p, 0, std::max<size_t>(n, 1) * sizeof(T)));
+}
+
 template <typename T>
 void dfree(T*& p) {
   if (p) (void)hipFree(p);
@@ -45,8 +52,8 @@ void free_all(Ctx& c) {
   dfree(d.jdb); dfree(d.jqb); dfree(d.bc_type); dfree(d.twall); dfree(d.he_nrm); dfree(d.spos);
   dfree(d.qref); dfree(d.q); dfree(d.grad); dfree(d.lim); dfree(d.lim2); dfree(d.edges); dfree(d.clip_flag); dfree(d.clip_cnt);
   dfree(d.clip_off); dfree(d.clip_list); dfree(d.b); dfree(d.dt);
-  dfree(d.srow); dfree(d.swidth); dfree(d.sbase); dfree(d.scol); dfree(d.Md); dfree(d.Mf); dfree(d.Dd);
-  dfree(d.Df); dfree(d.piv); dfree(d.bsd); dfree(d.bsf); dfree(d.xd); dfree(d.xf); dfree(d.red);
+  dfree(d.gslot); dfree(d.srow); dfree(d.swidth); dfree(d.swidth_lo); dfree(d.sbase); dfree(d.scol); dfree(d.Md); dfree(d.Mf); dfree(d.Dd);
+  dfree(d.Df); dfree(d.bsd); dfree(d.bsf); dfree(d.xsd); dfree(d.xsf); dfree(d.psd); dfree(d.psf); dfree(d.xd); dfree(d.xf); dfree(d.red);
   dfree(d.red_out); dfree(d.icount); dfree(d.dt_next); dfree(d.qjac);
   for (hipEvent_t* e : {&c.ev0, &c.ev1, &c.ev2, &c.ev3, &c.ev4, &c.ev5, &c.ev_fork, &c.ev_join}) {
     if (*e) (void)hipEventDestroy(*e);
@@ -97,11 +104,15 @@ void ensure_matrix(Ctx& c) {
     if (!c.d.Df) dalloc(c, &c.d.Df, dg);
     if (!c.d.bsf) dalloc(c, &c.d.bsf, 5 * (size_t)c.nrow_pad);
     if (!c.d.xf) dalloc(c, &c.d.xf, 5 * (size_t)c.nnode);
+    if (!c.d.xsf) dzero(c, &c.d.xsf, 5 * (size_t)c.nrow_pad);
+    if (!c.d.psf) dalloc(c, &c.d.psf, 5 * (size_t)c.nrow_pad);
   } else {
     if (!c.d.Md) dalloc(c, &c.d.Md, off);
     if (!c.d.Dd) dalloc(c, &c.d.Dd, dg);
     if (!c.d.bsd) dalloc(c, &c.d.bsd, 5 * (size_t)c.nrow_pad);
     if (!c.d.xd) dalloc(c, &c.d.xd, 5 * (size_t)c.nnode);
+    if (!c.d.xsd) dzero(c, &c.d.xsd, 5 * (size_t)c.nrow_pad);
+    if (!c.d.psd) dalloc(c, &c.d.psd, 5 * (size_t)c.nrow_pad);
   }
 }
 
@@ -321,44 +332,57 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     int ncol = pcfd_color_nodes(nn, ne, m->edges, colour.data());
     if (ncol < 0) throw std::runtime_error(pcfd_mesh_error());
     c.ncolor = ncol;
+    // neighbours of lower colours of each node
+    std::vector<int> nlow(nn, 0);
+    for (int i = 0; i < nn; ++i)
+      for (int p = row_ptr[i]; p < row_ptr[i + 1]; ++p) nlow[i] += colour[c.h_col[p]] < colour[i];
     std::vector<std::vector<int>> members(ncol);
     for (int i = 0; i < nn; ++i) members[colour[i]].push_back(i);
     std::vector<int> srow;
     c.color_chunk.assign(ncol + 1, 0);
     for (int k = 0; k < ncol; ++k) {
       auto& v = members[k];
-      std::stable_sort(v.begin(), v.end(), [&](int a, int b) { return deg(a) > deg(b); });
+      std::stable_sort(v.begin(), v.end(), [&](int a, int b) {
+        return deg(a) != deg(b) ? deg(a) > deg(b) : nlow[a] > nlow[b];
+      });
       srow.insert(srow.end(), v.begin(), v.end());
       while (srow.size() % kW) srow.push_back(-1);
       c.color_chunk[k + 1] = (int)(srow.size() / kW);
     }
     c.nrow_pad = (int)srow.size();
     c.nchunk_s = c.nrow_pad / kW;
-    std::vector<int> swidth(c.nchunk_s, 0), sbase(c.nchunk_s, 0), spos(nn, -1);
+    std::vector<int> swidth(c.nchunk_s, 0), swidth_lo(c.nchunk_s, 0), sbase(c.nchunk_s, 0), spos(nn, -1);
     slots = 0;
     for (int k = 0; k < c.nchunk_s; ++k) {
-      int w = 0;
+      int wl = 0, wh = 0;
       for (int l = 0; l < kW; ++l) {
         int i = srow[(size_t)k * kW + l];
         if (i >= 0) {
-          w = std::max(w, deg(i));
+          wl = std::max(wl, nlow[i]);
+          wh = std::max(wh, deg(i) - nlow[i]);
           spos[i] = k * kW + l;
         }
       }
-      swidth[k] = w;
+      swidth_lo[k] = wl;
+      swidth[k] = wl + wh;
       sbase[k] = (int)slots;
-      slots += w;
+      slots += wl + wh;
     }
     if (slots * kW * 25 > (1LL << 40)) throw std::runtime_error("pcfd_create: matrix too large");
     c.nslot_s = slots;
-    std::vector<int> scol((size_t)slots * kW, -1);
-    for (int k = 0; k < c.nchunk_s; ++k)
-      for (int l = 0; l < kW; ++l) {
-        int i = srow[(size_t)k * kW + l];
-        if (i < 0) continue;
-        for (int p = row_ptr[i]; p < row_ptr[i + 1]; ++p)
-          scol[((size_t)sbase[k] + (p - row_ptr[i])) * kW + l] = c.h_col[p];
+    std::vector<int> scol((size_t)slots * kW, -1), gslot((size_t)c.nslot_g * kW, -1);
+    c.h_slot.resize(c.nnz);
+    for (int i = 0; i < nn; ++i) {
+      const int r = spos[i], k = r / kW, l = r % kW;
+      int lo = 0, hi = swidth_lo[k];
+      for (int p = row_ptr[i]; p < row_ptr[i + 1]; ++p) {
+        const int j = c.h_col[p];
+        const int s = colour[j] < colour[i] ? lo++ : hi++;
+        c.h_slot[p] = s;
+        gslot[((size_t)gbase[i / kW] + (p - row_ptr[i])) * kW + (i % kW)] = s;
+        scol[((size_t)sbase[k] + s) * kW + l] = spos[j];
       }
+    }
     c.h_srow = srow;
     c.h_spos = spos;
     c.h_sbase = sbase;
@@ -406,10 +430,11 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     dalloc(c, &d.b, 5 * (size_t)nn);
     dalloc(c, &d.dt, (size_t)nn);
     dput(c, &d.srow, srow);
+    dput(c, &d.gslot, gslot);
     dput(c, &d.swidth, swidth);
+    dput(c, &d.swidth_lo, swidth_lo);
     dput(c, &d.sbase, sbase);
     dput(c, &d.scol, scol);
-    dalloc(c, &d.piv, (size_t)c.nrow_pad);
     dalloc(c, &d.red, 6 * (size_t)std::max(nblk(nn), 1024));
     dalloc(c, &d.red_out, 8);
     dalloc(c, &d.icount, 4);
@@ -680,7 +705,7 @@ int pcfd_download_jacobian(pcfd_ctx* ctx, const int* ia, const int* ja, double* 
                   ") is not in the mesh graph";
           return PCFD_ERR_ARG;
         }
-        const size_t s = (size_t)c.h_sbase[k] + (size_t)(f - cb);
+        const size_t s = (size_t)c.h_sbase[k] + (size_t)c.h_slot[c.h_row_ptr[i] + (f - cb)];
         for (int e = 0; e < 25; ++e) out[e] = off[(s * 25 + e) * kW + l];
       }
     }
@@ -713,6 +738,8 @@ int pcfd_sgs(pcfd_ctx* ctx, int nsgs, double* x_out, double* delta) {
     }
     launch_sgs(c, nsgs, delta);
     if (x_out) {
+      // the copy below runs on the null stream, which does not wait for ours
+      PCFD_HIP(hipStreamSynchronize(c.stream));
       std::vector<double> h;
       if (c.prm.precision == PCFD_CHOSEN_FP32) fetch(h, c.d.xf, 5 * (size_t)c.nnode);
       else fetch(h, c.d.xd, 5 * (size_t)c.nnode);

@@ -23,7 +23,7 @@ namespace pcfd {
 struct JacArgs {
   int nnode, ntot, ntag, nbnode, nrow_pad, sym2d;
   double gamma;
-  const int *gwidth, *gbase, *gcol;
+  const int *gwidth, *gbase, *gcol, *gslot;
   const double* gnrm;
   long long gstride;
   const int *he_ptr, *he_id, *he_tag;
@@ -322,7 +322,7 @@ __global__ void __launch_bounds__(kBlock) k_jacobian(JacArgs A, const int* __res
 #pragma unroll
     for (int k = 0; k < 5; ++k) qj[k] = A.q[k * A.ntot + j];
     perturb(qj, c, h, qjP);
-    T* blk = ob + (long long)s * 25 * kW;
+    T* blk = ob + (long long)A.gslot[gi] * 25 * kW;
     // offc: column c of this row's block A[i][j]; dcol: this edge's part of
     // column c of the diagonal block
     double offc[5], dcol[5];
@@ -462,7 +462,7 @@ template <typename T>
 __device__ __forceinline__ void blank_subrow(T* Moff, T* Dg, const int* scol, long long sb, int w, int chunk,
                                              int lane, int sub) {
   for (int s = 0; s < w; ++s) {
-    if (scol[(sb + s) * kW + lane] < 0) break;
+    if (scol[(sb + s) * kW + lane] < 0) continue;  // padding of either run
     T* blk = Moff + (sb + s) * 25 * kW + lane;
 #pragma unroll
     for (int k = 0; k < 5; ++k) blk[(sub * 5 + k) * kW] = (T)0;
@@ -498,10 +498,9 @@ __global__ void __launch_bounds__(kBlock) k_noslip_rows(JacArgs A, const int* __
       blank_subrow(Moff, Dg, scol, sb, w, chunk, lane, 0);
       blank_subrow(Moff, Dg, scol, sb, w, chunk, lane, 4);
       const int nn = A.he_nrm[hh];
-      for (int s = 0; nn >= 0 && s < w; ++s) {
-        const int j = scol[(sb + s) * kW + lane];
-        if (j < 0) break;
-        if (j != nn) continue;
+      const int rn = nn >= 0 ? spos[nn] : -1;
+      for (int s = 0; rn >= 0 && s < w; ++s) {
+        if (scol[(sb + s) * kW + lane] != rn) continue;
         T* blk = Moff + (sb + s) * 25 * kW + lane;
         blk[0 * kW] = (T)-1.0;
         blk[24 * kW] = (T)-1.0;
@@ -517,7 +516,7 @@ __global__ void __launch_bounds__(kBlock) k_noslip_rows(JacArgs A, const int* __
 static JacArgs jac_args(Ctx& c) {
   const pcfd_params& p = c.prm;
   return JacArgs{c.nnode, c.ntot, c.ntag, c.nbnode, c.nrow_pad, p.symmetry2d, p.gamma, c.d.gwidth, c.d.gbase,
-                 c.d.gcol, c.d.gnrm, c.nslot_g * kW, c.d.he_ptr, c.d.he_id, c.d.he_tag, c.d.he_a, c.d.bc_type,
+                 c.d.gcol, c.d.gslot, c.d.gnrm, c.nslot_g * kW, c.d.he_ptr, c.d.he_id, c.d.he_tag, c.d.he_a, c.d.bc_type,
                  c.d.qref, c.d.vol, c.d.dt, c.d.q, c.d.srow, c.d.sbase, c.d.xyz, c.d.twall, c.d.he_nrm, p.viscous,
                  ViscParams{p.gamma, p.re_tilde, p.prandtl, p.prandtl_t, p.sutherland_s, p.symmetry2d},
                  p.flux_type == PCFD_FLUX_ALGEBRAIC ? 1 : 0, p.jac_field_type == 1 ? 1 : 0,
@@ -620,29 +619,29 @@ void jacobian_join(Ctx& c) {
   }
 }
 
-// In-place LU with partial pivoting of each diagonal block (LU,
-// ucs/matrix.h:110-190; PrepareSGS, ucs/crsmatrix.tcc:839-876).  The
-// reference leaves rows in place and addresses them through the pivot
-// vector; here the pivot rows are swapped physically (compile-time register
-// indices, no scratch), which performs the same arithmetic.  Row r of the
-// stored factor is original row perm[r]; perm is packed 3 bits per entry.
+// PrepareSGS (ucs/crsmatrix.tcc:839-876): the reference factors each diagonal
+// block (LU with partial pivoting, ucs/matrix.h:110-190) and every row update
+// solves with the factor.  Here the block is replaced by its inverse, from
+// the same elimination (rows swapped physically: compile-time register
+// indices, no scratch) applied to the unit columns, so a row update is one
+// 5x5 product.  The elimination runs in FP64 for both storage types.
 template <typename T>
-__global__ void __launch_bounds__(kBlock) k_prepare_sgs(int nrow_pad, const int* __restrict__ srow, T* __restrict__ Dg,
-                                                       int* __restrict__ piv) {
+__global__ void __launch_bounds__(kBlock) k_prepare_sgs(int nrow_pad, const int* __restrict__ srow,
+                                                       T* __restrict__ Dg) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= nrow_pad || srow[r] < 0) return;
   T* a = Dg + (long long)(r >> 6) * 25 * kW + (r & 63);
-  T A[25];
+  double A[25];
 #pragma unroll
-  for (int k = 0; k < 25; ++k) A[k] = a[k * kW];
+  for (int k = 0; k < 25; ++k) A[k] = (double)a[k * kW];
   int p[5] = {0, 1, 2, 3, 4};
   int row = 0;  // persists across columns, like the reference's
 #pragma unroll
   for (int c = 0; c < 5; ++c) {
-    T large = 0;
+    double large = 0;
 #pragma unroll
     for (int j = c; j < 5; ++j) {
-      T v = A[j * 5 + c];
+      double v = A[j * 5 + c];
       if (fabs(v) > fabs(large)) {
         large = v;
         row = j;
@@ -653,7 +652,7 @@ __global__ void __launch_bounds__(kBlock) k_prepare_sgs(int nrow_pad, const int*
       if (j == row) {
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
-          T t = A[c * 5 + k];
+          double t = A[c * 5 + k];
           A[c * 5 + k] = A[j * 5 + k];
           A[j * 5 + k] = t;
         }
@@ -662,7 +661,7 @@ __global__ void __launch_bounds__(kBlock) k_prepare_sgs(int nrow_pad, const int*
         p[j] = t;
       }
     }
-    large = (T)1.0 / large;
+    large = 1.0 / large;
 #pragma unroll
     for (int j = c + 1; j < 5; ++j) A[j * 5 + c] *= large;
 #pragma unroll
@@ -670,18 +669,38 @@ __global__ void __launch_bounds__(kBlock) k_prepare_sgs(int nrow_pad, const int*
 #pragma unroll
       for (int k = c + 1; k < 5; ++k) A[j * 5 + k] -= A[j * 5 + c] * A[c * 5 + k];
   }
+  double id[5];
 #pragma unroll
-  for (int k = 0; k < 25; ++k) a[k * kW] = A[k];
-  piv[r] = p[0] | (p[1] << 3) | (p[2] << 6) | (p[3] << 9) | (p[4] << 12);
+  for (int k = 0; k < 5; ++k) id[k] = 1.0 / A[k * 5 + k];
+  // column `col` of the inverse: the unit vector, permuted, through both factors
+#pragma unroll
+  for (int col = 0; col < 5; ++col) {
+    double y[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      double s = (p[k] == col) ? 1.0 : 0.0;
+#pragma unroll
+      for (int c = 0; c < k; ++c) s -= A[k * 5 + c] * y[c];
+      y[k] = s;
+    }
+#pragma unroll
+    for (int k = 4; k >= 0; --k) {
+      double s = y[k];
+#pragma unroll
+      for (int c = 4; c > k; --c) s -= A[k * 5 + c] * y[c];
+      y[k] = s * id[k];
+      a[(k * 5 + col) * kW] = (T)y[k];
+    }
+  }
 }
 
 void launch_prepare_sgs(Ctx& c) {
   if (c.prm.precision == PCFD_CHOSEN_FP32)
     hipLaunchKernelGGL(k_prepare_sgs<float>, dim3(nblk(c.nrow_pad)), dim3(kBlock), 0, c.stream, c.nrow_pad, c.d.srow,
-                       c.d.Df, c.d.piv);
+                       c.d.Df);
   else
     hipLaunchKernelGGL(k_prepare_sgs<double>, dim3(nblk(c.nrow_pad)), dim3(kBlock), 0, c.stream, c.nrow_pad,
-                       c.d.srow, c.d.Dd, c.d.piv);
+                       c.d.srow, c.d.Dd);
   PCFD_HIP(hipGetLastError());
 }
 
