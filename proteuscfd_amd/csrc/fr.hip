@@ -80,37 +80,76 @@ __device__ __forceinline__ void store_state(double* __restrict__ q, long long i,
 }
 
 // ---- boundary states (UpdateBCs, ucs/bc.tcc:1399-1457) ---------------------
-// One thread per boundary node: its half-edges in half-edge order (a
-// Dirichlet / sonic-inflow half-edge resets the node's own state, which the
-// node's later half-edges then see, as in the reference's half-edge loop).
+// The reference walks the half-edges in order; a Dirichlet / sonic-inflow
+// half-edge resets its node's own state, which the node's later half-edges
+// then see.  Here every half-edge has a thread: the state it sees is the
+// reference state of the last such half-edge before it on its node, or the
+// node's own.  The threads read interior states and write their own phantom
+// only; k_fr_hardset then commits the resets.
+//
+// A characteristic state is ten sub-iterations of a 9x9 eigensystem, solve
+// and Newton loop in series.  One thread a node, its half-edges one after the
+// other and the 9x9 arrays in scratch, took 2.95 ms on 1,736 boundary nodes
+// with six half-edges each; one thread a half-edge with the arrays in
+// registers takes 0.094 ms (the same bits).
+constexpr int kBB = 64;  // threads per block of the half-edge kernels: one wavefront, up to 512 registers
+
+__device__ __forceinline__ bool resets_node(int type) { return type == fr::kSonicInflow || type == fr::kDirichlet; }
+
+// the node state half-edge p of node i sees
 template <int NS>
-__global__ void __launch_bounds__(kFB) k_fr_bcs(const Model* __restrict__ mp, int nbnd, const int* __restrict__ bnd,
+__device__ __forceinline__ void load_seen(const double* __restrict__ q, const double* __restrict__ qref, int i, int p,
+                                          const int* __restrict__ he_ptr, const int* __restrict__ he_id,
+                                          const int* __restrict__ he_tag, const int* __restrict__ bc_type,
+                                          State<NS>& L, const Model& m) {
+  int t = -1;
+  for (int k = he_ptr[i]; k < p; ++k) {
+    const int tag = he_tag[he_id[k]];
+    if (resets_node(bc_type[tag])) t = tag;
+  }
+  if (t >= 0) load_state<NS>(qref, t, L, m);
+  else load_state<NS>(q, i, L, m);
+}
+
+template <int NS>
+__global__ void __launch_bounds__(kBB) k_fr_bcs(const Model* __restrict__ mp, int nbe, const int* __restrict__ he_node,
                                                const int* __restrict__ he_ptr, const int* __restrict__ he_id,
                                                const int* __restrict__ he_tag, const double* __restrict__ he_a,
                                                const int* __restrict__ bc_type, const double* __restrict__ qref,
                                                int nnode, double beta, double* __restrict__ q) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= nbe) return;
+  const Model& m = *mp;
+  const int i = he_node[p], h = he_id[p], tag = he_tag[h];
+  State<NS> L, R, Qr;
+  load_seen<NS>(q, qref, i, p, he_ptr, he_id, he_tag, bc_type, L, m);
+  load_state<NS>(q, (long long)nnode + h, R, m);
+  load_state<NS>(qref, tag, Qr, m);
+  double a[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) a[k] = he_a[4LL * h + k];
+  if (fr::bc_state<NS>(m, bc_type[tag], L, R, Qr, a, beta)) store_state<NS>(q, (long long)nnode + h, R);
+}
+
+// boundary nodes with a Dirichlet / sonic-inflow half-edge take the reference
+// state of the last one
+template <int NS>
+__global__ void __launch_bounds__(kFB) k_fr_hardset(int nbnd, const int* __restrict__ bnd,
+                                                   const int* __restrict__ he_ptr, const int* __restrict__ he_id,
+                                                   const int* __restrict__ he_tag, const int* __restrict__ bc_type,
+                                                   const double* __restrict__ qref, double* __restrict__ q) {
+  constexpr int NE = NS + 4;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nbnd) return;
-  const Model& m = *mp;
   const int i = bnd[t];
-  State<NS> L;
-  load_state<NS>(q, i, L, m);
-  bool lchanged = false;
-  for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) {
-    const int h = he_id[p], tag = he_tag[h];
-    const int ty = bc_type[tag];
-    State<NS> R, Qr;
-    load_state<NS>(q, (long long)nnode + h, R, m);
-    load_state<NS>(qref, tag, Qr, m);
-    double a[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) a[k] = he_a[4LL * h + k];
-    if (fr::bc_state<NS>(m, ty, L, R, Qr, a, beta)) {
-      store_state<NS>(q, (long long)nnode + h, R);
-      if (ty == fr::kSonicInflow || ty == fr::kDirichlet) lchanged = true;
-    }
+  int last = -1;
+  for (int k = he_ptr[i]; k < he_ptr[i + 1]; ++k) {
+    const int tag = he_tag[he_id[k]];
+    if (resets_node(bc_type[tag])) last = tag;
   }
-  if (lchanged) store_state<NS>(q, i, L);
+  if (last < 0) return;
+#pragma unroll
+  for (int k = 0; k < NE; ++k) q[(long long)i * NE + k] = qref[(long long)last * NE + k];
 }
 
 // ---- edge passes -----------------------------------------------------------
@@ -374,104 +413,100 @@ __global__ void __launch_bounds__(kFB) k_fr_jac_edge(const Model* __restrict__ m
   }
 }
 
-// Bkernel_NumJac (ucs/jacobian.tcc:458-535) with jacobianBoundaryEval 0:
-// per boundary node, its half-edges in order; the BC state is set on the
-// stored states first (q updated, as the reference's in-place call does),
-// then each native variable of the node perturbed, the BC re-evaluated from
-// the perturbed state and the boundary flux differenced.  The node's
-// boundary blocks are summed in half-edge order into jdb.
-// Two passes: k_fr_jac_bnd_base walks each node's half-edges once, applies
-// the BC updates to q and records, per half-edge, the node's and the
-// boundary state's native values right after that half-edge's BC call and
-// the unperturbed flux (bhe, 3 NE values); k_fr_jac_bnd_cols gives each
-// (node, column) a thread that differences from those records and sums its
-// column over the half-edges in their order.  A State's auxiliary values are
-// always aux() of its native ones (load_state and bc_state recompute them),
-// so the records carry every bit the perturbed evaluations read.
+// Bkernel_NumJac (ucs/jacobian.tcc:458-535) with jacobianBoundaryEval 0: the
+// BC state is set on the stored states first (q updated, as the reference's
+// in-place call does), then each native variable of the node perturbed, the
+// BC re-evaluated from the perturbed state and the boundary flux differenced.
+// Three passes: k_fr_jac_bnd_base gives every half-edge a thread, which
+// applies its BC update and records the node's and the boundary state's native
+// values right after that call and the unperturbed flux (bhe, 3 NE values);
+// k_fr_jac_bnd_cols gives every (half-edge, column) a thread, which writes
+// its column of differences (bcol); k_fr_jac_bnd_sum adds a node's half-edges
+// in their order into jdb.  A State's auxiliary values are always aux() of
+// its native ones (load_state and bc_state recompute them), so the records
+// carry every bit the perturbed evaluations read.  On 1,736 boundary nodes
+// with six half-edges each (characteristic states): base 2.99 -> 0.094 ms,
+// columns 2.68 -> 0.132 + 0.006 ms against one thread a node and a (node,
+// column) with the 9x9 arrays in scratch; bit-identical.
 template <int NS>
-__global__ void __launch_bounds__(kFB) k_fr_jac_bnd_base(const Model* __restrict__ mp, int nbnd,
-                                                        const int* __restrict__ bnd, const int* __restrict__ he_ptr,
+__global__ void __launch_bounds__(kBB) k_fr_jac_bnd_base(const Model* __restrict__ mp, int nbe,
+                                                        const int* __restrict__ he_node,
+                                                        const int* __restrict__ he_ptr,
                                                         const int* __restrict__ he_id, const int* __restrict__ he_tag,
                                                         const double* __restrict__ he_a,
                                                         const int* __restrict__ bc_type,
                                                         const double* __restrict__ qref, int nnode, double beta,
                                                         double* __restrict__ q, double* __restrict__ bhe) {
   constexpr int NE = NS + 4;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nbnd) return;
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= nbe) return;
   const Model& m = *mp;
-  const int i = bnd[t];
-  State<NS> L;
-  load_state<NS>(q, i, L, m);
-  bool lchanged = false;
-  for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) {
-    const int h = he_id[p], tag = he_tag[h];
-    const int ty = bc_type[tag];
-    State<NS> R, Qr;
-    load_state<NS>(q, (long long)nnode + h, R, m);
-    load_state<NS>(qref, tag, Qr, m);
-    double a[4];
+  const int i = he_node[p], h = he_id[p], tag = he_tag[h];
+  State<NS> L, R, Qr;
+  load_seen<NS>(q, qref, i, p, he_ptr, he_id, he_tag, bc_type, L, m);
+  load_state<NS>(q, (long long)nnode + h, R, m);
+  load_state<NS>(qref, tag, Qr, m);
+  double a[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) a[k] = he_a[4LL * h + k];
-    if (fr::bc_state<NS>(m, ty, L, R, Qr, a, beta)) {
-      store_state<NS>(q, (long long)nnode + h, R);
-      if (ty == fr::kSonicInflow || ty == fr::kDirichlet) lchanged = true;
-    }
-    double fS[NE];
-    fr::hllc<NS>(m, L, R, a, beta, fS);
-    double* rec = bhe + (long long)p * 3 * NE;
+  for (int k = 0; k < 4; ++k) a[k] = he_a[4LL * h + k];
+  if (fr::bc_state<NS>(m, bc_type[tag], L, R, Qr, a, beta)) store_state<NS>(q, (long long)nnode + h, R);
+  double fS[NE];
+  fr::hllc<NS>(m, L, R, a, beta, fS);
+  double* rec = bhe + (long long)p * 3 * NE;
 #pragma unroll
-    for (int k = 0; k < NE; ++k) {
-      rec[k] = L.q[k];
-      rec[NE + k] = R.q[k];
-      rec[2 * NE + k] = fS[k];
-    }
+  for (int k = 0; k < NE; ++k) {
+    rec[k] = L.q[k];
+    rec[NE + k] = R.q[k];
+    rec[2 * NE + k] = fS[k];
   }
-  if (lchanged) store_state<NS>(q, i, L);
 }
 
 template <int NS>
-__global__ void __launch_bounds__(kFB) k_fr_jac_bnd_cols(const Model* __restrict__ mp, int nbnd,
-                                                        const int* __restrict__ bnd, const int* __restrict__ he_ptr,
+__global__ void __launch_bounds__(kBB) k_fr_jac_bnd_cols(const Model* __restrict__ mp, int nbe,
                                                         const int* __restrict__ he_id, const int* __restrict__ he_tag,
                                                         const double* __restrict__ he_a,
                                                         const int* __restrict__ bc_type,
                                                         const double* __restrict__ qref, double beta,
-                                                        const double* __restrict__ bhe, double* __restrict__ jdb) {
+                                                        const double* __restrict__ bhe, double* __restrict__ bcol) {
+  constexpr int NE = NS + 4;
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (long long)nbe * NE) return;
+  const int p = (int)(t / NE), c = (int)(t % NE);
+  const Model& m = *mp;
+  const double hh = 1.0e-8;
+  const int h = he_id[p], tag = he_tag[h];
+  const double* rec = bhe + (long long)p * 3 * NE;
+  State<NS> PL, PR, Qr;
+  load_state<NS>(rec, 0, PL, m);
+  load_state<NS>(rec + NE, 0, PR, m);
+  load_state<NS>(qref, tag, Qr, m);
+  double a[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) a[k] = he_a[4LL * h + k];
+  // PL.q[c] += hh without a dynamic register index
+#pragma unroll
+  for (int k = 0; k < NE; ++k) PL.q[k] = (k == c) ? PL.q[k] + hh : PL.q[k];
+  fr::aux(m, PL);
+  fr::bc_state<NS>(m, bc_type[tag], PL, PR, Qr, a, beta);
+  double fL[NE];
+  fr::hllc<NS>(m, PL, PR, a, beta, fL);
+#pragma unroll
+  for (int j = 0; j < NE; ++j) bcol[t * NE + j] = (fL[j] - rec[2 * NE + j]) / hh;
+}
+
+// jdb [node][row][column] = sum over the node's half-edges, in their order
+template <int NS>
+__global__ void __launch_bounds__(kFB) k_fr_jac_bnd_sum(int nbnd, const int* __restrict__ bnd,
+                                                       const int* __restrict__ he_ptr,
+                                                       const double* __restrict__ bcol, double* __restrict__ jdb) {
   constexpr int NE = NS + 4, NE2 = NE * NE;
   const long long t2 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t2 >= (long long)nbnd * NE) return;
-  const int t = (int)(t2 / NE), c = (int)(t2 % NE);
-  const Model& m = *mp;
+  if (t2 >= (long long)nbnd * NE2) return;
+  const int t = (int)(t2 / NE2), k = (int)(t2 % NE2);  // k = column * NE + row, as bcol stores them
   const int i = bnd[t];
-  const double hh = 1.0e-8;
-  double acc[NE];
-#pragma unroll
-  for (int j = 0; j < NE; ++j) acc[j] = 0.0;
-  for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) {
-    const int h = he_id[p], tag = he_tag[h];
-    const int ty = bc_type[tag];
-    const double* rec = bhe + (long long)p * 3 * NE;
-    State<NS> PL, PR, Qr;
-    load_state<NS>(rec, 0, PL, m);
-    load_state<NS>(rec + NE, 0, PR, m);
-    load_state<NS>(qref, tag, Qr, m);
-    double a[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) a[k] = he_a[4LL * h + k];
-    // PL.q[c] += hh without a dynamic register index
-#pragma unroll
-    for (int k = 0; k < NE; ++k) PL.q[k] = (k == c) ? PL.q[k] + hh : PL.q[k];
-    fr::aux(m, PL);
-    fr::bc_state<NS>(m, ty, PL, PR, Qr, a, beta);
-    double fL[NE];
-    fr::hllc<NS>(m, PL, PR, a, beta, fL);
-#pragma unroll
-    for (int j = 0; j < NE; ++j) acc[j] += (fL[j] - rec[2 * NE + j]) / hh;
-  }
-  double* J = jdb + (long long)t * NE2;
-#pragma unroll
-  for (int j = 0; j < NE; ++j) J[j * NE + c] = acc[j];
+  double acc = 0.0;
+  for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) acc += bcol[(long long)p * NE2 + k];
+  jdb[(long long)t * NE2 + (k % NE) * NE + k / NE] = acc;
 }
 
 // Per node: the temporal block (ContributeTemporalTerms applied to a zero
@@ -586,52 +621,6 @@ __global__ void __launch_bounds__(64 * (NS + 4)) k_fr_jac_diag(int nrow_pad, con
   for (int c = 0; c < NE; ++c) Dr[(long long)(rr * NE + c) * kLane] = (TM)A[c];
 }
 
-// fr::lu (LU with logical pivoting, ucs/matrix.h:184-235) with the rows
-// kept physically in pivot order: on return b[k * N + c] is lu's
-// a[p[k] * N + c].  Every element meets the same operations in the same
-// order, so the factor is the same bits, while all indices are static and
-// the block stays in registers (lu's a[p[j] * N + i] sends it to scratch);
-// a row swap is a select over the static row indices.  As in lu, the pivot
-// row index carries over from the previous column when a column holds no
-// nonzero, so the swap partner may be an earlier row.
-template <int N, typename T>
-__device__ __forceinline__ void lu_rows(T* b, int* p) {
-  int row = 0;
-#pragma unroll
-  for (int i = 0; i < N; ++i) p[i] = i;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    T large = 0.0;
-#pragma unroll
-    for (int j = i; j < N; ++j)
-      if (fabs(b[j * N + i]) > fabs(large)) {
-        large = b[j * N + i];
-        row = j;
-      }
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      if (j == i) continue;
-      const bool s = (j == row);
-      const int pi = p[i], pj = p[j];
-      p[i] = s ? pj : pi;
-      p[j] = s ? pi : pj;
-#pragma unroll
-      for (int k = 0; k < N; ++k) {
-        const T x = b[i * N + k], y = b[j * N + k];
-        b[i * N + k] = s ? y : x;
-        b[j * N + k] = s ? x : y;
-      }
-    }
-    large = (T)1.0 / large;
-#pragma unroll
-    for (int j = i + 1; j < N; ++j) b[j * N + i] *= large;
-#pragma unroll
-    for (int j = i + 1; j < N; ++j)
-#pragma unroll
-      for (int k = i + 1; k < N; ++k) b[j * N + k] -= b[j * N + i] * b[i * N + k];
-  }
-}
-
 // PrepareSGS (ucs/crsmatrix.tcc:839-876): LU with logical pivoting of every
 // diagonal block, in place; the row order is packed 4 bits per entry.
 template <int NS, typename TM>
@@ -645,7 +634,7 @@ __global__ void __launch_bounds__(64) k_fr_prepare(int nrow_pad, TM* __restrict_
 #pragma unroll
   for (int k = 0; k < NE2; ++k) A[k] = Dr[(long long)k * kLane];
   int p[NE];
-  lu_rows<NE, TM>(A, p);
+  fr::lu_rows<NE, TM>(A, p);
   long long pk = 0;
 #pragma unroll
   for (int k = 0; k < NE; ++k) pk |= (long long)p[k] << (4 * k);
@@ -654,31 +643,6 @@ __global__ void __launch_bounds__(64) k_fr_prepare(int nrow_pad, TM* __restrict_
   // solve indexes the factor statically
 #pragma unroll
   for (int k = 0; k < NE2; ++k) Dr[(long long)k * kLane] = A[k];
-}
-
-// LuSolve (ucs/matrix.h:237-264) on a factor stored with its rows in pivot
-// order: the same products and sums as the logical-pivot form, with only
-// the right-hand side picked by the pivot
-template <int N, typename T>
-__device__ __forceinline__ void lu_solve_rows(const T* a, T* b, const int* p) {
-  T x[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    T sum = 0.0;
-#pragma unroll
-    for (int j = 0; j < i; ++j) sum += a[i * N + j] * x[j];
-    T bp = b[0];
-#pragma unroll
-    for (int k = 1; k < N; ++k) bp = (p[i] == k) ? b[k] : bp;
-    x[i] = bp - sum;
-  }
-#pragma unroll
-  for (int i = N - 1; i >= 0; --i) {
-    T sum = 0.0;
-#pragma unroll
-    for (int j = N - 1; j > i; --j) sum += a[i * N + j] * b[j];
-    b[i] = (x[i] - sum) / a[i * N + i];
-  }
 }
 
 // One colour of a symmetric Gauss-Seidel sweep (CRS::SGS, ucs/crs.tcc:61-173):
@@ -749,7 +713,7 @@ __global__ void __launch_bounds__(64 * (NS + 4)) k_fr_sgs_color(int chunk0, cons
   int p[NE];
 #pragma unroll
   for (int k = 0; k < NE; ++k) p[k] = (int)((pk >> (4 * k)) & 15);
-  lu_solve_rows<NE, TM>(A, rv, p);
+  fr::lu_solve_rows<NE, TM>(A, rv, p);
 #pragma unroll
   for (int k = 0; k < NE; ++k) x[(long long)i * NE + k] = rv[k];
 }
@@ -836,6 +800,7 @@ struct pcfd_fr {
   std::string err;
   const pcfd_chem* chem = nullptr;
   int ns = 0, ne = 0, nnode = 0, nbnode = 0, nedge = 0, ntot = 0, ntag = 0, nbnd = 0;
+  bool has_hardset = false;  // a half-edge resets its node's state (Dirichlet, sonic inflow)
   int ncolor = 0, nchunk = 0, nrow_pad = 0;
   long long nslot = 0;
   std::vector<int> color_chunk, h_nptr, h_nslot, h_edges, h_srow, h_spos, h_sbase;
@@ -851,8 +816,8 @@ struct pcfd_fr {
   long long bytes = 0;
   // device arrays
   double *q = nullptr, *qref = nullptr, *vol = nullptr, *edge_a = nullptr, *he_a = nullptr, *eflux = nullptr,
-         *elam = nullptr, *b = nullptr, *dt = nullptr, *jdb = nullptr, *bhe = nullptr, *red = nullptr, *aux = nullptr;
-  int *edges = nullptr, *nptr = nullptr, *nslot_d = nullptr, *he_ptr = nullptr, *he_id = nullptr, *he_tag = nullptr,
+         *elam = nullptr, *b = nullptr, *dt = nullptr, *jdb = nullptr, *bhe = nullptr, *bcol = nullptr, *red = nullptr, *aux = nullptr;
+  int *edges = nullptr, *nptr = nullptr, *nslot_d = nullptr, *he_ptr = nullptr, *he_id = nullptr, *he_tag = nullptr, *he_node = nullptr,
       *bc_type = nullptr, *bnd = nullptr, *bidx = nullptr, *srow = nullptr, *swidth = nullptr, *sbase = nullptr,
       *scol = nullptr, *icount = nullptr;
   long long* piv = nullptr;
@@ -891,8 +856,8 @@ void dfree(T*& p) {
 
 void free_all(pcfd_fr& f) {
   dfree(f.q); dfree(f.qref); dfree(f.vol); dfree(f.edge_a); dfree(f.he_a); dfree(f.eflux); dfree(f.elam);
-  dfree(f.b); dfree(f.dt); dfree(f.jdb); dfree(f.bhe); dfree(f.red); dfree(f.aux); dfree(f.edges); dfree(f.nptr);
-  dfree(f.nslot_d); dfree(f.he_ptr); dfree(f.he_id); dfree(f.he_tag); dfree(f.bc_type); dfree(f.bnd);
+  dfree(f.b); dfree(f.dt); dfree(f.jdb); dfree(f.bhe); dfree(f.bcol); dfree(f.red); dfree(f.aux); dfree(f.edges); dfree(f.nptr);
+  dfree(f.nslot_d); dfree(f.he_ptr); dfree(f.he_id); dfree(f.he_tag); dfree(f.he_node); dfree(f.bc_type); dfree(f.bnd);
   dfree(f.bidx); dfree(f.srow); dfree(f.swidth); dfree(f.sbase); dfree(f.scol); dfree(f.icount);
   dfree(f.piv); dfree(f.Md); dfree(f.Dd); dfree(f.xd); dfree(f.Mf); dfree(f.Df); dfree(f.xf); dfree(f.dmodel);
   dfree(f.s_rhoi); dfree(f.s_T); dfree(f.s_w); dfree(f.s_lst); dfree(f.s_cnt); dfree(f.s_off);
@@ -948,11 +913,19 @@ void send(pcfd_fr& f, int k) {
 
 constexpr int NS5 = 5;
 
+void run_hardset(pcfd_fr& f) {
+  if (!f.has_hardset) return;
+  hipLaunchKernelGGL(k_fr_hardset<NS5>, dim3(nblocks(f.nbnd)), dim3(kFB), 0, f.stream, f.nbnd, f.bnd, f.he_ptr,
+                     f.he_id, f.he_tag, f.bc_type, f.qref, f.q);
+  hcheck(hipGetLastError(), "k_fr_hardset");
+}
+
 void run_bcs(pcfd_fr& f) {
   if (f.nbnd == 0) return;
-  hipLaunchKernelGGL(k_fr_bcs<NS5>, dim3(nblocks(f.nbnd)), dim3(kFB), 0, f.stream, f.dmodel, f.nbnd, f.bnd, f.he_ptr,
-                     f.he_id, f.he_tag, f.he_a, f.bc_type, f.qref, f.nnode, f.prm.beta, f.q);
+  hipLaunchKernelGGL(k_fr_bcs<NS5>, dim3(nblocks(f.nbnode, kBB)), dim3(kBB), 0, f.stream, f.dmodel, f.nbnode,
+                     f.he_node, f.he_ptr, f.he_id, f.he_tag, f.he_a, f.bc_type, f.qref, f.nnode, f.prm.beta, f.q);
   hcheck(hipGetLastError(), "k_fr_bcs");
+  run_hardset(f);
 }
 
 // residual into f.b; norms[1+neqn] (residGlobal, per-equation) when non-null
@@ -1031,14 +1004,18 @@ void run_jacobian_t(pcfd_fr& f, TM* M, TM* D) {
     send(f, 6);
   }
   if (f.nbnd > 0) {
-    hipLaunchKernelGGL(k_fr_jac_bnd_base<NS5>, dim3(nblocks(f.nbnd)), dim3(kFB), 0, f.stream, f.dmodel, f.nbnd,
-                       f.bnd, f.he_ptr, f.he_id, f.he_tag, f.he_a, f.bc_type, f.qref, f.nnode, f.prm.beta, f.q,
-                       f.bhe);
+    hipLaunchKernelGGL(k_fr_jac_bnd_base<NS5>, dim3(nblocks(f.nbnode, kBB)), dim3(kBB), 0, f.stream, f.dmodel,
+                       f.nbnode, f.he_node, f.he_ptr, f.he_id, f.he_tag, f.he_a, f.bc_type, f.qref, f.nnode,
+                       f.prm.beta, f.q, f.bhe);
     hcheck(hipGetLastError(), "k_fr_jac_bnd_base");
-    hipLaunchKernelGGL(k_fr_jac_bnd_cols<NS5>, dim3(nblocks((long long)f.nbnd * (NS5 + 4))), dim3(kFB), 0,
-                       f.stream, f.dmodel, f.nbnd, f.bnd, f.he_ptr, f.he_id, f.he_tag, f.he_a, f.bc_type, f.qref,
-                       f.prm.beta, f.bhe, f.jdb);
+    run_hardset(f);
+    hipLaunchKernelGGL(k_fr_jac_bnd_cols<NS5>, dim3(nblocks((long long)f.nbnode * (NS5 + 4), kBB)), dim3(kBB), 0,
+                       f.stream, f.dmodel, f.nbnode, f.he_id, f.he_tag, f.he_a, f.bc_type, f.qref, f.prm.beta, f.bhe,
+                       f.bcol);
     hcheck(hipGetLastError(), "k_fr_jac_bnd_cols");
+    hipLaunchKernelGGL(k_fr_jac_bnd_sum<NS5>, dim3(nblocks((long long)f.nbnd * (NS5 + 4) * (NS5 + 4))), dim3(kFB), 0,
+                       f.stream, f.nbnd, f.bnd, f.he_ptr, f.bcol, f.jdb);
+    hcheck(hipGetLastError(), "k_fr_jac_bnd_sum");
   }
   hipLaunchKernelGGL(k_fr_node_terms<NS5>, dim3(nblocks(f.nnode)), dim3(kFB), 0, f.stream, f.dmodel,
                      chem_device_model(f.chem), f.nnode, f.q, f.vol, f.dt, f.prm.reactions, f.prm.beta, f.nterm);
@@ -1279,6 +1256,14 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
         bnd.push_back(i);
       }
     f->nbnd = (int)bnd.size();
+    // node of each half-edge in list order
+    std::vector<int> he_node(nb);
+    for (int i = 0; i < nn; ++i)
+      for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) he_node[p] = i;
+    for (int h = 0; h < nb; ++h) {
+      const int ty = m->bc_type[m->bfactag[h]];
+      if (ty == fr::kSonicInflow || ty == fr::kDirichlet) f->has_hardset = true;
+    }
     // colouring and the SELL layout of the block matrix
     std::vector<int> colour(nn);
     const int ncol = pcfd_color_nodes(nn, ne, m->edges, colour.data());
@@ -1364,6 +1349,7 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
     dput(*f, &f->he_ptr, he_ptr);
     dput(*f, &f->he_id, he_id);
     dput(*f, &f->he_tag, he_tag);
+    dput(*f, &f->he_node, he_node);
     dput(*f, &f->bc_type, bct);
     dput(*f, &f->qref, qr);
     dput(*f, &f->bnd, bnd);
@@ -1381,6 +1367,7 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
     dalloc(*f, &f->dt, (size_t)nn);
     dalloc(*f, &f->jdb, (size_t)std::max(f->nbnd, 1) * NE2);
     dalloc(*f, &f->bhe, (size_t)std::max(nb, 1) * 3 * NE);
+    dalloc(*f, &f->bcol, (size_t)std::max(nb, 1) * NE2);
     dalloc(*f, &f->red, (size_t)(NE + 1) * std::max(nblocks(nn), 256));
     dalloc(*f, &f->icount, 4);
     dalloc(*f, &f->piv, (size_t)f->nrow_pad);

@@ -413,50 +413,84 @@ PCFD_HD double t_from_p(const Model& m, const double* rhoi, double p, double Tin
   return TDim / Tref;
 }
 
-// LU with partial (logical) pivoting and LuSolve (ucs/matrix.h:184-264):
-// p holds the row order; b is overwritten with the solution
-template <int N>
-PCFD_HD void lu(double* a, int* p) {
+// LU with logical pivoting (ucs/matrix.h:184-235) with the rows kept
+// physically in pivot order: on return b[k * N + c] is the reference's
+// a[p[k] * N + c].  Every element meets the same operations in the same
+// order, so the factor is the same bits, while all indices are static and
+// the block stays in registers; a row swap is a select over the static row
+// indices.  As in the reference, the pivot row index carries over from the
+// previous column when a column holds no nonzero, so the swap partner may be
+// an earlier row.
+template <int N, typename T>
+PCFD_HD void lu_rows(T* b, int* p) {
   int row = 0;
 #pragma unroll
   for (int i = 0; i < N; ++i) p[i] = i;
+#pragma unroll
   for (int i = 0; i < N; ++i) {
-    double large = 0.0;
+    T large = 0.0;
+#pragma unroll
     for (int j = i; j < N; ++j)
-      if (fabs(a[p[j] * N + i]) > fabs(large)) {
-        large = a[p[j] * N + i];
+      if (fabs(b[j * N + i]) > fabs(large)) {
+        large = b[j * N + i];
         row = j;
       }
-    const int t = p[i];
-    p[i] = p[row];
-    p[row] = t;
-    large = 1.0 / large;
-    for (int j = i + 1; j < N; ++j) a[p[j] * N + i] *= large;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (j == i) continue;
+      const bool s = (j == row);
+      const int pi = p[i], pj = p[j];
+      p[i] = s ? pj : pi;
+      p[j] = s ? pi : pj;
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const T x = b[i * N + k], y = b[j * N + k];
+        b[i * N + k] = s ? y : x;
+        b[j * N + k] = s ? x : y;
+      }
+    }
+    large = (T)1.0 / large;
+#pragma unroll
+    for (int j = i + 1; j < N; ++j) b[j * N + i] *= large;
+#pragma unroll
     for (int j = i + 1; j < N; ++j)
-      for (int k = i + 1; k < N; ++k) a[p[j] * N + k] -= a[p[j] * N + i] * a[p[i] * N + k];
+#pragma unroll
+      for (int k = i + 1; k < N; ++k) b[j * N + k] -= b[j * N + i] * b[i * N + k];
   }
 }
 
+// LuSolve (ucs/matrix.h:237-264) on a factor stored with its rows in pivot
+// order: the same products and sums as the logical-pivot form, with only
+// the right-hand side picked by the pivot
 template <int N, typename T>
-PCFD_HD void lu_solve(const T* a, T* b, const int* p) {
+PCFD_HD void lu_solve_rows(const T* a, T* b, const int* p) {
   T x[N];
+#pragma unroll
   for (int i = 0; i < N; ++i) {
     T sum = 0.0;
-    for (int j = 0; j < i; ++j) sum += a[p[i] * N + j] * x[j];
-    x[i] = b[p[i]] - sum;
+#pragma unroll
+    for (int j = 0; j < i; ++j) sum += a[i * N + j] * x[j];
+    T bp = b[0];
+#pragma unroll
+    for (int k = 1; k < N; ++k) bp = (p[i] == k) ? b[k] : bp;
+    x[i] = bp - sum;
   }
+#pragma unroll
   for (int i = N - 1; i >= 0; --i) {
     T sum = 0.0;
-    for (int j = N - 1; j > i; --j) sum += a[p[i] * N + j] * b[j];
-    b[i] = (x[i] - sum) / a[p[i] * N + i];
+#pragma unroll
+    for (int j = N - 1; j > i; --j) sum += a[i * N + j] * b[j];
+    b[i] = (x[i] - sum) / a[i * N + i];
   }
 }
 
 // MatVecMult (ucs/matrix.h:63-74)
 template <int N>
 PCFD_HD void matvec(const double* a, const double* v, double* out) {
+#pragma unroll
   for (int i = 0; i < N; ++i) {
     out[i] = a[i * N] * v[0];
+#pragma unroll
     for (int j = 1; j < N; ++j) out[i] += a[i * N + j] * v[j];
   }
 }
@@ -494,10 +528,12 @@ PCFD_HD void farfield(const Model& m, const State<NS>& L, State<NS>& R, const St
     const double Tguess = ql[NE - 1];
     ql[NE - 1] = L.P;
     qi[NE - 1] = Qinf.P;
+#pragma unroll
     for (int i = 0; i < NE; ++i) {
       rhs[i] = 0.0;
-      const double* src = eig[i] >= 0.0 ? ql : qi;
-      for (int j = 0; j < NE; ++j) rhs[i] += Ti[i * NE + j] * src[j];
+      const bool own = eig[i] >= 0.0;
+#pragma unroll
+      for (int j = 0; j < NE; ++j) rhs[i] += Ti[i * NE + j] * (own ? ql[j] : qi[j]);
     }
     matvec<NE>(T, rhs, R.q);
 #pragma unroll
@@ -542,8 +578,10 @@ PCFD_HD void wall(const Model& m, const State<NS>& L, State<NS>& R, const double
     for (int i = 0; i < NE; ++i) ql[i] = L.q[i];
     const double Tguess = ql[NE - 1];
     ql[NE - 1] = L.P;
+#pragma unroll
     for (int i = 0; i < NE; ++i) {
       rhs[i] = 0.0;
+#pragma unroll
       for (int j = 0; j < NE; ++j) rhs[i] += Ti[i * NE + j] * ql[j];
     }
 #pragma unroll
@@ -553,8 +591,8 @@ PCFD_HD void wall(const Model& m, const State<NS>& L, State<NS>& R, const double
     Ti[(NE - 1) * NE + NS + 2] = a[2];
     Ti[(NE - 1) * NE + NS + 3] = 0.0;
     rhs[NE - 1] = 0.0;
-    lu<NE>(Ti, p);
-    lu_solve<NE>(Ti, rhs, p);
+    lu_rows<NE>(Ti, p);
+    lu_solve_rows<NE>(Ti, rhs, p);
 #pragma unroll
     for (int i = 0; i < NE; ++i) R.q[i] = rhs[i];
     R.q[NE - 1] = t_from_p<NS>(m, R.q, R.q[NE - 1], Tguess);
