@@ -51,16 +51,21 @@ struct Dev {
   int* he_ptr = nullptr;    // nnode+1: half-edges of node i, in half-edge order
   int* he_id = nullptr;     // nbnode
   int* he_tag = nullptr;    // nbnode
+  int* he_node = nullptr;   // nbnode: node i of each half-edge, in he_id's order; ~i where a half-edge resets it
+  int4* he_desc = nullptr;  // nbnode, in he_id's order: half-edge id, face tag, BC type, wall-normal neighbour or -1
+  int* rst = nullptr;       // nrst: the boundary nodes that a half-edge resets (index into bnd_nodes)
+  double* seen = nullptr;   // 5 x nbnode: the node state each half-edge of such a node sees
   double* he_a = nullptr;   // 4 x nbnode
   int* bnd_nodes = nullptr; // nodes with >= 1 half-edge
   int* bidx = nullptr;      // nnode: index into bnd_nodes, -1 for nodes without half-edges
   double* jdb = nullptr;    // 25 x nbnd boundary part of the Jacobian diagonal
+  double* jhe = nullptr;    // 10 x nbnode: boundary state and unperturbed flux of each half-edge
+  double* jcol = nullptr;   // 25 x nbnode: each half-edge's columns of that part
   double* jqb = nullptr;    // 5 x nbnd boundary-node states after the Jacobian's BC re-evaluation
   // boundary-condition tables per face tag
   int* bc_type = nullptr;   // ntag
   double* qref = nullptr;   // 5 x ntag (conservative), aux pressure at [5*ntag + tag]
   double* twall = nullptr;  // ntag non-dimensional noSlip wall temperature (<0 adiabatic)
-  int* he_nrm = nullptr;    // nbnode: wall-normal neighbour of a noSlip half-edge's node, else -1
   int* spos = nullptr;      // nnode: SELL row of each node
   // state
   double* q = nullptr;      // 5 x ntot (interior then phantoms)
@@ -109,11 +114,12 @@ struct Ctx {
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   bool overlap = true;            // PCFD_JACOBIAN_STREAM=0 turns the overlap off
   bool jac_pending = false;
-  bool has_hardset = false;       // a Dirichlet / sonic-inflow / noSlip tag exists
   std::string err;
   int nnode = 0, nbnode = 0, nedge = 0, ntot = 0, ntag = 0, nnz = 0, nbnd = 0;
   int nchunk_g = 0, nchunk_s = 0, nrow_pad = 0;
   long long nslot_g = 0, nslot_s = 0;
+  int nrst = 0;           // boundary nodes that a hard-set half-edge resets
+  int max_swidth = 0;     // slots of the widest SELL row
   long long nblocks = 0;  // nnode + 2*nedge (reference count)
   int ncolor = 0;
   bool has_noslip = false;

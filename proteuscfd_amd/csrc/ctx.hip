@@ -48,8 +48,8 @@ void dfree(T*& p) {
 void free_all(Ctx& c) {
   Dev& d = c.d;
   dfree(d.xyz); dfree(d.vol); dfree(d.vol23); dfree(d.sw); dfree(d.gwidth); dfree(d.gbase); dfree(d.gcol); dfree(d.gnrm); dfree(d.qrk);
-  dfree(d.he_ptr); dfree(d.he_id); dfree(d.he_tag); dfree(d.he_a); dfree(d.bnd_nodes); dfree(d.bidx);
-  dfree(d.jdb); dfree(d.jqb); dfree(d.bc_type); dfree(d.twall); dfree(d.he_nrm); dfree(d.spos);
+  dfree(d.he_ptr); dfree(d.he_id); dfree(d.he_tag); dfree(d.he_node); dfree(d.seen); dfree(d.he_desc); dfree(d.rst); dfree(d.he_a); dfree(d.bnd_nodes); dfree(d.bidx);
+  dfree(d.jdb); dfree(d.jhe); dfree(d.jcol); dfree(d.jqb); dfree(d.bc_type); dfree(d.twall); dfree(d.spos);
   dfree(d.qref); dfree(d.q); dfree(d.grad); dfree(d.lim); dfree(d.lim2); dfree(d.edges); dfree(d.clip_flag); dfree(d.clip_cnt);
   dfree(d.clip_off); dfree(d.clip_list); dfree(d.b); dfree(d.dt);
   dfree(d.gslot); dfree(d.srow); dfree(d.swidth); dfree(d.swidth_lo); dfree(d.sbase); dfree(d.scol); dfree(d.Md); dfree(d.Mf); dfree(d.Dd);
@@ -98,6 +98,8 @@ int need_params(Ctx& c) {
 }
 
 void ensure_matrix(Ctx& c) {
+  if (!c.d.jhe) dalloc(c, &c.d.jhe, 10 * (size_t)c.nbnode);
+  if (!c.d.jcol) dalloc(c, &c.d.jcol, 25 * (size_t)c.nbnode);
   const size_t off = (size_t)c.nslot_s * kW * 25, dg = (size_t)c.nchunk_s * kW * 25;
   if (c.prm.precision == PCFD_CHOSEN_FP32) {
     if (!c.d.Mf) dalloc(c, &c.d.Mf, off);
@@ -145,7 +147,7 @@ void sub_end(Ctx& c, int k) {
 void ensure_matrix_alloc(Ctx& c) { ensure_matrix(c); }
 void ensure_overlap_buffers(Ctx& c) {
   if (!c.d.dt_next) dalloc(c, &c.d.dt_next, (size_t)c.nnode);
-  if (c.has_hardset && !c.d.qjac) dalloc(c, &c.d.qjac, 5 * (size_t)c.ntot);
+  if (c.nrst > 0 && !c.d.qjac) dalloc(c, &c.d.qjac, 5 * (size_t)c.ntot);
 }
 }  // namespace pcfd
 
@@ -274,13 +276,22 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
       std::vector<int> hfill(he_ptr.begin(), he_ptr.end() - 1);
       for (int h = 0; h < nb; ++h) he_id[hfill[m->bedges[2 * h]]++] = h;
     }
-    std::vector<int> bnd, bidx(nn, -1);
+    // boundary nodes; hard-set BC types reset the state of their node
+    std::vector<int> bnd, rst, bidx(nn, -1), he_node(nb);
     for (int i = 0; i < nn; ++i)
       if (he_ptr[i + 1] > he_ptr[i]) {
+        bool resets = false;
+        for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) {
+          const int ty = m->bc_type[m->bfactag[he_id[p]]];
+          resets |= ty == 1 /* dirichlet */ || ty == 7 /* sonicInflow */ || ty == 4 /* noSlip */;
+        }
+        for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) he_node[p] = resets ? ~i : i;
+        if (resets) rst.push_back((int)bnd.size());
         bidx[i] = (int)bnd.size();
         bnd.push_back(i);
       }
     c.nbnd = (int)bnd.size();
+    c.nrst = (int)rst.size();
     std::vector<int> he_tag(m->bfactag, m->bfactag + nb);
     std::vector<double> he_a(4 * (size_t)nb);
     for (int h = 0; h < nb; ++h)
@@ -291,11 +302,6 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
       for (int k = 0; k < 3; ++k) xyz[(size_t)k * nn + i] = m->xyz[3 * (size_t)i + k];
     std::vector<double> vol(m->vol, m->vol + nn);
     c.h_bc_type.assign(m->bc_type, m->bc_type + nt);
-    // hard-set BC types overwrite boundary node states inside the Jacobian
-    for (int h = 0; h < nb; ++h) {
-      const int ty = c.h_bc_type[m->bfactag[h]];
-      if (ty == 1 /* dirichlet */ || ty == 7 /* sonicInflow */ || ty == 4 /* noSlip */) c.has_hardset = true;
-    }
     std::vector<double> qref(6 * (size_t)nt, 0.0);
     for (int t = 0; t < nt; ++t)
       for (int k = 0; k < 5; ++k) qref[(size_t)k * nt + t] = m->qref[5 * (size_t)t + k];
@@ -367,6 +373,7 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
       swidth[k] = wl + wh;
       sbase[k] = (int)slots;
       slots += wl + wh;
+      c.max_swidth = std::max(c.max_swidth, wl + wh);
     }
     if (slots * kW * 25 > (1LL << 40)) throw std::runtime_error("pcfd_create: matrix too large");
     c.nslot_s = slots;
@@ -404,6 +411,17 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     dput(c, &d.he_ptr, he_ptr);
     dput(c, &d.he_id, he_id);
     dput(c, &d.he_tag, he_tag);
+    dput(c, &d.he_node, he_node);
+    {
+      std::vector<int4> desc(nb);
+      for (int p = 0; p < nb; ++p) {
+        const int h = he_id[p], tag = m->bfactag[h];
+        desc[p] = int4{h, tag, m->bc_type[tag], he_nrm[h]};
+      }
+      dput(c, &d.he_desc, desc);
+    }
+    dput(c, &d.rst, rst);
+    if (c.nrst > 0) dalloc(c, &d.seen, 5 * (size_t)nb);
     dput(c, &d.he_a, he_a);
     dput(c, &d.bnd_nodes, bnd);
     dput(c, &d.bidx, bidx);
@@ -412,7 +430,6 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     dput(c, &d.bc_type, c.h_bc_type);
     dput(c, &d.qref, qref);
     dput(c, &d.twall, twall);
-    dput(c, &d.he_nrm, he_nrm);
     dput(c, &d.spos, spos);
     dalloc(c, &d.q, 5 * (size_t)c.ntot);
     dalloc(c, &d.grad, 27 * (size_t)nn);

@@ -11,6 +11,7 @@
 // (common.h): the s-th neighbours of 64 consecutive nodes are contiguous.
 #include <stdexcept>
 
+#include "boundary.h"
 #include "common.h"
 #include "physics.h"
 #include "scan.h"
@@ -57,75 +58,110 @@ void launch_lsq_moments(Ctx& c) {
 }
 
 // ---------------------------------------------------------------------------
-// UpdateBCs (ucs/bc.tcc:1399-1457): one thread per boundary node walks its
-// half-edges in half-edge order, so a Dirichlet/sonic-inflow overwrite of the
-// node state is seen by the node's later half-edges exactly as in the
-// reference's sequential loop.  Each phantom is written by its owner only.
-__global__ void __launch_bounds__(kBlock) k_update_bcs(int nbnd, int nnode, int ntot, int ntag,
-                                                      const int* __restrict__ bnd_nodes,
-                                                      const int* __restrict__ he_ptr, const int* __restrict__ he_id,
-                                                      const int* __restrict__ he_tag,
-                                                      const double* __restrict__ he_a, int nbnode,
-                                                      const int* __restrict__ bc_type,
-                                                      const double* __restrict__ qref,
-                                                      const double* __restrict__ twall,
-                                                      const int* __restrict__ he_nrm, double gamma,
-                                                      double* __restrict__ q) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nbnd) return;
-  int i = bnd_nodes[t];
-  double QL[5];
+// UpdateBCs (ucs/bc.tcc:1399-1457).  The reference walks the half-edges in
+// order; a Dirichlet / sonic-inflow or noSlip half-edge resets its node's own
+// state, which the node's later half-edges then see.  The characteristic
+// states (ten sub-iterations in series) are what costs, and they change
+// nothing but their phantom, so every half-edge has a thread for them.  On the
+// nodes that have resetting half-edges, k_bnd_resets first walks the
+// half-edges through the resets alone, sets those half-edges' phantoms and
+// leaves the state every half-edge of the node sees in `seen`.
+// (With one thread a node for everything: 118 us on the 74k-node bump, 123 us
+// on the 36k-node plate, 29 us on the 5.7k-node wedge; now 41, 28 + 11 and 7 + 8
+// us, beside the Jacobian rows in the first two.)
+//
+// JAC: the Jacobian's re-evaluation, which keeps the interior states for its
+// rows to read; the reset states go to Qb, and q's interior part is committed
+// later.
+template <bool JAC>
+__global__ void __launch_bounds__(kBndBlock) k_bnd_resets(BndArgs A, double* __restrict__ Qb) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= A.nrst) return;
+  const int bt = A.rst[t], i = A.bnd_nodes[bt];
+  double QL[5], Q0[5];
 #pragma unroll
-  for (int k = 0; k < 5; ++k) QL[k] = q[k * ntot + i];
-  double Q0[5] = {QL[0], QL[1], QL[2], QL[3], QL[4]};
-  for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) {
-    int h = he_id[p];
-    int tag = he_tag[h];
-    int ph = nnode + h;
-    double a[4] = {he_a[h], he_a[nbnode + h], he_a[2 * nbnode + h], he_a[3 * nbnode + h]};
-    double QR[5], Qr[5];
+  for (int k = 0; k < 5; ++k) Q0[k] = QL[k] = A.q[k * A.ntot + i];
+  const int p1 = A.he_ptr[i + 1];
+  for (int p0 = A.he_ptr[i]; p0 < p1; p0 += 4) {
+    // four descriptors at a time, so that their loads overlap
+    int4 d[4];
 #pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      QR[k] = q[k * ntot + ph];
-      Qr[k] = qref[k * ntag + tag];
-    }
-    double pref = qref[5 * ntag + tag];
-    const int type = bc_type[tag];
-    if (type == BC_NOSLIP) {
-      // hard-set wall node (adiabatic walls read the wall-normal neighbour
-      // as it stands before this update)
-      const double tw = twall[tag];
-      const int nn = he_nrm[h];
-      if (tw < 0.0 && nn < 0) continue;
-      double nQ[5] = {0, 0, 0, 0, 0};
-      if (tw < 0.0) {
+    for (int u = 0; u < 4; ++u) d[u] = A.he_desc[p0 + u < p1 ? p0 + u : p0];
 #pragma unroll
-        for (int k = 0; k < 5; ++k) nQ[k] = q[k * ntot + nn];
+    for (int u = 0; u < 4; ++u) {
+      const int p = p0 + u;
+      if (p >= p1) break;
+      const int tag = d[u].y, type = d[u].z, nn = d[u].w, ph = A.nnode + d[u].x;
+      if (type == BC_NOSLIP) {
+        // hard-set wall node (adiabatic walls read the wall-normal neighbour
+        // as it stands before this update)
+        const double tw = A.twall[tag];
+        if (!(tw < 0.0 && nn < 0)) {
+          double nQ[5] = {0, 0, 0, 0, 0}, QR[5];
+#pragma unroll
+          for (int k = 0; k < 5; ++k) QR[k] = A.q[k * A.ntot + ph];
+          if (tw < 0.0) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) nQ[k] = A.q[k * A.ntot + nn];
+          }
+          noslip_state(QL, QR, tw, nQ, A.gamma);
+#pragma unroll
+          for (int k = 0; k < 5; ++k) A.q[k * A.ntot + ph] = QR[k];
+        }
+      } else if (is_dirichlet(type)) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+          QL[k] = A.qref[k * A.ntag + tag];
+          A.q[k * A.ntot + ph] = QL[k];
+        }
       }
-      noslip_state(QL, QR, tw, nQ, gamma);
 #pragma unroll
-      for (int k = 0; k < 5; ++k) q[k * ntot + ph] = QR[k];
-    } else if (is_dirichlet(type)) {
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        QL[k] = Qr[k];
-        q[k * ntot + ph] = Qr[k];
-      }
-    } else if (bc_state(type, QL, QR, Qr, pref, a, gamma)) {
-#pragma unroll
-      for (int k = 0; k < 5; ++k) q[k * ntot + ph] = QR[k];
+      for (int k = 0; k < 5; ++k) A.seen[k * A.nbnode + p] = QL[k];
     }
   }
 #pragma unroll
-  for (int k = 0; k < 5; ++k)
-    if (QL[k] != Q0[k]) q[k * ntot + i] = QL[k];
+  for (int k = 0; k < 5; ++k) {
+    if (JAC) Qb[(long long)bt * 5 + k] = QL[k];
+    else if (QL[k] != Q0[k]) A.q[k * A.ntot + i] = QL[k];
+  }
+}
+
+__global__ void __launch_bounds__(kBndBlock) k_update_bcs(BndArgs A) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= A.nbnode) return;
+  const int4 d = A.he_desc[p];
+  const int h = d.x, tag = d.y, type = d.z, ph = A.nnode + h;
+  if (type == BC_NOSLIP || is_dirichlet(type)) return;  // set by k_bnd_resets
+  double QL[5], QR[5], Qr[5];
+  bnd_seen(A, p, QL);
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    QR[k] = A.q[k * A.ntot + ph];
+    Qr[k] = A.qref[k * A.ntag + tag];
+  }
+  const double a[4] = {A.he_a[h], A.he_a[A.nbnode + h], A.he_a[2 * A.nbnode + h], A.he_a[3 * A.nbnode + h]};
+  if (bc_state(type, QL, QR, Qr, A.qref[5 * A.ntag + tag], a, A.gamma)) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) A.q[k * A.ntot + ph] = QR[k];
+  }
+}
+
+BndArgs bnd_args(Ctx& c) {
+  return BndArgs{c.nbnd, c.nnode, c.ntot, c.ntag, c.nbnode, c.nrst, c.d.bnd_nodes, c.d.rst, c.d.he_ptr,
+                 c.d.he_node, c.d.he_desc, c.d.he_a, c.d.qref, c.d.twall, c.prm.gamma, c.d.q, c.d.seen};
+}
+
+void launch_bnd_resets(Ctx& c, hipStream_t s, double* Qb) {
+  if (c.nrst == 0) return;
+  hipLaunchKernelGGL(Qb ? k_bnd_resets<true> : k_bnd_resets<false>, dim3(nblk(c.nrst, kBndBlock)), dim3(kBndBlock), 0,
+                     s, bnd_args(c), Qb);
+  PCFD_HIP(hipGetLastError());
 }
 
 void launch_update_bcs(Ctx& c) {
   if (c.nbnd == 0) return;
-  hipLaunchKernelGGL(k_update_bcs, dim3(nblk(c.nbnd)), dim3(kBlock), 0, c.stream, c.nbnd, c.nnode, c.ntot,
-                     c.ntag, c.d.bnd_nodes, c.d.he_ptr, c.d.he_id, c.d.he_tag, c.d.he_a, c.nbnode, c.d.bc_type,
-                     c.d.qref, c.d.twall, c.d.he_nrm, c.prm.gamma, c.d.q);
+  launch_bnd_resets(c, c.stream, nullptr);
+  hipLaunchKernelGGL(k_update_bcs, dim3(nblk(c.nbnode, kBndBlock)), dim3(kBndBlock), 0, c.stream, bnd_args(c));
   PCFD_HIP(hipGetLastError());
 }
 

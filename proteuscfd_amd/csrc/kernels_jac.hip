@@ -15,28 +15,22 @@
 // (plain) or float (chosen form); the differences are always taken in FP64.
 #include <stdexcept>
 
+#include "boundary.h"
 #include "common.h"
 #include "physics.h"
 
 namespace pcfd {
 
 struct JacArgs {
-  int nnode, ntot, ntag, nbnode, nrow_pad, sym2d;
+  int nnode, ntot, nrow_pad, sym2d;
   double gamma;
   const int *gwidth, *gbase, *gcol, *gslot;
   const double* gnrm;
   long long gstride;
-  const int *he_ptr, *he_id, *he_tag;
-  const double* he_a;
-  const int* bc_type;
-  const double* qref;
   const double *vol, *dt;
-  double* q;
+  const double* q;
   const int *srow, *sbase;
   const double* xyz;       // SoA, for the viscous directional weights
-  const double* twall;     // per tag, noSlip walls
-  const int* he_nrm;       // per half-edge, wall-normal neighbour (noSlip)
-  int viscous;
   ViscParams vp;
   int flux_alg;            // 1: algebraic flux (generic form only)
   int centred;             // 1: centred differences, jacobianFieldType 1 (generic form only)
@@ -61,10 +55,15 @@ __device__ __forceinline__ void perturb(const double* Q, int c, double h, double
   for (int k = 0; k < 5; ++k) QP[k] = Q[k] + (k == c ? h : 0.0);
 }
 
-// Boundary half-edges (Bkernel_NumJac), sequential per boundary node, five
-// lanes per node as in k_jacobian.  Writes the node's boundary part of the
-// diagonal block to Db[t*25 + r*5 + c] (t = boundary-node index) and the
-// re-evaluated phantom states (lane 0).
+// Boundary half-edges (Bkernel_NumJac).  k_bnd_resets has walked the nodes'
+// resets; then every half-edge has a thread for its boundary state and
+// unperturbed flux (k_jac_bnd_base), every (half-edge, column) one for the
+// perturbed evaluation (k_jac_bnd_cols), and k_jac_bnd_sum adds a node's
+// half-edges in their order into its part Db of the diagonal block
+// (Db[t*25 + r*5 + c], t = boundary-node index).  One thread a (node, column)
+// that walked the half-edges took 95 us on the 386 boundary nodes of the 8^3
+// bump, 126 us on the 36k-node plate, 259 us on the 416k-node one; the four
+// passes take 36, 60 and 160 us.
 //
 // With A.bcentred (Bkernel_NumJac_Centered, ucs/jacobian.tcc:538-640, at the
 // default jacobianBoundaryEval 0) column c is (F(q+h e_c, BC(q+h e_c)) -
@@ -77,170 +76,105 @@ __device__ __forceinline__ void bnd_down(const double* QL, const double* QR, int
   perturb(QL, c, -1.0e-8, QPD);
   num_flux<ALG>(QPD, QR, a, gamma, sym2d, fD);
 }
+// rec[p]: the boundary state QR and the flux the columns difference against
+// (one-sided form), or for a centred Dirichlet half-edge the +h side's flux
 template <bool ALG>
-__global__ void __launch_bounds__(kBlock) k_jac_boundary(JacArgs A, const int* __restrict__ bnd_nodes, int nbnd,
-                                                        double* __restrict__ Db, double* __restrict__ Qb) {
-  const int lane64 = threadIdx.x & 63;
-  if (lane64 >= 60) return;
-  const int t = ((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * 12 + lane64 / 5;
-  const int c = lane64 % 5;
-  if (t >= nbnd) return;
-  const int i = bnd_nodes[t];
-  const double h = 1.0e-8;
-  const double gamma = A.gamma;
-  const bool cen = A.bcentred != 0;
-  const double w = cen ? kInv2H : kInvH;
-  double Dc[5] = {0, 0, 0, 0, 0};
-  const int p0 = A.he_ptr[i], p1 = A.he_ptr[i + 1];
-  // A node whose half-edges are all of types that leave its own state alone
-  // (no noSlip / Dirichlet re-set) sees the same unperturbed phantom state
-  // and flux in its five lanes: at every fifth half-edge lane c evaluates
-  // them for half-edge p + c (and writes that phantom), and each lane reads
-  // half-edge p's from lane (p - p0) % 5 of its group.
-  bool plain = true;
-  for (int p = p0; p < p1; ++p) {
-    const int type = A.bc_type[A.he_tag[A.he_id[p]]];
-    if (type == BC_NOSLIP || is_dirichlet(type)) plain = false;
+__global__ void __launch_bounds__(kBndBlock) k_jac_bnd_base(BndArgs B, int sym2d, int cen, double* __restrict__ rec) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= B.nbnode) return;
+  const int4 d = B.he_desc[p];
+  const int h = d.x, tag = d.y, type = d.z, ph = B.nnode + h;
+  const double a[4] = {B.he_a[h], B.he_a[B.nbnode + h], B.he_a[2 * B.nbnode + h], B.he_a[3 * B.nbnode + h]};
+  double QL[5], QR[5], Qr[5];
+  bnd_seen(B, p, QL);
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    QR[k] = B.q[k * B.ntot + ph];
+    Qr[k] = B.qref[k * B.ntag + tag];
   }
-  if (plain) {
-    double QL[5];
+  // noSlip and Dirichlet phantoms are set by k_bnd_resets
+  if (type != BC_NOSLIP && !is_dirichlet(type) && bc_state(type, QL, QR, Qr, B.qref[5 * B.ntag + tag], a, B.gamma)) {
 #pragma unroll
-    for (int k = 0; k < 5; ++k) QL[k] = A.q[k * A.ntot + i];
-    const int g0 = lane64 - c;
-    double fSg[5] = {0, 0, 0, 0, 0}, QRg[5] = {0, 0, 0, 0, 0};
-    for (int p = p0; p < p1; ++p) {
-      const int k5 = (p - p0) % 5;
-      if (k5 == 0 && p + c < p1) {
-        const int hc = A.he_id[p + c];
-        const int tc = A.he_tag[hc];
-        const double ac[4] = {A.he_a[hc], A.he_a[A.nbnode + hc], A.he_a[2 * A.nbnode + hc],
-                              A.he_a[3 * A.nbnode + hc]};
-        double Qr[5];
+    for (int k = 0; k < 5; ++k) B.q[k * B.ntot + ph] = QR[k];
+  }
+  double fS[5] = {0, 0, 0, 0, 0};
+  if (!cen || is_dirichlet(type)) num_flux<ALG>(QL, QR, a, B.gamma, sym2d, fS);
 #pragma unroll
-        for (int k = 0; k < 5; ++k) {
-          QRg[k] = A.q[k * A.ntot + A.nnode + hc];
-          Qr[k] = A.qref[k * A.ntag + tc];
-        }
-        if (bc_state(A.bc_type[tc], QL, QRg, Qr, A.qref[5 * A.ntag + tc], ac, gamma)) {
+  for (int k = 0; k < 5; ++k) {
+    rec[(long long)p * 10 + k] = QR[k];
+    rec[(long long)p * 10 + 5 + k] = fS[k];
+  }
+}
+
+template <bool ALG>
+__global__ void __launch_bounds__(kBndBlock) k_jac_bnd_cols(BndArgs B, int sym2d, int cen,
+                                                           const double* __restrict__ rec,
+                                                           double* __restrict__ col) {
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= 5LL * B.nbnode) return;
+  const int p = (int)(t / 5), c = (int)(t % 5);
+  const int4 d = B.he_desc[p];
+  const int h = d.x, tag = d.y, type = d.z;
+  const double a[4] = {B.he_a[h], B.he_a[B.nbnode + h], B.he_a[2 * B.nbnode + h], B.he_a[3 * B.nbnode + h]};
+  const double w = cen ? kInv2H : kInvH;
+  double QL[5], QR[5], fS[5], fL[5], Dc[5] = {0, 0, 0, 0, 0};
+  bnd_seen(B, p, QL);
 #pragma unroll
-          for (int k = 0; k < 5; ++k) A.q[k * A.ntot + A.nnode + hc] = QRg[k];
-        }
-        if (!cen) num_flux<ALG>(QL, QRg, ac, gamma, A.sym2d, fSg);
+  for (int k = 0; k < 5; ++k) {
+    QR[k] = rec[(long long)p * 10 + k];
+    fS[k] = rec[(long long)p * 10 + 5 + k];
+  }
+  bool live = true;
+  if (is_dirichlet(type)) {
+    // QL = QR = Qref and every perturbed evaluation resets both to Qref, so
+    // the one-sided contribution is exactly zero; the centred one keeps its
+    // -h side: (F(Qref, Qref) - F(Qref - h e_c, Qref)) / 2h
+    live = cen != 0;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) fL[k] = fS[k];
+  } else {
+    double QPL[5], QPR[5] = {QR[0], QR[1], QR[2], QR[3], QR[4]};
+    perturb(QL, c, 1.0e-8, QPL);
+    if (type == BC_NOSLIP) {
+      // CalculateBoundaryVariables hard-sets the wall node for the base and
+      // for every perturbed state (ucs/jacobian.tcc:484-512)
+      const double tw = B.twall[tag];
+      const int nn = d.w;
+      live = !(tw < 0.0 && nn < 0);
+      double nQ[5] = {0, 0, 0, 0, 0};
+      if (tw < 0.0 && live) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) nQ[k] = B.q[k * B.ntot + nn];
       }
-      double fS[5], QR[5];
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        fS[k] = __shfl(fSg[k], g0 + k5);
-        QR[k] = __shfl(QRg[k], g0 + k5);
-      }
-      const int hh = A.he_id[p];
-      const int tag = A.he_tag[hh];
-      const double a[4] = {A.he_a[hh], A.he_a[A.nbnode + hh], A.he_a[2 * A.nbnode + hh], A.he_a[3 * A.nbnode + hh]};
+      noslip_state(QPL, QPR, tw, nQ, B.gamma);
+    } else {
       double Qr[5];
 #pragma unroll
-      for (int k = 0; k < 5; ++k) Qr[k] = A.qref[k * A.ntag + tag];
-      double QPL[5];
-      perturb(QL, c, h, QPL);
-      double QPR[5] = {QR[0], QR[1], QR[2], QR[3], QR[4]};
-      bc_state(A.bc_type[tag], QPL, QPR, Qr, A.qref[5 * A.ntag + tag], a, gamma);
-      double fL[5];
-      num_flux<ALG>(QPL, QPR, a, gamma, A.sym2d, fL);
-      if (cen) bnd_down<ALG>(QL, QR, c, a, gamma, A.sym2d, fS);
-#pragma unroll
-      for (int rr = 0; rr < 5; ++rr) Dc[rr] += (fL[rr] - fS[rr]) * w;
+      for (int k = 0; k < 5; ++k) Qr[k] = B.qref[k * B.ntag + tag];
+      bc_state(type, QPL, QPR, Qr, B.qref[5 * B.ntag + tag], a, B.gamma);
     }
-    if (c == 0) {
+    num_flux<ALG>(QPL, QPR, a, B.gamma, sym2d, fL);
+  }
+  if (live) {
+    if (cen) bnd_down<ALG>(QL, QR, c, a, B.gamma, sym2d, fS);
 #pragma unroll
-      for (int k = 0; k < 5; ++k) Qb[(long long)t * 5 + k] = QL[k];
-    }
-  } else {
-    double QL[5];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) QL[k] = A.q[k * A.ntot + i];
-    for (int p = p0; p < p1; ++p) {
-      const int hh = A.he_id[p];
-      const int tag = A.he_tag[hh];
-      const int type = A.bc_type[tag];
-      const int ph = A.nnode + hh;
-      const double a[4] = {A.he_a[hh], A.he_a[A.nbnode + hh], A.he_a[2 * A.nbnode + hh],
-                           A.he_a[3 * A.nbnode + hh]};
-      double QR[5], Qr[5];
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        QR[k] = A.q[k * A.ntot + ph];
-        Qr[k] = A.qref[k * A.ntag + tag];
-      }
-      const double pref = A.qref[5 * A.ntag + tag];
-      if (type == BC_NOSLIP) {
-        // CalculateBoundaryVariables hard-sets the wall node for the base
-        // and for every perturbed state (ucs/jacobian.tcc:484-512)
-        const double tw = A.twall[tag];
-        const int nn = A.he_nrm[hh];
-        if (tw < 0.0 && nn < 0) continue;
-        double nQ[5] = {0, 0, 0, 0, 0};
-        if (tw < 0.0) {
-#pragma unroll
-          for (int k = 0; k < 5; ++k) nQ[k] = A.q[k * A.ntot + nn];
-        }
-        noslip_state(QL, QR, tw, nQ, gamma);
-        if (c == 0) {
-#pragma unroll
-          for (int k = 0; k < 5; ++k) A.q[k * A.ntot + ph] = QR[k];
-        }
-        double fS[5], fL[5], QPL[5];
-        if (cen) bnd_down<ALG>(QL, QR, c, a, gamma, A.sym2d, fS);
-        else num_flux<ALG>(QL, QR, a, gamma, A.sym2d, fS);
-        perturb(QL, c, h, QPL);
-        double QPR[5] = {QR[0], QR[1], QR[2], QR[3], QR[4]};
-        noslip_state(QPL, QPR, tw, nQ, gamma);
-        num_flux<ALG>(QPL, QPR, a, gamma, A.sym2d, fL);
-#pragma unroll
-        for (int rr = 0; rr < 5; ++rr) Dc[rr] += (fL[rr] - fS[rr]) * w;
-        continue;
-      }
-      if (is_dirichlet(type)) {
-        // QL = QR = Qref and every perturbed evaluation resets both to Qref,
-        // so the one-sided contribution is exactly zero; the centred one keeps
-        // its -h side: (F(Qref, Qref) - F(Qref - h e_c, Qref)) / 2h
-#pragma unroll
-        for (int k = 0; k < 5; ++k) {
-          QL[k] = Qr[k];
-          if (c == 0) A.q[k * A.ntot + ph] = Qr[k];
-        }
-        if (cen) {
-          double fU[5], fD[5];
-          num_flux<ALG>(Qr, Qr, a, gamma, A.sym2d, fU);
-          bnd_down<ALG>(Qr, Qr, c, a, gamma, A.sym2d, fD);
-#pragma unroll
-          for (int rr = 0; rr < 5; ++rr) Dc[rr] += (fU[rr] - fD[rr]) * w;
-        }
-        continue;
-      }
-      if (bc_state(type, QL, QR, Qr, pref, a, gamma) && c == 0) {
-#pragma unroll
-        for (int k = 0; k < 5; ++k) A.q[k * A.ntot + ph] = QR[k];
-      }
-      double fS[5];
-      if (cen) bnd_down<ALG>(QL, QR, c, a, gamma, A.sym2d, fS);
-      else num_flux<ALG>(QL, QR, a, gamma, A.sym2d, fS);
-      double QPL[5];
-      perturb(QL, c, h, QPL);
-      double QPR[5] = {QR[0], QR[1], QR[2], QR[3], QR[4]};
-      bc_state(type, QPL, QPR, Qr, pref, a, gamma);
-      double fL[5];
-      num_flux<ALG>(QPL, QPR, a, gamma, A.sym2d, fL);
-#pragma unroll
-      for (int rr = 0; rr < 5; ++rr) Dc[rr] += (fL[rr] - fS[rr]) * w;
-    }
-    // the node state after the re-evaluation: the viscous Jacobian, which
-    // the reference runs after Bkernel_NumJac, sees it
-    if (c == 0) {
-#pragma unroll
-      for (int k = 0; k < 5; ++k) Qb[(long long)t * 5 + k] = QL[k];
-    }
+    for (int rr = 0; rr < 5; ++rr) Dc[rr] = (fL[rr] - fS[rr]) * w;
   }
 #pragma unroll
-  for (int rr = 0; rr < 5; ++rr) Db[(long long)t * 25 + rr * 5 + c] = Dc[rr];
+  for (int rr = 0; rr < 5; ++rr) col[t * 5 + rr] = Dc[rr];
+}
+
+// ... and the states of the nodes that no half-edge resets, as they stand, to Qb
+__global__ void __launch_bounds__(kBlock) k_jac_bnd_sum(BndArgs B, const double* __restrict__ col,
+                                                       double* __restrict__ Db, double* __restrict__ Qb) {
+  const long long t25 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t25 >= 25LL * B.nbnd) return;
+  const int t = (int)(t25 / 25), k = (int)(t25 % 25);  // k = column * 5 + row, as col stores them
+  const int i = B.bnd_nodes[t];
+  if (k < 5 && B.he_node[B.he_ptr[i]] >= 0) Qb[5LL * t + k] = B.q[k * B.ntot + i];
+  double s = 0.0;
+  for (int p = B.he_ptr[i]; p < B.he_ptr[i + 1]; ++p) s += col[25LL * p + k];
+  Db[25LL * t + (k % 5) * 5 + k / 5] = s;
 }
 
 // the edge flux of the generic form, evaluated from node i's side (x is
@@ -457,67 +391,64 @@ __global__ void __launch_bounds__(kBlock) k_commit_hardset(int nbnd, int ntot, c
 // half-edge, BlankSubRow (ucs/crsmatrix.tcc:525-541) zeroes sub-row r of
 // every block of the row and puts 1 on the diagonal; isothermal walls then
 // tie the energy change to the density change, adiabatic walls tie density
-// and energy to the wall-normal neighbour.  One thread per boundary node.
+// and energy to the wall-normal neighbour.  Of a node's half-edges the last
+// noSlip one decides sub-rows 1-4 and the last adiabatic one sub-row 0, so one
+// thread per (boundary node, slot) writes the end state (slot `w` of the grid:
+// the diagonal).  One thread a node that replayed every half-edge: 71 us on
+// the 36k-node plate; now 8 us.
 template <typename T>
-__device__ __forceinline__ void blank_subrow(T* Moff, T* Dg, const int* scol, long long sb, int w, int chunk,
-                                             int lane, int sub) {
-  for (int s = 0; s < w; ++s) {
-    if (scol[(sb + s) * kW + lane] < 0) continue;  // padding of either run
-    T* blk = Moff + (sb + s) * 25 * kW + lane;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) blk[(sub * 5 + k) * kW] = (T)0;
-  }
-  T* dg = Dg + (long long)chunk * 25 * kW + lane;
-#pragma unroll
-  for (int k = 0; k < 5; ++k) dg[(sub * 5 + k) * kW] = (T)0;
-  dg[(sub * 5 + sub) * kW] = (T)1;
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock) k_noslip_rows(JacArgs A, const int* __restrict__ bnd_nodes, int nbnd,
-                                                       const int* __restrict__ spos, const int* __restrict__ swidth,
+__global__ void __launch_bounds__(kBlock) k_noslip_rows(BndArgs B, const int* __restrict__ spos,
+                                                       const int* __restrict__ swidth, const int* __restrict__ sbase,
                                                        const int* __restrict__ scol, T* __restrict__ Moff,
                                                        T* __restrict__ Dg) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nbnd) return;
-  const int i = bnd_nodes[t];
-  const int r = spos[i];
-  const int chunk = r >> 6, lane = r & 63;
-  const long long sb = A.sbase[chunk];
-  const int w = swidth[chunk];
-  const double g = A.gamma;
-  for (int p = A.he_ptr[i]; p < A.he_ptr[i + 1]; ++p) {
-    const int hh = A.he_id[p];
-    const int tag = A.he_tag[hh];
-    if (A.bc_type[tag] != BC_NOSLIP) continue;
-    const double tw = A.twall[tag];
-    blank_subrow(Moff, Dg, scol, sb, w, chunk, lane, 1);
-    blank_subrow(Moff, Dg, scol, sb, w, chunk, lane, 2);
-    blank_subrow(Moff, Dg, scol, sb, w, chunk, lane, 3);
-    if (tw < 0.0) {
-      blank_subrow(Moff, Dg, scol, sb, w, chunk, lane, 0);
-      blank_subrow(Moff, Dg, scol, sb, w, chunk, lane, 4);
-      const int nn = A.he_nrm[hh];
-      const int rn = nn >= 0 ? spos[nn] : -1;
-      for (int s = 0; rn >= 0 && s < w; ++s) {
-        if (scol[(sb + s) * kW + lane] != rn) continue;
-        T* blk = Moff + (sb + s) * 25 * kW + lane;
-        blk[0 * kW] = (T)-1.0;
-        blk[24 * kW] = (T)-1.0;
-      }
-    } else {
-      const double v2 = 0.0;
-      blank_subrow(Moff, Dg, scol, sb, w, chunk, lane, 4);
-      Dg[(long long)chunk * 25 * kW + lane + 20 * kW] = (T)(-(tw / (g * (g - 1.0)) + 0.5 * v2));
-    }
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= B.nbnd) return;
+  const int i = B.bnd_nodes[t];
+  if (B.he_node[B.he_ptr[i]] >= 0) return;  // no half-edge resets it
+  int last = -1, adia = -1;  // list positions
+  for (int p = B.he_ptr[i]; p < B.he_ptr[i + 1]; ++p) {
+    if (B.he_desc[p].z != BC_NOSLIP) continue;
+    last = p;
+    if (B.twall[B.he_desc[p].y] < 0.0) adia = p;
   }
+  if (last < 0) return;
+  const int r = spos[i];
+  const int chunk = r >> 6, lane = r & 63, s = blockIdx.y;
+  const bool last_adia = last == adia;
+  if (s == (int)gridDim.y - 1) {  // the diagonal block
+    T* dg = Dg + (long long)chunk * 25 * kW + lane;
+    const double tw = B.twall[B.he_desc[last].y], g = B.gamma, v2 = 0.0;
+#pragma unroll
+    for (int rr = 0; rr < 5; ++rr) {
+      if (rr == 0 && adia < 0) continue;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) dg[(rr * 5 + k) * kW] = (T)(k == rr ? 1 : 0);
+    }
+    if (!last_adia) dg[20 * kW] = (T)(-(tw / (g * (g - 1.0)) + 0.5 * v2));
+    return;
+  }
+  if (s >= swidth[chunk]) return;
+  const long long sb = (long long)sbase[chunk] + s;
+  const int col = scol[sb * kW + lane];
+  if (col < 0) return;  // padding
+  T* blk = Moff + sb * 25 * kW + lane;
+#pragma unroll
+  for (int rr = 0; rr < 5; ++rr) {
+    if (rr == 0 && adia < 0) continue;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) blk[(rr * 5 + k) * kW] = (T)0;
+  }
+  // the last adiabatic half-edge's wall-normal neighbour
+  const int nn = adia >= 0 ? B.he_desc[adia].w : -1;
+  if (nn < 0 || col != spos[nn]) return;
+  blk[0 * kW] = (T)-1.0;
+  if (last_adia) blk[24 * kW] = (T)-1.0;
 }
 
 static JacArgs jac_args(Ctx& c) {
   const pcfd_params& p = c.prm;
-  return JacArgs{c.nnode, c.ntot, c.ntag, c.nbnode, c.nrow_pad, p.symmetry2d, p.gamma, c.d.gwidth, c.d.gbase,
-                 c.d.gcol, c.d.gslot, c.d.gnrm, c.nslot_g * kW, c.d.he_ptr, c.d.he_id, c.d.he_tag, c.d.he_a, c.d.bc_type,
-                 c.d.qref, c.d.vol, c.d.dt, c.d.q, c.d.srow, c.d.sbase, c.d.xyz, c.d.twall, c.d.he_nrm, p.viscous,
+  return JacArgs{c.nnode, c.ntot, c.nrow_pad, p.symmetry2d, p.gamma, c.d.gwidth, c.d.gbase, c.d.gcol, c.d.gslot,
+                 c.d.gnrm, c.nslot_g * kW, c.d.vol, c.d.dt, c.d.q, c.d.srow, c.d.sbase, c.d.xyz,
                  ViscParams{p.gamma, p.re_tilde, p.prandtl, p.prandtl_t, p.sutherland_s, p.symmetry2d},
                  p.flux_type == PCFD_FLUX_ALGEBRAIC ? 1 : 0, p.jac_field_type == 1 ? 1 : 0,
                  p.jac_boundary_type == 1 ? 1 : 0};
@@ -525,9 +456,15 @@ static JacArgs jac_args(Ctx& c) {
 
 static void jac_boundary(Ctx& c, const JacArgs& A, hipStream_t s) {
   if (c.nbnd == 0) return;
-  const long long bw = (c.nbnd + 11) / 12;
-  hipLaunchKernelGGL(A.flux_alg ? k_jac_boundary<true> : k_jac_boundary<false>, dim3(nblk(bw * kW)), dim3(kBlock),
-                     0, s, A, c.d.bnd_nodes, c.nbnd, c.d.jdb, c.d.jqb);
+  launch_bnd_resets(c, s, c.d.jqb);
+  const BndArgs B = bnd_args(c);
+  hipLaunchKernelGGL(A.flux_alg ? k_jac_bnd_base<true> : k_jac_bnd_base<false>, dim3(nblk(c.nbnode, kBndBlock)),
+                     dim3(kBndBlock), 0, s, B, A.sym2d, A.bcentred, c.d.jhe);
+  PCFD_HIP(hipGetLastError());
+  hipLaunchKernelGGL(A.flux_alg ? k_jac_bnd_cols<true> : k_jac_bnd_cols<false>, dim3(nblk(5LL * c.nbnode, kBndBlock)),
+                     dim3(kBndBlock), 0, s, B, A.sym2d, A.bcentred, c.d.jhe, c.d.jcol);
+  PCFD_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_jac_bnd_sum, dim3(nblk(25LL * c.nbnd)), dim3(kBlock), 0, s, B, c.d.jcol, c.d.jdb, c.d.jqb);
   PCFD_HIP(hipGetLastError());
 }
 
@@ -556,14 +493,15 @@ static void jac_rows(Ctx& c, const JacArgs& A, hipStream_t s) {
   PCFD_HIP(hipGetLastError());
 }
 
-static void jac_noslip(Ctx& c, const JacArgs& A, hipStream_t s) {
+static void jac_noslip(Ctx& c, hipStream_t s) {
   if (!c.has_noslip) return;
+  const dim3 grid(nblk(c.nbnd), c.max_swidth + 1);
   if (c.prm.precision == PCFD_CHOSEN_FP32)
-    hipLaunchKernelGGL(k_noslip_rows<float>, dim3(nblk(c.nbnd)), dim3(kBlock), 0, s, A, c.d.bnd_nodes, c.nbnd,
-                       c.d.spos, c.d.swidth, c.d.scol, c.d.Mf, c.d.Df);
+    hipLaunchKernelGGL(k_noslip_rows<float>, grid, dim3(kBlock), 0, s, bnd_args(c), c.d.spos, c.d.swidth, c.d.sbase,
+                       c.d.scol, c.d.Mf, c.d.Df);
   else
-    hipLaunchKernelGGL(k_noslip_rows<double>, dim3(nblk(c.nbnd)), dim3(kBlock), 0, s, A, c.d.bnd_nodes, c.nbnd,
-                       c.d.spos, c.d.swidth, c.d.scol, c.d.Md, c.d.Dd);
+    hipLaunchKernelGGL(k_noslip_rows<double>, grid, dim3(kBlock), 0, s, bnd_args(c), c.d.spos, c.d.swidth,
+                       c.d.sbase, c.d.scol, c.d.Md, c.d.Dd);
   PCFD_HIP(hipGetLastError());
 }
 
@@ -575,7 +513,7 @@ void launch_jacobian(Ctx& c) {
   jac_boundary(c, A, c.stream);
   jac_rows(c, A, c.stream);
   jac_commit(c, c.stream);
-  jac_noslip(c, A, c.stream);
+  jac_noslip(c, c.stream);
   sub_end(c, 11);
 }
 
@@ -590,7 +528,7 @@ void launch_jacobian(Ctx& c) {
 void launch_jacobian_overlapped(Ctx& c) {
   JacArgs A = jac_args(c);
   jac_boundary(c, A, c.stream);
-  if (c.has_hardset && c.nbnd > 0) {
+  if (c.nrst > 0) {
     PCFD_HIP(hipMemcpyAsync(c.d.qjac, c.d.q, sizeof(double) * 5 * (size_t)c.ntot, hipMemcpyDeviceToDevice,
                             c.stream));
     A.q = c.d.qjac;
@@ -600,7 +538,7 @@ void launch_jacobian_overlapped(Ctx& c) {
   PCFD_HIP(hipStreamWaitEvent(c.stream2, c.ev_fork, 0));
   if (c.timing) PCFD_HIP(hipEventRecord(c.ev4, c.stream2));
   jac_rows(c, A, c.stream2);
-  jac_noslip(c, A, c.stream2);
+  jac_noslip(c, c.stream2);
   if (c.timing) PCFD_HIP(hipEventRecord(c.ev5, c.stream2));
   PCFD_HIP(hipEventRecord(c.ev_join, c.stream2));
   c.jac_pending = true;
