@@ -176,6 +176,84 @@ __device__ __forceinline__ long long gbase_of(const Gell& g, int i) {
   return (long long)g.base[i >> 6] * kW + (i & 63);
 }
 
+// Lanes per node of the edge passes.  A node's neighbours are a serial chain
+// of gathers and fluxes, so a mesh that leaves the chip idle takes four lanes
+// a node and a larger one two (us at 1 / 2 / 4 lanes): second-order residual
+// 50 / 36 / 31 (729 nodes), 78 / 60 / 64 (74k), 164 / 138 / 166 (275k); residual
+// with viscous fluxes 95 / 79 / 75 (36k), 406 / 381 / 486 (416k); time step 22 /
+// 14 / 11 (9k), 94 / 73 / 85 (416k).  The gradient's 27 sums cost more to combine:
+// 20 / 15 / 13 (9k), 27 / 23 / 28 (74k), 56 / 60 / 81 (275k).
+inline int lanes_per_node(int nnode) { return nnode <= 49152 ? 4 : 2; }
+inline int gradient_lanes(int nnode) { return nnode <= 49152 ? 4 : nnode <= 131072 ? 2 : 1; }
+
+// LPN (1, 2 or 4) adjacent lanes share a node and take alternate neighbours;
+// these move values among them with DPP quad permutes (no LDS).
+template <int CTRL>
+__device__ __forceinline__ double quad_perm(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+constexpr int kXor1 = 0xB1, kXor2 = 0x4E;  // lanes [1,0,3,2] and [2,3,0,1] of a quad
+
+// the value of lane U of the node's lanes
+template <int LPN, int U>
+__device__ __forceinline__ double lane_bcast(double v) {
+  if constexpr (LPN == 1) return v;
+  else if constexpr (LPN == 2) return quad_perm<U | (U << 2) | ((2 + U) << 4) | ((2 + U) << 6)>(v);
+  else return quad_perm<U * 0x55>(v);
+}
+
+// acc += the lanes' values, lane by lane: the order of one thread that takes
+// the neighbours one after the other
+template <int LPN, int N>
+__device__ __forceinline__ void lane_add(double* acc, const double* v) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) acc[k] += lane_bcast<LPN, 0>(v[k]);
+  if constexpr (LPN > 1) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) acc[k] += lane_bcast<LPN, 1>(v[k]);
+  }
+  if constexpr (LPN > 2) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) acc[k] += lane_bcast<LPN, 2>(v[k]);
+#pragma unroll
+    for (int k = 0; k < N; ++k) acc[k] += lane_bcast<LPN, 3>(v[k]);
+  }
+}
+
+// combine per-lane partial results: every lane ends with the same value
+template <int LPN, int N, typename OP>
+__device__ __forceinline__ void lane_reduce(double* v, OP op) {
+  if constexpr (LPN > 1) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = op(v[k], quad_perm<kXor1>(v[k]));
+  }
+  if constexpr (LPN > 2) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = op(v[k], quad_perm<kXor2>(v[k]));
+  }
+}
+template <int LPN, int N>
+__device__ __forceinline__ void lane_sum(double* v) {
+  lane_reduce<LPN, N>(v, [](double a, double b) { return a + b; });
+}
+template <int LPN, int N>
+__device__ __forceinline__ void lane_min(double* v) {
+  lane_reduce<LPN, N>(v, [](double a, double b) { return a < b ? a : b; });
+}
+template <int LPN, int N>
+__device__ __forceinline__ void lane_max(double* v) {
+  lane_reduce<LPN, N>(v, [](double a, double b) { return a > b ? a : b; });
+}
+template <int LPN>
+__device__ __forceinline__ bool lane_any(bool p) {
+  int v = p ? 1 : 0;
+  if constexpr (LPN > 1) v |= __builtin_amdgcn_update_dpp(0, v, kXor1, 0xf, 0xf, true);
+  if constexpr (LPN > 2) v |= __builtin_amdgcn_update_dpp(0, v, kXor2, 0xf, 0xf, true);
+  return v != 0;
+}
+
 // Per-block partial sums of b^2 for the residual norms: total and per
 // equation, reduced with a fixed-shape tree (deterministic), written to
 // red[k*gridDim.x + blk].  Every thread of the block must call it.

@@ -452,7 +452,7 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     dput(c, &d.swidth_lo, swidth_lo);
     dput(c, &d.sbase, sbase);
     dput(c, &d.scol, scol);
-    dalloc(c, &d.red, 6 * (size_t)std::max(nblk(nn), 1024));
+    dalloc(c, &d.red, 6 * (size_t)std::max(nblk(4LL * nn), 1024));
     dalloc(c, &d.red_out, 8);
     dalloc(c, &d.icount, 4);
     PCFD_HIP(hipMemset(d.grad, 0, 27 * sizeof(double) * (size_t)nn));

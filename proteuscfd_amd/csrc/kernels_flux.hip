@@ -1,12 +1,11 @@
 // Edge-loop kernels of the residual path, written as node gathers.
 //
 // The reference loops over edges and scatters both edge contributions into
-// node arrays (ucs/driver.tcc:5-67, 274-306).  Here one thread owns one node
-// and visits its incident edges in ascending neighbour order -- the same
-// order in which the reference's edge loop (edges sorted by (n0, n1))
-// reaches that node -- evaluating every edge function with the canonical
-// (n0, n1) argument order.  Both ends of an edge therefore see bit-identical
-// edge values, sums come out in the reference's order, and no
+// node arrays (ucs/driver.tcc:5-67, 274-306).  Here a few adjacent lanes own a
+// node and visit its incident edges in turn, evaluating every edge function
+// with the canonical (n0, n1) argument order.  Both ends of an edge therefore
+// see bit-identical edge values, residuals are summed in the reference's
+// order (the others combine the lanes' partial sums in a fixed one), and no
 // floating-point atomics are needed.  Neighbour lists use the gELL layout
 // (common.h): the s-th neighbours of 64 consecutive nodes are contiguous.
 #include <stdexcept>
@@ -189,52 +188,65 @@ __device__ __forceinline__ void grad_terms(const double* Q, double gm1, double g
 // bounds starting at 0 (:59-63), then the per-edge-end limiter value, the
 // minimum over the node's edges.  limit_node is the second part, given the
 // node's state, its first five gradient terms and the neighbour bounds.
-__device__ __forceinline__ void limit_node(int i, int nnode, int ntot, int type, double K3, double chi,
+template <int LPN>
+__device__ __forceinline__ void limit_node(int i, int sub, int nnode, int ntot, int type, double K3, double chi,
                                            const Gell& g, const double* __restrict__ xyz,
                                            const double* __restrict__ vol, const double* __restrict__ q,
                                            const double* qi, const double* gi, const double* qmin,
                                            const double* qmax, double* phi) {
-#pragma unroll
-  for (int k = 0; k < 5; ++k) phi[k] = 1.0;
   const long long b = gbase_of(g, i);
   const int w = g.width[i >> 6];
   double xi[3] = {xyz[i], xyz[nnode + i], xyz[2 * nnode + i]};
   const double ep2 = 6.0 * 3.141592653589793 * vol[i] * K3;
-  for (int s = 0; s < w; ++s) {
-    const int j = g.col[b + (long long)s * kW];
-    if (j < 0) break;
-    const bool left = i < j;
-    double xj[3] = {xyz[j], xyz[nnode + j], xyz[2 * nnode + j]};
-    double dx[3];
-    // dx = 0.5 (xR - xL) for the left end, its negation for the right end
-    if (left) { dx[0] = 0.5 * (xj[0] - xi[0]); dx[1] = 0.5 * (xj[1] - xi[1]); dx[2] = 0.5 * (xj[2] - xi[2]); }
-    else { dx[0] = -(0.5 * (xi[0] - xj[0])); dx[1] = -(0.5 * (xi[1] - xj[1])); dx[2] = -(0.5 * (xi[2] - xj[2])); }
+  int start = sub, step = LPN;
+  for (;;) {
+    bool nan = false;
 #pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      double qj = q[k * ntot + j];
-      double dQ = left ? (qj - qi[k]) : -(qi[k] - qj);
-      double Qh = extrap1(qi[k], dQ, gi[3 * k], gi[3 * k + 1], gi[3 * k + 2], dx, chi, 1.0);
-      double t;
-      if (type == 3) {
-        double DM = Qh - qi[k];
-        double DP;
-        if (left) DP = (Qh > qi[k]) ? qmax[k] - qi[k] : ((Qh < qi[k]) ? qmin[k] - qi[k] : 0.0);
-        else DP = (Qh > qi[k]) ? qmax[k] - qi[k] : qmin[k] - qi[k];
-        t = (DP * DP + ep2 + 2.0 * DM * DP) / (DP * DP + 2.0 * DM * DM + DM * DP + ep2);
-      } else {
-        t = 1.0;
-        if (Qh > qi[k]) t = (qmax[k] - qi[k]) / (Qh - qi[k]);
-        else if (Qh < qi[k]) t = (qmin[k] - qi[k]) / (Qh - qi[k]);
-        if (type == 2) {
-          t = (t * t + 2.0 * t) / (t * t + t + 2.0);
+    for (int k = 0; k < 5; ++k) phi[k] = 1.0;
+    for (int s = start; s < w; s += step) {
+      const int j = g.col[b + (long long)s * kW];
+      if (j < 0) break;
+      const bool left = i < j;
+      double xj[3] = {xyz[j], xyz[nnode + j], xyz[2 * nnode + j]};
+      double dx[3];
+      // dx = 0.5 (xR - xL) for the left end, its negation for the right end
+      if (left) { dx[0] = 0.5 * (xj[0] - xi[0]); dx[1] = 0.5 * (xj[1] - xi[1]); dx[2] = 0.5 * (xj[2] - xi[2]); }
+      else { dx[0] = -(0.5 * (xi[0] - xj[0])); dx[1] = -(0.5 * (xi[1] - xj[1])); dx[2] = -(0.5 * (xi[2] - xj[2])); }
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        double qj = q[k * ntot + j];
+        double dQ = left ? (qj - qi[k]) : -(qi[k] - qj);
+        double Qh = extrap1(qi[k], dQ, gi[3 * k], gi[3 * k + 1], gi[3 * k + 2], dx, chi, 1.0);
+        double t;
+        if (type == 3) {
+          double DM = Qh - qi[k];
+          double DP;
+          if (left) DP = (Qh > qi[k]) ? qmax[k] - qi[k] : ((Qh < qi[k]) ? qmin[k] - qi[k] : 0.0);
+          else DP = (Qh > qi[k]) ? qmax[k] - qi[k] : qmin[k] - qi[k];
+          t = (DP * DP + ep2 + 2.0 * DM * DP) / (DP * DP + 2.0 * DM * DM + DM * DP + ep2);
         } else {
-          t = dmax(0.0, t);
-          t = dmin(1.0, t);
+          t = 1.0;
+          if (Qh > qi[k]) t = (qmax[k] - qi[k]) / (Qh - qi[k]);
+          else if (Qh < qi[k]) t = (qmin[k] - qi[k]) / (Qh - qi[k]);
+          if (type == 2) {
+            t = (t * t + 2.0 * t) / (t * t + t + 2.0);
+          } else {
+            t = dmax(0.0, t);
+            t = dmin(1.0, t);
+          }
         }
+        phi[k] = dmin(phi[k], t);
+        nan |= t != t;
       }
-      phi[k] = dmin(phi[k], t);
     }
+    if (step == 1) return;
+    if (!lane_any<LPN>(nan)) break;
+    // what the running minimum keeps depends on a NaN's place among the
+    // edges: each lane walks them all, in order
+    start = 0;
+    step = 1;
   }
+  lane_min<LPN, 5>(phi);
 }
 
 struct LimArgs {  // the fused limiter's inputs and output (LIM = true)
@@ -247,7 +259,7 @@ struct LimArgs {  // the fused limiter's inputs and output (LIM = true)
 // With LIM the same kernel also forms the limiter (k_limiter's arithmetic):
 // the neighbour bounds come from the states the gradient loop reads, and the
 // per-edge limiter loop runs on the gradient still in registers.
-template <int NT, bool LIM>
+template <int NT, bool LIM, int LPN>
 __global__ void __launch_bounds__(kBlock) k_gradient(int nnode, int ntot, Gell g, const double* __restrict__ xyz,
                                                     const double* __restrict__ sw, const double* __restrict__ q,
                                                     const int* __restrict__ he_ptr, const int* __restrict__ he_id,
@@ -255,8 +267,8 @@ __global__ void __launch_bounds__(kBlock) k_gradient(int nnode, int ntot, Gell g
                                                     const double* __restrict__ he_a, int nbnode,
                                                     const int* __restrict__ bc_type, double gamma,
                                                     double* __restrict__ grad, LimArgs L) {
-  int i = xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= nnode) return;
+  const int i = (xcd_block() * blockDim.x + threadIdx.x) / LPN, sub = threadIdx.x % LPN;
+  if (i >= nnode) return;  // all lanes of a node together
   const double gm1 = gamma - 1.0;
   double gr[NT * 3];
 #pragma unroll
@@ -279,9 +291,10 @@ __global__ void __launch_bounds__(kBlock) k_gradient(int nnode, int ntot, Gell g
   grad_terms<NT>(Qi, gm1, gamma, ti);
   double xi = xyz[i], yi = xyz[nnode + i], zi = xyz[2 * nnode + i];
   double qmin[5] = {0, 0, 0, 0, 0}, qmax[5] = {0, 0, 0, 0, 0};
+  bool nan = false;
   const long long b = gbase_of(g, i);
   const int w = g.width[i >> 6];
-  for (int s = 0; s < w; ++s) {
+  for (int s = sub; s < w; s += LPN) {
     const int j = g.col[b + (long long)s * kW];
     if (j < 0) break;
     double Qj[5];
@@ -292,6 +305,7 @@ __global__ void __launch_bounds__(kBlock) k_gradient(int nnode, int ntot, Gell g
       for (int k = 0; k < 5; ++k) {
         qmax[k] = dmax(qmax[k], Qj[k]);
         qmin[k] = dmin(qmin[k], Qj[k]);
+        nan |= Qj[k] != Qj[k];
       }
     }
     double tj[NT];
@@ -320,6 +334,7 @@ __global__ void __launch_bounds__(kBlock) k_gradient(int nnode, int ntot, Gell g
       }
     }
   }
+  lane_sum<LPN, NT * 3>(gr);
   for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) {
     int h = he_id[p];
     if (bc_type[he_tag[h]] != BC_SYMMETRY) continue;
@@ -332,13 +347,37 @@ __global__ void __launch_bounds__(kBlock) k_gradient(int nnode, int ntot, Gell g
       gr[3 * t + 2] -= dt * a2;
     }
   }
+  // every lane holds the sums: they share the stores
 #pragma unroll
-  for (int k = 0; k < NT * 3; ++k) grad[k * nnode + i] = gr[k];
+  for (int k = 0; k < NT * 3; ++k)
+    if (k % LPN == sub) grad[k * nnode + i] = gr[k];
   if constexpr (LIM) {
     double phi[5];
-    limit_node(i, nnode, ntot, L.type, L.K3, L.chi, g, xyz, L.vol, q, Qi, gr, qmin, qmax, phi);
+    if constexpr (LPN > 1) {
+      if (!lane_any<LPN>(nan)) {
+        lane_max<LPN, 5>(qmax);
+        lane_min<LPN, 5>(qmin);
+      } else {
+        // a NaN state's place among the neighbours decides what the running
+        // bounds keep: take them in order
 #pragma unroll
-    for (int k = 0; k < 5; ++k) L.lim2[k * nnode + i] = phi[k];
+        for (int k = 0; k < 5; ++k) qmin[k] = qmax[k] = 0.0;
+        for (int s = 0; s < w; ++s) {
+          const int j = g.col[b + (long long)s * kW];
+          if (j < 0) break;
+#pragma unroll
+          for (int k = 0; k < 5; ++k) {
+            const double v = q[k * ntot + j];
+            qmax[k] = dmax(qmax[k], v);
+            qmin[k] = dmin(qmin[k], v);
+          }
+        }
+      }
+    }
+    limit_node<LPN>(i, sub, nnode, ntot, L.type, L.K3, L.chi, g, xyz, L.vol, q, Qi, gr, qmin, qmax, phi);
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+      if (k % LPN == sub) L.lim2[k * nnode + i] = phi[k];
   }
 }
 
@@ -425,6 +464,13 @@ __global__ void __launch_bounds__(kBlock) k_gradient_gg(int nnode, int ntot, Gel
   for (int k = 0; k < NT * 3; ++k) grad[k * nnode + i] = gr[k];
 }
 
+template <bool LIM>
+static auto gradient_kernel(int nterms, int lpn) {
+  if (nterms == 9)
+    return lpn == 4 ? k_gradient<9, LIM, 4> : lpn == 2 ? k_gradient<9, LIM, 2> : k_gradient<9, LIM, 1>;
+  return lpn == 4 ? k_gradient<5, LIM, 4> : lpn == 2 ? k_gradient<5, LIM, 2> : k_gradient<5, LIM, 1>;
+}
+
 void launch_gradient(Ctx& c, int nterms) {
   if (c.prm.gradient_type == 1) {
     if (nterms == 9)
@@ -439,8 +485,10 @@ void launch_gradient(Ctx& c, int nterms) {
     return;
   }
   const LimArgs none{0, 0.0, 0.0, nullptr, nullptr};
-  auto kern = nterms == 9 ? k_gradient<9, false> : k_gradient<5, false>;
-  hipLaunchKernelGGL(kern, dim3(nblk(c.nnode)), dim3(kBlock), 0, c.stream, c.nnode, c.ntot, gell(c), c.d.xyz,
+  const int lpn = gradient_lanes(c.nnode);
+  auto kern = gradient_kernel<false>(nterms, lpn);
+  hipLaunchKernelGGL(kern, dim3(nblk((long long)c.nnode * lpn)), dim3(kBlock), 0, c.stream, c.nnode, c.ntot, gell(c),
+                     c.d.xyz,
                      c.d.sw, c.d.q, c.d.he_ptr, c.d.he_id, c.d.he_tag, c.d.he_a, c.nbnode, c.d.bc_type, c.prm.gamma,
                      c.d.grad, none);
   PCFD_HIP(hipGetLastError());
@@ -476,7 +524,7 @@ __global__ void __launch_bounds__(kBlock) k_limiter(int nnode, int ntot, int typ
       qmin[k] = dmin(qmin[k], v);
     }
   }
-  limit_node(i, nnode, ntot, type, K3, chi, g, xyz, vol, q, qi, gi, qmin, qmax, phi);
+  limit_node<1>(i, 0, nnode, ntot, type, K3, chi, g, xyz, vol, q, qi, gi, qmin, qmax, phi);
 #pragma unroll
   for (int k = 0; k < 5; ++k) lim2[k * nnode + i] = phi[k];
 }
@@ -507,13 +555,14 @@ __device__ __forceinline__ bool bad_state_r(const double* Q, double gamma) {
 //  3. k_clip_replay: one thread runs the reference's loop over that list on
 //     the current limiters.  Edges off the list cannot fire, so the result
 //     is the reference's full loop.
+template <int LPN>
 __global__ void __launch_bounds__(kBlock) k_clip_flag(int nnode, int ntot, double chi, double gamma, Gell g,
                                                      const double* __restrict__ xyz, const double* __restrict__ q,
                                                      const double* __restrict__ grad,
                                                      const double* __restrict__ lim2, double* __restrict__ lim,
                                                      unsigned char* __restrict__ flag) {
-  int i = xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= nnode) return;
+  const int i = (xcd_block() * blockDim.x + threadIdx.x) / LPN, sub = threadIdx.x % LPN;
+  if (i >= nnode) return;  // all lanes of a node together
   // The node's own state, gradient and limiter stay in registers; only the
   // neighbour side is gathered.  Both extrapolations are written relative to
   // node i: dQ = qj - qi and dx = (xj - xi)/2 give bit-identical states to
@@ -531,7 +580,7 @@ __global__ void __launch_bounds__(kBlock) k_clip_flag(int nnode, int ntot, doubl
   const double xi[3] = {xyz[i], xyz[nnode + i], xyz[2 * nnode + i]};
   const long long b = gbase_of(g, i);
   const int w = g.width[i >> 6];
-  for (int s = 0; s < w && !fire; ++s) {
+  for (int s = sub; s < w && !fire; s += LPN) {
     const int j = g.col[b + (long long)s * kW];
     if (j < 0) break;
     const double dx[3] = {0.5 * (xyz[j] - xi[0]), 0.5 * (xyz[nnode + j] - xi[1]), 0.5 * (xyz[2 * nnode + j] - xi[2])};
@@ -551,9 +600,11 @@ __global__ void __launch_bounds__(kBlock) k_clip_flag(int nnode, int ntot, doubl
     else roe_state(Qj, Qi, gamma, Qr);
     if (bad_state(Qr, gamma)) fire = true;
   }
-  flag[i] = fire ? 1 : 0;
+  fire = lane_any<LPN>(fire);
+  if (sub == 0) flag[i] = fire ? 1 : 0;
 #pragma unroll
-  for (int k = 0; k < 5; ++k) lim[k * nnode + i] = li[k] < 0.0 ? 0.0 : li[k];
+  for (int k = 0; k < 5; ++k)
+    if (k % LPN == sub) lim[k * nnode + i] = li[k] < 0.0 ? 0.0 : li[k];
 }
 
 // cnt[p] = number of edges p*64 .. p*64+63 with a flagged end
@@ -626,7 +677,9 @@ __global__ void __launch_bounds__(64) k_clip_replay(int nnode, int ntot, int npa
 
 void launch_pressure_clip(Ctx& c) {
   const pcfd_params& p = c.prm;
-  hipLaunchKernelGGL(k_clip_flag, dim3(nblk(c.nnode)), dim3(kBlock), 0, c.stream, c.nnode, c.ntot, p.chi, p.gamma,
+  const int lpn = lanes_per_node(c.nnode);
+  hipLaunchKernelGGL(lpn == 4 ? k_clip_flag<4> : k_clip_flag<2>, dim3(nblk((long long)c.nnode * lpn)), dim3(kBlock),
+                     0, c.stream, c.nnode, c.ntot, p.chi, p.gamma,
                      gell(c), c.d.xyz, c.d.q, c.d.grad, c.d.lim2, c.d.lim, c.d.clip_flag);
   PCFD_HIP(hipGetLastError());
   if (c.nedge == 0) return;
@@ -657,8 +710,10 @@ void launch_limiter(Ctx& c) {
 void launch_gradient_limiter(Ctx& c, int nterms) {
   const pcfd_params& p = c.prm;
   const LimArgs L{p.limiter, p.venkat_K * p.venkat_K * p.venkat_K, p.chi, c.d.vol, c.d.lim2};
-  auto kern = nterms == 9 ? k_gradient<9, true> : k_gradient<5, true>;
-  hipLaunchKernelGGL(kern, dim3(nblk(c.nnode)), dim3(kBlock), 0, c.stream, c.nnode, c.ntot, gell(c), c.d.xyz,
+  const int lpn = gradient_lanes(c.nnode);
+  auto kern = gradient_kernel<true>(nterms, lpn);
+  hipLaunchKernelGGL(kern, dim3(nblk((long long)c.nnode * lpn)), dim3(kBlock), 0, c.stream, c.nnode, c.ntot, gell(c),
+                     c.d.xyz,
                      c.d.sw, c.d.q, c.d.he_ptr, c.d.he_id, c.d.he_tag, c.d.he_a, c.nbnode, c.d.bc_type, p.gamma,
                      c.d.grad, L);
   PCFD_HIP(hipGetLastError());
@@ -670,7 +725,7 @@ void launch_gradient_limiter(Ctx& c, int nterms) {
 // b[L] -= F, b[R] += F) gathered per node, then Bkernel_Inviscid_Flux
 // (:298-387, b[L] -= F on the unextrapolated state vs the phantom).
 // Also writes per-block partial sums of b^2 (total + per equation).
-template <bool HO, bool ALG>
+template <bool HO, bool ALG, int LPN>
 __global__ void __launch_bounds__(kBlock) k_residual(int nnode, int ntot, double gamma, double chi, int sym2d, Gell g,
                                                     const double* __restrict__ xyz, const double* __restrict__ q,
                                                     const double* __restrict__ grad, const double* __restrict__ lim,
@@ -678,7 +733,7 @@ __global__ void __launch_bounds__(kBlock) k_residual(int nnode, int ntot, double
                                                     const double* __restrict__ he_a, int nbnode,
                                                     double* __restrict__ b, double* __restrict__ red) {
   const int blk = xcd_block();
-  int i = blk * blockDim.x + threadIdx.x;
+  const int i = (blk * blockDim.x + threadIdx.x) / LPN, sub = threadIdx.x % LPN;
   double bi[5] = {0, 0, 0, 0, 0};
   if (i < nnode) {
     double qi[5], gi[15], li[5], xi[3];
@@ -693,56 +748,74 @@ __global__ void __launch_bounds__(kBlock) k_residual(int nnode, int ntot, double
     }
     const long long base = gbase_of(g, i);
     const int w = g.width[i >> 6];
-    for (int s = 0; s < w; ++s) {
+    for (int s0 = 0; s0 < w; s0 += LPN) {
+      // the lanes' edges together, then their fluxes added in edge order (a
+      // residual near a steady state is what is left of large terms)
+      const int s = s0 + sub;
       const long long idx = base + (long long)s * kW;
-      const int j = g.col[idx];
-      if (j < 0) break;
-      const bool left = i < j;
-      double a[4] = {g.nrm[idx], g.nrm[g.stride + idx], g.nrm[2 * g.stride + idx], g.nrm[3 * g.stride + idx]};
-      double qj[5];
+      const int j = s < w ? g.col[idx] : -1;
+      if (!lane_any<LPN>(j >= 0)) break;
+      double v[5] = {0, 0, 0, 0, 0};
+      if (j >= 0) {
+        const bool left = i < j;
+        double a[4] = {g.nrm[idx], g.nrm[g.stride + idx], g.nrm[2 * g.stride + idx], g.nrm[3 * g.stride + idx]};
+        double qj[5];
 #pragma unroll
-      for (int k = 0; k < 5; ++k) qj[k] = q[k * ntot + j];
-      double QL[5], QR[5];
-      if (HO) {
-        // both ends extrapolated relative to node i (dQ = qj - qi, dx =
-        // (xj - xi)/2), then assigned to L/R: the same bits as the (L,R)
-        // form because a - b == -(b - a) and 0.5*(-d) == -(0.5*d) in IEEE
-        // arithmetic, with two selects per variable instead of eight
-        const double dx[3] = {0.5 * (xyz[j] - xi[0]), 0.5 * (xyz[nnode + j] - xi[1]),
-                              0.5 * (xyz[2 * nnode + j] - xi[2])};
-        const double mdx[3] = {-dx[0], -dx[1], -dx[2]};
+        for (int k = 0; k < 5; ++k) qj[k] = q[k * ntot + j];
+        double QL[5], QR[5];
+        if (HO) {
+          // both ends extrapolated relative to node i (dQ = qj - qi, dx =
+          // (xj - xi)/2), then assigned to L/R: the same bits as the (L,R)
+          // form because a - b == -(b - a) and 0.5*(-d) == -(0.5*d) in IEEE
+          // arithmetic, with two selects per variable instead of eight
+          const double dx[3] = {0.5 * (xyz[j] - xi[0]), 0.5 * (xyz[nnode + j] - xi[1]),
+                                0.5 * (xyz[2 * nnode + j] - xi[2])};
+          const double mdx[3] = {-dx[0], -dx[1], -dx[2]};
 #pragma unroll
-        for (int k = 0; k < 5; ++k) {
-          const double dQ = qj[k] - qi[k];
-          const double Qi = extrap1(qi[k], dQ, gi[3 * k], gi[3 * k + 1], gi[3 * k + 2], dx, chi, li[k]);
-          const double Qj = extrap1(qj[k], -dQ, grad[(3 * k) * nnode + j], grad[(3 * k + 1) * nnode + j],
-                                    grad[(3 * k + 2) * nnode + j], mdx, chi, lim[k * nnode + j]);
-          QL[k] = left ? Qi : Qj;
-          QR[k] = left ? Qj : Qi;
+          for (int k = 0; k < 5; ++k) {
+            const double dQ = qj[k] - qi[k];
+            const double Qi = extrap1(qi[k], dQ, gi[3 * k], gi[3 * k + 1], gi[3 * k + 2], dx, chi, li[k]);
+            const double Qj = extrap1(qj[k], -dQ, grad[(3 * k) * nnode + j], grad[(3 * k + 1) * nnode + j],
+                                      grad[(3 * k + 2) * nnode + j], mdx, chi, lim[k * nnode + j]);
+            QL[k] = left ? Qi : Qj;
+            QR[k] = left ? Qj : Qi;
+          }
+        } else {
+#pragma unroll
+          for (int k = 0; k < 5; ++k) {
+            QL[k] = left ? qi[k] : qj[k];
+            QR[k] = left ? qj[k] : qi[k];
+          }
         }
-      } else {
+        double F[5];
+        num_flux<ALG>(QL, QR, a, gamma, sym2d, F);
 #pragma unroll
-        for (int k = 0; k < 5; ++k) {
-          QL[k] = left ? qi[k] : qj[k];
-          QR[k] = left ? qj[k] : qi[k];
-        }
+        for (int k = 0; k < 5; ++k) v[k] = left ? -F[k] : F[k];
       }
-      double F[5];
-      num_flux<ALG>(QL, QR, a, gamma, sym2d, F);
-#pragma unroll
-      for (int k = 0; k < 5; ++k) bi[k] += left ? -F[k] : F[k];
+      lane_add<LPN, 5>(bi, v);
     }
-    for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) {
-      int h = he_id[p];
-      double a[4] = {he_a[h], he_a[nbnode + h], he_a[2 * nbnode + h], he_a[3 * nbnode + h]};
-      double QR[5];
+    const int p1 = he_ptr[i + 1];
+    for (int p0 = he_ptr[i]; p0 < p1; p0 += LPN) {
+      const int p = p0 + sub;
+      double v[5] = {0, 0, 0, 0, 0};
+      if (p < p1) {
+        int h = he_id[p];
+        double a[4] = {he_a[h], he_a[nbnode + h], he_a[2 * nbnode + h], he_a[3 * nbnode + h]};
+        double QR[5];
 #pragma unroll
-      for (int k = 0; k < 5; ++k) QR[k] = q[k * ntot + nnode + h];
-      double F[5];
-      num_flux<ALG>(qi, QR, a, gamma, sym2d, F);
+        for (int k = 0; k < 5; ++k) QR[k] = q[k * ntot + nnode + h];
+        double F[5];
+        num_flux<ALG>(qi, QR, a, gamma, sym2d, F);
 #pragma unroll
-      for (int k = 0; k < 5; ++k) bi[k] += -F[k];
+        for (int k = 0; k < 5; ++k) v[k] = -F[k];
+      }
+      lane_add<LPN, 5>(bi, v);
     }
+  }
+  if (sub != 0) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) bi[k] = 0.0;
+  } else if (i < nnode) {
 #pragma unroll
     for (int k = 0; k < 5; ++k) b[k * nnode + i] = bi[k];
   }
@@ -767,13 +840,19 @@ __global__ void __launch_bounds__(kBlock) k_reduce6(int nparts, const double* __
   }
 }
 
+template <int LPN>
+static auto residual_kernel(int ho, bool alg) {
+  return ho ? (alg ? k_residual<true, true, LPN> : k_residual<true, false, LPN>)
+            : (alg ? k_residual<false, true, LPN> : k_residual<false, false, LPN>);
+}
+
 void launch_residual(Ctx& c, int ho) {
   const pcfd_params& p = c.prm;
-  int nb = nblk(c.nnode);
   sub_begin(c);
   const bool alg = p.flux_type == PCFD_FLUX_ALGEBRAIC;
-  auto kern = ho ? (alg ? k_residual<true, true> : k_residual<true, false>)
-                 : (alg ? k_residual<false, true> : k_residual<false, false>);
+  const int lpn = lanes_per_node(c.nnode);
+  const int nb = nblk((long long)c.nnode * lpn);
+  auto kern = lpn == 4 ? residual_kernel<4>(ho, alg) : residual_kernel<2>(ho, alg);
   hipLaunchKernelGGL(kern, dim3(nb), dim3(kBlock), 0, c.stream, c.nnode, c.ntot, p.gamma, p.chi, p.symmetry2d,
                      gell(c), c.d.xyz, c.d.q, c.d.grad, c.d.lim, c.d.he_ptr, c.d.he_id, c.d.he_a, c.nbnode, c.d.b,
                      c.d.red);
@@ -811,21 +890,22 @@ __device__ __forceinline__ double max_eig_r(const double* Q, const double* a, do
 // ComputeTimesteps, local time stepping (ucs/timestep.tcc:6-47).  With
 // vol23 set, the von Neumann limit dt = min(dt, VNN vol^(2/3)) is applied
 // from node 1 on, as the reference's loop does (:37-45).
+template <int LPN>
 __global__ void __launch_bounds__(kBlock) k_timestep(int nnode, int ntot, double gamma, double cfl, Gell g,
                                                     const double* __restrict__ q, const double* __restrict__ vol,
                                                     const int* __restrict__ he_ptr, const int* __restrict__ he_id,
                                                     const double* __restrict__ he_a, int nbnode,
                                                     const double* __restrict__ vol23, double vnn,
                                                     double* __restrict__ dt) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nnode) return;
+  const int i = (blockIdx.x * blockDim.x + threadIdx.x) / LPN, sub = threadIdx.x % LPN;
+  if (i >= nnode) return;  // all lanes of a node together
   double qi[5];
 #pragma unroll
   for (int k = 0; k < 5; ++k) qi[k] = q[k * ntot + i];
   double s = 0.0;
   const long long base = gbase_of(g, i);
   const int w = g.width[i >> 6];
-  for (int p = 0; p < w; ++p) {
+  for (int p = sub; p < w; p += LPN) {
     const long long idx = base + (long long)p * kW;
     const int j = g.col[idx];
     if (j < 0) break;
@@ -835,7 +915,7 @@ __global__ void __launch_bounds__(kBlock) k_timestep(int nnode, int ntot, double
     for (int k = 0; k < 5; ++k) t[k] = 0.5 * (qi[k] + q[k * ntot + j]);
     s += max_eig_r(t, a, gamma) * a[3];
   }
-  for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) {
+  for (int p = he_ptr[i] + sub; p < he_ptr[i + 1]; p += LPN) {
     int h = he_id[p];
     double a[4] = {he_a[h], he_a[nbnode + h], he_a[2 * nbnode + h], he_a[3 * nbnode + h]};
     double t[5];
@@ -843,6 +923,8 @@ __global__ void __launch_bounds__(kBlock) k_timestep(int nnode, int ntot, double
     for (int k = 0; k < 5; ++k) t[k] = 0.5 * (qi[k] + q[k * ntot + nnode + h]);
     s += max_eig_r(t, a, gamma) * a[3];
   }
+  lane_sum<LPN, 1>(&s);
+  if (sub != 0) return;
   double d = cfl * (vol[i] / s);
   if (vol23 && i > 0) d = dmin(d, vnn * vol23[i]);
   dt[i] = d;
@@ -892,7 +974,9 @@ void launch_timestep(Ctx& c, double cfl) {
     PCFD_HIP(hipGetLastError());
     return;
   }
-  hipLaunchKernelGGL(k_timestep, dim3(nblk(c.nnode)), dim3(kBlock), 0, c.stream, c.nnode, c.ntot, p.gamma, cfl,
+  const int lpn = lanes_per_node(c.nnode);
+  hipLaunchKernelGGL(lpn == 4 ? k_timestep<4> : k_timestep<2>, dim3(nblk((long long)c.nnode * lpn)), dim3(kBlock), 0,
+                     c.stream, c.nnode, c.ntot, p.gamma, cfl,
                      gell(c), c.d.q, c.d.vol, c.d.he_ptr, c.d.he_id, c.d.he_a, c.nbnode,
                      p.enable_vnn ? c.d.vol23 : nullptr, p.vnn, c.d.dt);
   PCFD_HIP(hipGetLastError());
