@@ -20,78 +20,129 @@ struct ChemDev {
   double nup[PCFD_CHEM_MAXR][PCFD_CHEM_MAXS], nupp[PCFD_CHEM_MAXR][PCFD_CHEM_MAXS],
       eff[PCFD_CHEM_MAXR][PCFD_CHEM_MAXS];
   double ref_density, ref_time, ref_temperature;
+  // per reaction, formed once from the above: net coefficient of every species
+  // (its first local occurrence's) and their sum over the local list
+  double net[PCFD_CHEM_MAXR][PCFD_CHEM_MAXS], nu[PCFD_CHEM_MAXR];
 };
 
 // isWholeNumber (ucs/macros.h:24-30); integer exponents go through pow of
-// the promoted integer like the reference's pow(Type, Int)
+// the promoted integer like the reference's pow(Type, Int).  The small whole
+// exponents that mass action is made of are products: 1 and x are pow's
+// results, x*x is rounded once, the cube's second rounding is corrected.  (A
+// pow is some 200 instructions; with them source and Jacobian of 400k
+// five-species cells took 1.58 ms, with products, rate constants shared by the
+// columns and whole-line stores 0.24 ms.)
 __device__ __forceinline__ double powr(double x, double e) {
   const int up = (int)(e + 0.5), flat = (int)e;
-  return pow(x, up == flat ? (double)flat : e);
+  if (up == flat) e = (double)flat;
+  if (e == 0.0) return 1.0;
+  if (e == 1.0) return x;
+  if (e == 2.0) return x * x;
+  if (e == -1.0) return 1.0 / x;
+  if (e == 3.0) {
+    const double x2 = x * x, r = x2 * x;
+    const double c = __builtin_fma(x2, x, __builtin_fma(x, x, -x2) * x);
+    return __builtin_isinf(x2) || __builtin_isnan(c) ? r : c;
+  }
+  return pow(x, e);
 }
 
 __device__ __forceinline__ double kf_of(const ChemDev& m, int r, double T) {
   const double A = m.A[r], EA = m.EA[r], n = m.n[r];
+  // pow(T, n) in the reference: whole and half exponents up to 3/2 as products
+  // and quotients of T and sqrt(T), at most three roundings
+  double Tn;
+  if (n == 0.0) Tn = 1.0;
+  else if (n == 1.0) Tn = T;
+  else if (n == -1.0) Tn = 1.0 / T;
+  else if (fabs(n) == 0.5 || fabs(n) == 1.5) {
+    Tn = sqrt(T);
+    if (fabs(n) == 1.5) Tn *= T;
+    if (n < 0.0) Tn = 1.0 / Tn;
+  } else Tn = pow(T, n);
   switch (m.type[r]) {
     case 0: return (A * exp(-EA / (kUnivR * T)));
-    case 1: return (A * pow(T, n) * exp(-EA / (kUnivR * T)));
-    case 2: return (A * pow(T, n) * exp(-EA / T));
-    case 3: return (A * pow(T, n));
+    case 1: return (A * Tn * exp(-EA / (kUnivR * T)));
+    case 2: return (A * Tn * exp(-EA / T));
+    case 3: return (A * Tn);
   }
   return -999.0;
 }
 
-// GetEquilibriumReactionRate (ucs/reaction.tcc:628-679)
-__device__ __forceinline__ double kc_of(const ChemDev& m, int r, double T) {
-  double nu = 0.0, d[7] = {0, 0, 0, 0, 0, 0, 0};
+// GetEquilibriumReactionRate (ucs/reaction.tcc:628-679); lnT = log(T)
+__device__ __forceinline__ double kc_of(const ChemDev& m, int r, double T, double lnT) {
+  double d[7] = {0, 0, 0, 0, 0, 0, 0};
   const bool high = T > 1000.0;  // GetThermoCoeff: pinned ranges pick the same set
   for (int i = 0; i < m.nloc[r]; ++i) {
     const int s = m.loc[r][i];
     const double* a = high ? m.hi[s] : m.lo[s];
     const double dnu = m.nupp[r][i] - m.nup[r][i];
-    nu += dnu;
 #pragma unroll
     for (int k = 0; k < 7; ++k) d[k] += dnu * a[k];
   }
   const double Kp =
-      exp(d[0] * (log(T) - 1.0) + T * (d[1] / 2.0 + T * (d[2] / 6.0 + T * (d[3] / 12.0 + d[4] / 20.0 * T))) -
+      exp(d[0] * (lnT - 1.0) + T * (d[1] / 2.0 + T * (d[2] / 6.0 + T * (d[3] / 12.0 + d[4] / 20.0 * T))) -
           d[5] / T + d[6]);
   double Kc = Kp;
-  if (!(fabs(nu) < 1.0e-15)) Kc *= powr(101325.0 / (kUnivR * T), nu);
+  if (!(fabs(m.nu[r]) < 1.0e-15)) Kc *= powr(101325.0 / (kUnivR * T), m.nu[r]);
   return Kc;
 }
 
+// The functions below take the species count as a template argument (0: the
+// model's at run time): with it known the per-species arrays stay in
+// registers, where an indexed array would live in scratch memory.
+template <int NS>
+__device__ __forceinline__ int nspecies_of(const ChemDev& m) {
+  return NS > 0 ? NS : m.ns;
+}
+
+// v[k] for a k that is the same in every lane
+template <int NS>
+__device__ __forceinline__ double pick(const double* v, int k) {
+  if constexpr (NS == 0) return v[k];
+  double x = v[0];
+#pragma unroll
+  for (int i = 1; i < NS; ++i) x = k == i ? v[i] : x;
+  return x;
+}
+
 // GetMassProductionRates for one state: rhoi (kg/m^3), T (K) -> wdot (kg/m^3/s)
+template <int NS>
 __device__ inline void wdot_of(const ChemDev& m, const double* rhoi, double T, double* wdot) {
-  double X[PCFD_CHEM_MAXS];
-  for (int k = 0; k < m.ns; ++k) {
+  constexpr int MS = NS > 0 ? NS : PCFD_CHEM_MAXS;
+  const int ns = nspecies_of<NS>(m);
+  double X[MS];
+#pragma unroll
+  for (int k = 0; k < MS; ++k) {
+    if (k >= ns) break;
     X[k] = rhoi[k] / m.mw[k];
     wdot[k] = 0.0;
   }
+  const double lnT = log(T);
   for (int r = 0; r < m.nr; ++r) {
     const double Kf = kf_of(m, r, T);
-    const double Kb = Kf / kc_of(m, r, T);
+    const double Kb = Kf / kc_of(m, r, T, lnT);
     double pf = 1.0, pd = 1.0;
     for (int k = 0; k < m.nloc[r]; ++k) {
-      const double x = X[m.loc[r][k]];
+      const double x = pick<NS>(X, m.loc[r][k]);
       pf *= powr(x, m.nup[r][k]);
       pd *= powr(x, m.nupp[r][k]);
     }
     double Mc = 1.0;
     if (m.tb[r]) {
       Mc = 0.0;
-      for (int k = 0; k < m.ns; ++k) Mc += X[k];
-      for (int k = 0; k < m.nloc[r]; ++k) Mc += (m.eff[r][k] - 1.0) * X[m.loc[r][k]];
+#pragma unroll
+      for (int k = 0; k < MS; ++k) {
+        if (k >= ns) break;
+        Mc += X[k];
+      }
+      for (int k = 0; k < m.nloc[r]; ++k) Mc += (m.eff[r][k] - 1.0) * pick<NS>(X, m.loc[r][k]);
     }
     const double net = Kf * pf - Kb * pd;
-    // species order; the first local occurrence of a species carries its nu
-    for (int i = 0; i < m.ns; ++i) {
-      int kk = -1;
-      for (int k = 0; k < m.nloc[r]; ++k)
-        if (m.loc[r][k] == i) {
-          kk = k;
-          break;
-        }
-      const double nu = kk >= 0 ? m.nupp[r][kk] - m.nup[r][kk] : 0.0;
+#pragma unroll
+    for (int i = 0; i < MS; ++i) {
+      if (i >= ns) break;
+      const double nu = m.net[r][i];
       if (nu == 0.0) continue;  // AlmostEqualRelative(nu, 0, 1e-15): contributes +0
       double w = nu * Mc * net;
       w *= m.mw[i];
@@ -101,12 +152,21 @@ __device__ inline void wdot_of(const ChemDev& m, const double* rhoi, double T, d
 }
 
 // SourceTerm (ucs/compressibleFR.tcc:1276-1312) on the FR state
+template <int NS>
 __device__ inline void source_of(const ChemDev& m, const double* Q, double vol, double* src) {
-  double rhoi[PCFD_CHEM_MAXS], w[PCFD_CHEM_MAXS];
-  const double T = Q[m.ns + 3] * m.ref_temperature;
-  for (int i = 0; i < m.ns; ++i) rhoi[i] = Q[i] * m.ref_density;
-  wdot_of(m, rhoi, T, w);
-  for (int i = 0; i < m.ns; ++i) {
+  constexpr int MS = NS > 0 ? NS : PCFD_CHEM_MAXS;
+  const int ns = nspecies_of<NS>(m);
+  double rhoi[MS], w[MS];
+  const double T = Q[ns + 3] * m.ref_temperature;
+#pragma unroll
+  for (int i = 0; i < MS; ++i) {
+    if (i >= ns) break;
+    rhoi[i] = Q[i] * m.ref_density;
+  }
+  wdot_of<NS>(m, rhoi, T, w);
+#pragma unroll
+  for (int i = 0; i < MS; ++i) {
+    if (i >= ns) break;
     w[i] /= (m.ref_density / m.ref_time);
     src[i] = vol * w[i];
   }
@@ -119,62 +179,69 @@ __device__ inline void source_of(const ChemDev& m, const double* Q, double vol, 
 // reaction and shared; every copy's products and sums, in their order, are
 // wdot_of's, so w[(1 + c) * ns + i] equals wdot_of of copy c bit for bit
 // and w[i] that of the state.  w [(ns + 1) * ns].
+template <int NS>
 __device__ inline void wdot_rho_columns(const ChemDev& m, const double* rhoi, const double* rhop, double T,
                                         double* w) {
-  const int ns = m.ns;
-  double X[PCFD_CHEM_MAXS], Xp[PCFD_CHEM_MAXS];
-  for (int k = 0; k < ns; ++k) {
+  constexpr int MS = NS > 0 ? NS : PCFD_CHEM_MAXS;
+  const int ns = nspecies_of<NS>(m);
+  double X[MS], Xp[MS];
+#pragma unroll
+  for (int k = 0; k < MS; ++k) {
+    if (k >= ns) break;
     X[k] = rhoi[k] / m.mw[k];
     Xp[k] = rhop[k] / m.mw[k];
   }
-  for (int k = 0; k < (ns + 1) * ns; ++k) w[k] = 0.0;
+#pragma unroll
+  for (int k = 0; k < (MS + 1) * MS; ++k) {
+    if (k >= (ns + 1) * ns) break;
+    w[k] = 0.0;
+  }
+  const double lnT = log(T);
   for (int r = 0; r < m.nr; ++r) {
     const double Kf = kf_of(m, r, T);
-    const double Kb = Kf / kc_of(m, r, T);
-    const int nl = m.nloc[r];
-    double ff[PCFD_CHEM_MAXS], fd[PCFD_CHEM_MAXS], nu[PCFD_CHEM_MAXS];
-    for (int k = 0; k < nl; ++k) {
-      const double x = X[m.loc[r][k]];
-      ff[k] = powr(x, m.nup[r][k]);
-      fd[k] = powr(x, m.nupp[r][k]);
-    }
-    for (int i = 0; i < ns; ++i) {
-      int kk = -1;
-      for (int k = 0; k < nl; ++k)
-        if (m.loc[r][k] == i) {
-          kk = k;
-          break;
-        }
-      nu[i] = kk >= 0 ? m.nupp[r][kk] - m.nup[r][kk] : 0.0;
-    }
-    for (int s = 0; s <= ns; ++s) {
-      const int c = s - 1;  // -1: the state itself
-      double pf = 1.0, pd = 1.0;
-      for (int k = 0; k < nl; ++k) {
-        if (m.loc[r][k] == c) {
-          pf *= powr(Xp[c], m.nup[r][k]);
-          pd *= powr(Xp[c], m.nupp[r][k]);
-        } else {
-          pf *= ff[k];
-          pd *= fd[k];
-        }
-      }
-      double Mc = 1.0;
+    const double Kb = Kf / kc_of(m, r, T, lnT);
+    // copy s has species s - 1 raised (0: the state itself)
+    double pf[MS + 1], pd[MS + 1], Mc[MS + 1];
+#pragma unroll
+    for (int s = 0; s <= MS; ++s) {
+      if (s > ns) break;
+      pf[s] = pd[s] = Mc[s] = 1.0;
       if (m.tb[r]) {
-        Mc = 0.0;
-        for (int k = 0; k < ns; ++k) Mc += k == c ? Xp[k] : X[k];
-        for (int k = 0; k < nl; ++k) {
-          const int l = m.loc[r][k];
-          Mc += (m.eff[r][k] - 1.0) * (l == c ? Xp[l] : X[l]);
+        Mc[s] = 0.0;
+#pragma unroll
+        for (int k = 0; k < MS; ++k) {
+          if (k >= ns) break;
+          Mc[s] += k == s - 1 ? Xp[k] : X[k];
         }
       }
-      const double net = Kf * pf - Kb * pd;
-      double* ws = w + s * ns;
-      for (int i = 0; i < ns; ++i) {
-        if (nu[i] == 0.0) continue;
-        double v = nu[i] * Mc * net;
+    }
+    for (int k = 0; k < m.nloc[r]; ++k) {
+      const int l = m.loc[r][k];
+      const double x = pick<NS>(X, l), xp = pick<NS>(Xp, l);
+      const double eu = m.nup[r][k], ed = m.nupp[r][k];
+      const double fu = powr(x, eu), fup = powr(xp, eu), fd = powr(x, ed), fdp = powr(xp, ed);
+      const double w1 = m.eff[r][k] - 1.0;
+#pragma unroll
+      for (int s = 0; s <= MS; ++s) {
+        if (s > ns) break;
+        const bool raised = l == s - 1;
+        pf[s] *= raised ? fup : fu;
+        pd[s] *= raised ? fdp : fd;
+        if (m.tb[r]) Mc[s] += w1 * (raised ? xp : x);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < MS; ++i) {
+      if (i >= ns) break;
+      const double nu = m.net[r][i];
+      if (nu == 0.0) continue;
+#pragma unroll
+      for (int s = 0; s <= MS; ++s) {
+        if (s > ns) break;
+        const double net = Kf * pf[s] - Kb * pd[s];
+        double v = nu * Mc[s] * net;
         v *= m.mw[i];
-        ws[i] += v;
+        w[s * ns + i] += v;
       }
     }
   }
@@ -184,21 +251,26 @@ __device__ inline void wdot_rho_columns(const ChemDev& m, const double* rhoi, co
 // (the species columns of the forward-difference source Jacobian):
 // src[i] is the state's, src[(1 + c) * ns + i] copy c's, each bit for bit
 // what source_of gives.  src [(ns + 1) * ns].
+template <int NS>
 __device__ inline void source_rho_columns(const ChemDev& m, const double* Q, double h, double vol, double* src) {
-  const int ns = m.ns;
-  double rhoi[PCFD_CHEM_MAXS], rhop[PCFD_CHEM_MAXS];
+  constexpr int MS = NS > 0 ? NS : PCFD_CHEM_MAXS;
+  const int ns = nspecies_of<NS>(m);
+  double rhoi[MS], rhop[MS];
   const double T = Q[ns + 3] * m.ref_temperature;
-  for (int i = 0; i < ns; ++i) {
+#pragma unroll
+  for (int i = 0; i < MS; ++i) {
+    if (i >= ns) break;
     rhoi[i] = Q[i] * m.ref_density;
     rhop[i] = (Q[i] + h) * m.ref_density;
   }
-  wdot_rho_columns(m, rhoi, rhop, T, src);
-  for (int k = 0; k < (ns + 1) * ns; ++k) {
+  wdot_rho_columns<NS>(m, rhoi, rhop, T, src);
+#pragma unroll
+  for (int k = 0; k < (MS + 1) * MS; ++k) {
+    if (k >= (ns + 1) * ns) break;
     double v = src[k];
     v /= (m.ref_density / m.ref_time);
     src[k] = vol * v;
   }
 }
-
 
 }  // namespace pcfd

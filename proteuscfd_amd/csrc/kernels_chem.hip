@@ -21,47 +21,96 @@
 
 namespace pcfd {
 
+template <int NS>
 __global__ void __launch_bounds__(kChemBlock) k_wdot(const ChemDev* __restrict__ md, int n,
                                                     const double* __restrict__ rhoi, const double* __restrict__ T,
                                                     double* __restrict__ wdot) {
+  constexpr int MS = NS > 0 ? NS : PCFD_CHEM_MAXS;
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= n) return;
   const ChemDev& m = *md;
-  double r[PCFD_CHEM_MAXS], w[PCFD_CHEM_MAXS];
-  for (int k = 0; k < m.ns; ++k) r[k] = rhoi[(long long)c * m.ns + k];
-  wdot_of(m, r, T[c], w);
-  for (int k = 0; k < m.ns; ++k) wdot[(long long)c * m.ns + k] = w[k];
+  const int ns = nspecies_of<NS>(m);
+  double r[MS], w[MS];
+#pragma unroll
+  for (int k = 0; k < MS; ++k) {
+    if (k >= ns) break;
+    r[k] = rhoi[(long long)c * ns + k];
+  }
+  wdot_of<NS>(m, r, T[c], w);
+#pragma unroll
+  for (int k = 0; k < MS; ++k) {
+    if (k >= ns) break;
+    wdot[(long long)c * ns + k] = w[k];
+  }
 }
 
 // SourceTerm + SourceTermJacobian (ucs/eqnset.tcc:162-187): one-sided
 // differences with h = 1e-8 on every FR variable.  The velocity columns are
 // exactly zero (the source does not read u, v, w: (S - S)/h = 0) and the
-// momentum and energy rows are zero, so only the species and T columns
-// are evaluated.
-__global__ void __launch_bounds__(kChemBlock) k_source(const ChemDev* __restrict__ md, int n,
-                                                      const double* __restrict__ q, const double* __restrict__ vol,
-                                                      double* __restrict__ src, double* __restrict__ jac) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n) return;
+// momentum and energy rows are zero, so only the species columns (which share
+// the state's rate constants) and the T column are evaluated.  A cell's 81
+// entries are contiguous in the output, so a wavefront leaves what is not zero
+// of its 64 cells in LDS and writes their blocks together, 64 consecutive
+// doubles a store.
+constexpr int kSrcBlock = 64;
+
+template <int NS>
+__global__ void __launch_bounds__(kSrcBlock) k_source(const ChemDev* __restrict__ md, int n,
+                                                     const double* __restrict__ q, const double* __restrict__ vol,
+                                                     double* __restrict__ src, double* __restrict__ jac) {
+  constexpr int MS = NS > 0 ? NS : PCFD_CHEM_MAXS;
+  // per cell: the source, then its columns rho_1 .. rho_ns, T; cell fastest
+  __shared__ double sh[MS * (MS + 2)][kSrcBlock];
   const ChemDev& m = *md;
-  const int ns = m.ns, neqn = ns + 4;
-  double Q[PCFD_CHEM_MAXS + 4], s[PCFD_CHEM_MAXS], sp[PCFD_CHEM_MAXS];
-  for (int k = 0; k < neqn; ++k) Q[k] = q[(long long)c * neqn + k];
-  const double v = vol[c];
-  source_of(m, Q, v, s);
-  double* so = src + (long long)c * neqn;
-  for (int k = 0; k < neqn; ++k) so[k] = k < ns ? s[k] : 0.0;
+  const int ns = nspecies_of<NS>(m), neqn = ns + 4;
+  const int c0 = blockIdx.x * kSrcBlock, t = threadIdx.x, c = c0 + t;
+  if (c < n) {
+    double Q[MS + 4], sc[(MS + 1) * MS], sp[MS];
+#pragma unroll
+    for (int k = 0; k < MS + 4; ++k) {
+      if (k >= neqn) break;
+      Q[k] = q[(long long)c * neqn + k];
+    }
+    const double v = vol[c], h = 1.0e-8;
+    if (jac) {
+      source_rho_columns<NS>(m, Q, h, v, sc);
+      // the T column
+#pragma unroll
+      for (int k = 0; k < MS + 4; ++k)
+        if (k == ns + 3) Q[k] += h;
+      source_of<NS>(m, Q, v, sp);
+#pragma unroll
+      for (int j = 0; j < MS; ++j) {
+        if (j >= ns) break;
+        sh[j][t] = sc[j];
+#pragma unroll
+        for (int i = 0; i < MS; ++i) {
+          if (i >= ns) break;
+          sh[(1 + i) * ns + j][t] = (sc[(1 + i) * ns + j] - sc[j]) / h;
+        }
+        sh[(1 + ns) * ns + j][t] = (sp[j] - sc[j]) / h;
+      }
+    } else {
+      source_of<NS>(m, Q, v, sp);
+#pragma unroll
+      for (int j = 0; j < MS; ++j) {
+        if (j >= ns) break;
+        sh[j][t] = sp[j];
+      }
+    }
+  }
+  __syncthreads();
+  const int cells = n - c0 < kSrcBlock ? n - c0 : kSrcBlock;
+  for (int e = t; e < cells * neqn; e += kSrcBlock) {
+    const int k = e % neqn;
+    src[(long long)c0 * neqn + e] = k < ns ? sh[k][e / neqn] : 0.0;
+  }
   if (!jac) return;
-  double* J = jac + (long long)c * neqn * neqn;
-  for (int k = 0; k < neqn * neqn; ++k) J[k] = 0.0;
-  const double h = 1.0e-8;
-  for (int i = 0; i < neqn; ++i) {
-    if (i >= ns && i < ns + 3) continue;
-    const double keep = Q[i];
-    Q[i] += h;
-    source_of(m, Q, v, sp);
-    Q[i] = keep;
-    for (int j = 0; j < ns; ++j) J[j * neqn + i] = (sp[j] - s[j]) / h;
+  const int ne2 = neqn * neqn;
+  for (int e = t; e < cells * ne2; e += kSrcBlock) {
+    const int cell = e / ne2, k = e % ne2, j = k / neqn, i = k % neqn;
+    const bool zero = j >= ns || (i >= ns && i < ns + 3);
+    jac[(long long)c0 * ne2 + e] = zero ? 0.0 : sh[(1 + (i < ns ? i : ns)) * ns + j][cell];
   }
 }
 
@@ -113,8 +162,8 @@ struct DevBuf {
 int launch_source(pcfd_chem& c, int n, const double* q, const double* vol, double* src, double* jac) {
   if (n == 0) return PCFD_OK;
   check(hipEventRecord(c.e0, c.stream), "hipEventRecord");
-  hipLaunchKernelGGL(k_source, dim3((n + kChemBlock - 1) / kChemBlock), dim3(kChemBlock), 0, c.stream, c.dev, n, q,
-                     vol, src, jac);
+  hipLaunchKernelGGL(c.host.ns == 5 ? k_source<5> : k_source<0>, dim3((n + kSrcBlock - 1) / kSrcBlock),
+                     dim3(kSrcBlock), 0, c.stream, c.dev, n, q, vol, src, jac);
   check(hipGetLastError(), "k_source");
   check(hipEventRecord(c.e1, c.stream), "hipEventRecord");
   check(hipEventSynchronize(c.e1), "hipEventSynchronize");
@@ -181,6 +230,16 @@ int pcfd_chem_create(const pcfd_chem_desc* d, pcfd_chem** out) {
       m.nup[r][k] = d->nup[PCFD_CHEM_MAXS * r + k];
       m.nupp[r][k] = d->nupp[PCFD_CHEM_MAXS * r + k];
       m.eff[r][k] = d->tb_eff[PCFD_CHEM_MAXS * r + k];
+    }
+  }
+  for (int r = 0; r < m.nr; ++r) {
+    for (int k = 0; k < m.nloc[r]; ++k) {
+      const int g = m.loc[r][k];
+      const double dnu = m.nupp[r][k] - m.nup[r][k];
+      m.nu[r] += dnu;
+      bool seen = false;
+      for (int j = 0; j < k; ++j) seen |= m.loc[r][j] == g;
+      if (!seen) m.net[r][g] = dnu;
     }
   }
   m.ref_density = d->ref_density;
@@ -363,7 +422,8 @@ int pcfd_chem_wdot(pcfd_chem* c, int n, const double* rhoi, const double* T, dou
     check(hipMemcpyAsync(dr.p, rhoi, sizeof(double) * (size_t)n * ns, hipMemcpyHostToDevice, cc.stream), "copy");
     check(hipMemcpyAsync(dt.p, T, sizeof(double) * (size_t)n, hipMemcpyHostToDevice, cc.stream), "copy");
     check(hipEventRecord(cc.e0, cc.stream), "hipEventRecord");
-    hipLaunchKernelGGL(k_wdot, dim3((n + kChemBlock - 1) / kChemBlock), dim3(kChemBlock), 0, cc.stream, cc.dev, n,
+    hipLaunchKernelGGL(cc.host.ns == 5 ? k_wdot<5> : k_wdot<0>, dim3((n + kChemBlock - 1) / kChemBlock),
+                       dim3(kChemBlock), 0, cc.stream, cc.dev, n,
                        dr.as<double>(), dt.as<double>(), dw.as<double>());
     check(hipGetLastError(), "k_wdot");
     check(hipEventRecord(cc.e1, cc.stream), "hipEventRecord");
@@ -382,7 +442,8 @@ int pcfd_chem_wdot_device(pcfd_chem* c, int n, const double* rhoi, const double*
     }
     if (n == 0) return PCFD_OK;
     check(hipEventRecord(cc.e0, cc.stream), "hipEventRecord");
-    hipLaunchKernelGGL(k_wdot, dim3((n + kChemBlock - 1) / kChemBlock), dim3(kChemBlock), 0, cc.stream, cc.dev, n,
+    hipLaunchKernelGGL(cc.host.ns == 5 ? k_wdot<5> : k_wdot<0>, dim3((n + kChemBlock - 1) / kChemBlock),
+                       dim3(kChemBlock), 0, cc.stream, cc.dev, n,
                        rhoi, T, wdot);
     check(hipGetLastError(), "k_wdot");
     check(hipEventRecord(cc.e1, cc.stream), "hipEventRecord");

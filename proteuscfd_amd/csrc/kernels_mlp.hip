@@ -921,10 +921,13 @@ __global__ void __launch_bounds__(kChemBlock) k_wdot_list(const ChemDev* __restr
   }
   const int c = lst[(long long)lo * 64 + (t - off[lo])];
   const ChemDev& m = *md;
-  double r[PCFD_CHEM_MAXS], w[PCFD_CHEM_MAXS];
-  for (int k = 0; k < m.ns; ++k) r[k] = rhoi[(long long)c * m.ns + k];
-  wdot_of(m, r, T[c], w);
-  for (int k = 0; k < m.ns; ++k) wdot[(long long)c * m.ns + k] = w[k];
+  // the surrogate is built for five species
+  double r[kNout], w[kNout];
+#pragma unroll
+  for (int k = 0; k < kNout; ++k) r[k] = rhoi[(long long)c * kNout + k];
+  wdot_of<kNout>(m, r, T[c], w);
+#pragma unroll
+  for (int k = 0; k < kNout; ++k) wdot[(long long)c * kNout + k] = w[k];
 }
 
 const ChemDev* chem_device_model(const pcfd_chem* c);
