@@ -54,6 +54,7 @@ namespace {
 
 constexpr int kFB = 128;  // threads per block for the FR kernels
 constexpr int kLane = 64;
+constexpr double kFrH = 1.0e-8;  // step of the differenced Jacobians
 
 thread_local std::string g_fr_create_err;
 
@@ -349,7 +350,31 @@ __global__ void __launch_bounds__(kFB) k_fr_timestep(const Model* __restrict__ m
 // ---- Jacobian --------------------------------------------------------------
 // Kernel_NumJac (ucs/jacobian.tcc:253-304): one-sided differences (h = 1e-8)
 // of the edge's HLLC flux in each native variable of either side, aux
-// recomputed for every perturbed state.  Block (n0,n1) = dF/dq_n1, block
+// recomputed for every perturbed state.  A flux takes pressure, density, sound
+// speed and total energy of its two sides; a node's are the same on all its
+// edges, so k_fr_jac_states forms them once per node, for the state itself
+// (entry 0) and with variable c raised by h (entry 1 + c): the same arithmetic
+// on the same values.  Formed in every flux they were two thirds of its
+// divisions: 1.38 ms for 1.24M edges in FP32 storage against 0.58 + 0.04 ms.
+template <int NS>
+__global__ void __launch_bounds__(kFB) k_fr_jac_states(const Model* __restrict__ mp, int nnode,
+                                                      const double* __restrict__ q, fr::Side* __restrict__ st) {
+  constexpr int NE = NS + 4;
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (long long)nnode * (NE + 1)) return;
+  const Model& m = *mp;
+  const int c = (int)(t % (NE + 1)) - 1;
+  State<NS> S;
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const double v = q[t / (NE + 1) * NE + k];
+    S.q[k] = k == c ? v + kFrH : v;
+  }
+  fr::aux(m, S);
+  st[t] = fr::side_of<NS>(m, S);
+}
+
+// Block (n0,n1) = dF/dq_n1, block
 // (n1,n0) = -dF/dq_n0; their negations, the two diagonal contributions of
 // Kernel_Diag_NumJac (:436-456; the n0 row's diagonal gets minus block
 // (n1,n0)), are written to ediag, contiguously per edge side, and
@@ -362,7 +387,8 @@ __global__ void __launch_bounds__(kFB) k_fr_timestep(const Model* __restrict__ m
 template <int NS, typename TM>
 __global__ void __launch_bounds__(kFB) k_fr_jac_edge(const Model* __restrict__ mp, int nedge,
                                                     const int* __restrict__ edges, const double* __restrict__ ea,
-                                                    const double* __restrict__ q, double beta,
+                                                    const double* __restrict__ q,
+                                                    const fr::Side* __restrict__ st, double beta,
                                                     const double* __restrict__ fs,
                                                     TM* __restrict__ ediag) {
   constexpr int NE = NS + 4;
@@ -370,46 +396,41 @@ __global__ void __launch_bounds__(kFB) k_fr_jac_edge(const Model* __restrict__ m
   if (t >= (long long)nedge * NE) return;
   const int e = (int)(t / NE), i = (int)(t % NE);
   const Model& m = *mp;
-  State<NS> L, R;
-  load_state<NS>(q, edges[2 * e], L, m);
-  load_state<NS>(q, edges[2 * e + 1], R, m);
-  double a[4];
+  const long long nL = edges[2 * e], nR = edges[2 * e + 1];
+  double qL[NE], qR[NE], a[4];
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    qL[k] = q[nL * NE + k];
+    qR[k] = q[nR * NE + k];
+  }
+  const fr::Side sL = st[nL * (NE + 1)], sR = st[nR * (NE + 1)];
 #pragma unroll
   for (int k = 0; k < 4; ++k) a[k] = ea[4LL * e + k];
   // the unperturbed flux, evaluated once per edge by k_fr_edge_flux
-  double fS[NE], fX[NE];
+  double fS[NE], fX[NE], qP[NE];
 #pragma unroll
   for (int k = 0; k < NE; ++k) fS[k] = fs[(long long)e * NE + k];
-  const double h = 1.0e-8;
   // in the storage precision: the FP32 form's diagonal sums FP32 terms
   TM* dL = ediag + (long long)e * 2 * NE * NE;
   TM* dR = dL + NE * NE;
-  {
-    State<NS> P = L;
-    // P.q[i] += h without a dynamic register index
+  // variable i raised, without a dynamic register index
 #pragma unroll
-    for (int k = 0; k < NE; ++k) P.q[k] = (k == i) ? P.q[k] + h : P.q[k];
-    fr::aux(m, P);
-    fr::hllc<NS>(m, P, R, a, beta, fX);
+  for (int k = 0; k < NE; ++k) qP[k] = k == i ? qL[k] + kFrH : qL[k];
+  fr::hllc_sides<NS>(m, qP, st[nL * (NE + 1) + 1 + i], qR, sR, a, beta, fX);
 #pragma unroll
-    for (int j = 0; j < NE; ++j) {
-      // added to a zeroed block, as the reference's scatter does; the
-      // off-diagonal block A[R][L] is -dL (written by k_fr_jac_diag)
-      const double tl = 0.0 + (fS[j] - fX[j]) / h;
-      dL[j * NE + i] = (TM)(-tl);
-    }
+  for (int j = 0; j < NE; ++j) {
+    // added to a zeroed block, as the reference's scatter does; the
+    // off-diagonal block A[R][L] is -dL (written by k_fr_jac_diag)
+    const double tl = 0.0 + (fS[j] - fX[j]) / kFrH;
+    dL[j * NE + i] = (TM)(-tl);
   }
-  {
-    State<NS> P = R;
 #pragma unroll
-    for (int k = 0; k < NE; ++k) P.q[k] = (k == i) ? P.q[k] + h : P.q[k];
-    fr::aux(m, P);
-    fr::hllc<NS>(m, L, P, a, beta, fX);
+  for (int k = 0; k < NE; ++k) qP[k] = k == i ? qR[k] + kFrH : qR[k];
+  fr::hllc_sides<NS>(m, qL, sL, qP, st[nR * (NE + 1) + 1 + i], a, beta, fX);
 #pragma unroll
-    for (int j = 0; j < NE; ++j) {
-      const double tr = 0.0 + (fX[j] - fS[j]) / h;
-      dR[j * NE + i] = (TM)(-tr);  // A[L][R] = -dR
-    }
+  for (int j = 0; j < NE; ++j) {
+    const double tr = 0.0 + (fX[j] - fS[j]) / kFrH;
+    dR[j * NE + i] = (TM)(-tr);  // A[L][R] = -dR
   }
 }
 
@@ -513,18 +534,21 @@ __global__ void __launch_bounds__(kFB) k_fr_jac_bnd_sum(int nbnd, const int* __r
 // block, ucs/jacobian.tcc:213-250) and the source Jacobian's species rows
 // (EqnSet::SourceTermJacobian, ucs/eqnset.tcc:162-187: forward differences,
 // h = 1e-8; the velocity columns are exactly zero, the source not reading
-// u, v, w).  nterm[i] = [temporal NE*NE | source NS x (NS+1), columns
+// u, v, w).  nterm, rows in the matrix's order, 64 a chunk, entry k of a row at
+// (chunk * NT + k) * 64 + lane: [temporal NE*NE | source NS x (NS+1), columns
 // rho_1..rho_NS, T].
 template <int NS>
 __global__ void __launch_bounds__(kFB) k_fr_node_terms(const Model* __restrict__ mp, const ChemDev* __restrict__ cm,
-                                                      int nnode, const double* __restrict__ q,
+                                                      int nrow_pad, const int* __restrict__ srow,
+                                                      const double* __restrict__ q,
                                                       const double* __restrict__ vol, const double* __restrict__ dt,
                                                       int rxn, double beta, double* __restrict__ nterm) {
   constexpr int NE = NS + 4, NE2 = NE * NE, NT = NE2 + NS * (NS + 1);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nnode) return;
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = r < nrow_pad ? srow[r] : -1;
+  if (i < 0) return;
   const Model& m = *mp;
-  double* o = nterm + (long long)i * NT;
+  double* o = nterm + (long long)(r / kLane) * NT * kLane + r % kLane;
   State<NS> S;
   load_state<NS>(q, i, S, m);
   const double v = vol[i];
@@ -533,12 +557,12 @@ __global__ void __launch_bounds__(kFB) k_fr_node_terms(const Model* __restrict__
   for (int k = 0; k < NE2; ++k) T[k] = 0.0;
   fr::temporal<NS>(m, S, v, dt[i], beta, T);
 #pragma unroll
-  for (int k = 0; k < NE2; ++k) o[k] = T[k];
+  for (int k = 0; k < NE2; ++k) o[(long long)k * kLane] = T[k];
   if (!rxn) return;
   double sc[(NS + 1) * NS], s1[NS], Q[NE];
 #pragma unroll
   for (int k = 0; k < NE; ++k) Q[k] = S.q[k];
-  const double h = 1.0e-8;
+  const double h = kFrH;
   // the state and its species columns (Q[c] + h) share the T-only rate
   // constants: the same values as NS + 1 separate source evaluations
   source_rho_columns<NS>(*cm, Q, h, v, sc);
@@ -546,12 +570,12 @@ __global__ void __launch_bounds__(kFB) k_fr_node_terms(const Model* __restrict__
 #pragma unroll
   for (int c = 0; c < NS; ++c)
 #pragma unroll
-    for (int j = 0; j < NS; ++j) o[NE2 + j * (NS + 1) + c] = (sc[(1 + c) * NS + j] - s0[j]) / h;
+    for (int j = 0; j < NS; ++j) o[(long long)(NE2 + j * (NS + 1) + c) * kLane] = (sc[(1 + c) * NS + j] - s0[j]) / h;
   // the T column
   Q[NS + 3] += h;
   source_of<NS>(*cm, Q, v, s1);
 #pragma unroll
-  for (int j = 0; j < NS; ++j) o[NE2 + j * (NS + 1) + NS] = (s1[j] - s0[j]) / h;
+  for (int j = 0; j < NS; ++j) o[(long long)(NE2 + j * (NS + 1) + NS) * kLane] = (s1[j] - s0[j]) / h;
 }
 
 // whether ContributeTemporalTerms adds to entry (r, c) of the diagonal block
@@ -569,57 +593,96 @@ __device__ __forceinline__ bool temporal_entry(int r, int c) {
 // (:213-250); and the row's off-diagonal blocks from the other sides of
 // its edges.  A workgroup takes one 64-row SELL chunk; wave w builds block
 // row w of those 64 rows (so every store is 64 consecutive rows' entry).
+//
+// The edge sides' blocks lie whole, 81 entries, at 64 unrelated places.  The
+// workgroup reads a slot's 2 x 64 of them together, consecutive lanes
+// consecutive entries, into LDS and takes its rows from there (a row's stride of
+// 81 entries is odd: no bank conflicts), while the next slot's are on their way
+// to registers.  With every lane reading its own 9 entries a load touched 64
+// lines: 1.04 ms for 185k nodes of 13.5 edges in FP32 storage against 0.82,
+// 79 against 44 us for 5.9k nodes in FP64.
 template <int NS, typename TM>
-__global__ void __launch_bounds__(64 * (NS + 4)) k_fr_jac_diag(int nrow_pad, const int* __restrict__ srow,
-                                                             const int* __restrict__ nptr,
-                                                             const int* __restrict__ nslot,
+__global__ void __launch_bounds__(64 * (NS + 4)) k_fr_jac_diag(const int* __restrict__ srow,
+                                                             const int* __restrict__ swidth,
+                                                             const int* __restrict__ sbase,
+                                                             const int* __restrict__ sedge,
                                                              const TM* __restrict__ ediag,
                                                              const int* __restrict__ bidx,
                                                              const double* __restrict__ jdb,
                                                              const double* __restrict__ nterm, int rxn,
-                                                             const int* __restrict__ sbase, TM* __restrict__ M,
-                                                             TM* __restrict__ D) {
+                                                             TM* __restrict__ M, TM* __restrict__ D) {
   constexpr int NE = NS + 4, NE2 = NE * NE, NT = NE2 + NS * (NS + 1);
+  __shared__ TM own[64 * NE2], oth[64 * NE2];
+  __shared__ int side[2][64];
   const int lane = threadIdx.x & 63, rr = threadIdx.x >> 6;
-  const int r = blockIdx.x * 64 + lane;
-  if (r >= nrow_pad) return;
-  const int i = srow[r];
-  TM* Dr = D + (long long)(r >> 6) * NE2 * kLane + (r & 63);
+  const int chunk = blockIdx.x;
+  const int i = srow[chunk * 64 + lane];
+  const int w = swidth[chunk];
+  const int* se = sedge + (long long)sbase[chunk] * kLane;
+  TM* mo = M + (long long)sbase[chunk] * NE2 * kLane + (long long)(rr * NE) * kLane + lane;
+  TM* Dr = D + (long long)chunk * NE2 * kLane + lane;
+  double A[NE];
+  const int bi = i >= 0 ? bidx[i] : -1;
+#pragma unroll
+  for (int c = 0; c < NE; ++c) A[c] = bi >= 0 ? jdb[(long long)bi * NE2 + rr * NE + c] : 0.0;
+  if (rr == 0) {
+    side[0][lane] = w > 0 ? se[lane] : -1;
+    side[1][lane] = w > 1 ? se[kLane + lane] : -1;
+  }
+  __syncthreads();
+  TM vo[NE], vt[NE];
+  // this thread's entries of the slot whose sides are in side[b]
+  auto fetch = [&](int b) {
+#pragma unroll
+    for (int k = 0; k < NE; ++k) {
+      const int t = k * 64 * NE + (int)threadIdx.x, row = t / NE2;
+      const int sd = side[b][row];
+      const long long at = t - row * NE2;
+      vo[k] = sd >= 0 ? ediag[(long long)sd * NE2 + at] : (TM)0;
+      vt[k] = sd >= 0 ? ediag[(long long)(sd ^ 1) * NE2 + at] : (TM)0;
+    }
+  };
+  if (w > 0) fetch(0);
+  for (int s = 0; s < w; ++s) {
+    const int sd = side[s & 1][lane];
+#pragma unroll
+    for (int k = 0; k < NE; ++k) {
+      own[k * 64 * NE + threadIdx.x] = vo[k];
+      oth[k * 64 * NE + threadIdx.x] = vt[k];
+    }
+    const int next = rr == 0 && s + 2 < w ? se[(s + 2) * kLane + lane] : -1;
+    __syncthreads();
+    if (rr == 0) side[s & 1][lane] = next;  // every wave has its sd of this slot
+    if (s + 1 < w) fetch((s + 1) & 1);
+    if (sd >= 0) {
+      // the row's own side of the edge adds to the diagonal, the other side,
+      // negated, is the row's off-diagonal block (A[L][R] = -dR, A[R][L] = -dL)
+      const TM* e = own + lane * NE2 + rr * NE;
+      const TM* o = oth + lane * NE2 + rr * NE;
+      TM* mb = mo + (long long)s * NE2 * kLane;
+#pragma unroll
+      for (int c = 0; c < NE; ++c) {
+        A[c] += (double)e[c];
+        mb[(long long)c * kLane] = -o[c];
+      }
+    }
+    __syncthreads();
+  }
   if (i < 0) {
     // padding rows: identity, so the factorisation of the chunk stays finite
 #pragma unroll
     for (int c = 0; c < NE; ++c) Dr[(long long)(rr * NE + c) * kLane] = (TM)(c == rr ? 1.0 : 0.0);
     return;
   }
-  double A[NE];
-  const int bi = bidx[i];
-#pragma unroll
-  for (int c = 0; c < NE; ++c) A[c] = bi >= 0 ? jdb[(long long)bi * NE2 + rr * NE + c] : 0.0;
-  // slot s of the row is its CSR slot nptr[i] + s: the row's own side of
-  // the edge adds to the diagonal, the other side, negated, is the row's
-  // off-diagonal block (A[L][R] = -dR, A[R][L] = -dL), written here with
-  // contiguous lanes
-  TM* mo = M + (long long)sbase[r >> 6] * NE2 * kLane + (long long)(rr * NE) * kLane + (r & 63);
-  for (int p = nptr[i]; p < nptr[i + 1]; ++p) {
-    const int sd = nslot[p];
-    const TM* e = ediag + (long long)sd * NE2 + rr * NE;
-    const TM* o = ediag + (long long)(sd ^ 1) * NE2 + rr * NE;
-    TM* mb = mo + (long long)(p - nptr[i]) * NE2 * kLane;
-#pragma unroll
-    for (int c = 0; c < NE; ++c) {
-      A[c] += (double)e[c];
-      mb[(long long)c * kLane] = -o[c];
-    }
-  }
-  const double* nt = nterm + (long long)i * NT;
+  const double* nt = nterm + (long long)chunk * NT * kLane + lane;
   if (rxn && rr < NS) {
 #pragma unroll
-    for (int c = 0; c < NS; ++c) A[c] -= nt[NE2 + rr * (NS + 1) + c];
-    A[NS + 3] -= nt[NE2 + rr * (NS + 1) + NS];
+    for (int c = 0; c < NS; ++c) A[c] -= nt[(long long)(NE2 + rr * (NS + 1) + c) * kLane];
+    A[NS + 3] -= nt[(long long)(NE2 + rr * (NS + 1) + NS) * kLane];
   }
 #pragma unroll
   for (int c = 0; c < NE; ++c)
-    if (temporal_entry<NS>(rr, c)) A[c] += nt[rr * NE + c];
+    if (temporal_entry<NS>(rr, c)) A[c] += nt[(long long)(rr * NE + c) * kLane];
 #pragma unroll
   for (int c = 0; c < NE; ++c) Dr[(long long)(rr * NE + c) * kLane] = (TM)A[c];
 }
@@ -785,11 +848,12 @@ __global__ void __launch_bounds__(kFB) k_fr_full_aux(const Model* __restrict__ m
   o[0] = s.P;
   o[1] = s.rho;
   const double TDim = s.q[NS + 3] * m.ref_temperature;
+  fr::with_coeffs(m, TDim, [&](fr::CoeffTable t) {
 #pragma unroll
-  for (int k = 0; k < NS; ++k) {
-    o[2 + k] = (fr::cp_species(m, k, TDim) - m.R[k]) / m.s_ref;
-    o[2 + NS + k] = s.q[k] / m.mw[k] / 1000.0;
-  }
+    for (int k = 0; k < NS; ++k) o[2 + k] = (fr::cp_species(m, t, k, TDim) - m.R[k]) / m.s_ref;
+  });
+#pragma unroll
+  for (int k = 0; k < NS; ++k) o[2 + NS + k] = s.q[k] / m.mw[k] / 1000.0;
 }
 
 }  // namespace
@@ -822,9 +886,10 @@ struct pcfd_fr {
          *elam = nullptr, *b = nullptr, *dt = nullptr, *jdb = nullptr, *bhe = nullptr, *bcol = nullptr, *red = nullptr, *aux = nullptr;
   int *edges = nullptr, *nptr = nullptr, *nslot_d = nullptr, *he_ptr = nullptr, *he_id = nullptr, *he_tag = nullptr, *he_node = nullptr,
       *bc_type = nullptr, *bnd = nullptr, *bidx = nullptr, *srow = nullptr, *swidth = nullptr, *sbase = nullptr,
-      *scol = nullptr, *icount = nullptr;
+      *scol = nullptr, *sedge = nullptr, *icount = nullptr;
   long long* piv = nullptr;
-  double *ediag = nullptr, *nterm = nullptr;  // Jacobian diagonal parts: per edge side, per node
+  double *ediag = nullptr, *nterm = nullptr;  // Jacobian diagonal parts: per edge side, per row
+  fr::Side* jst = nullptr;                    // and the nodes' plain and raised states' properties
   double *Md = nullptr, *Dd = nullptr, *xd = nullptr;
   float *Mf = nullptr, *Df = nullptr, *xf = nullptr;
   // production-rate surrogate in the residual (null: exact rates)
@@ -864,7 +929,7 @@ void free_all(pcfd_fr& f) {
   dfree(f.bidx); dfree(f.srow); dfree(f.swidth); dfree(f.sbase); dfree(f.scol); dfree(f.icount);
   dfree(f.piv); dfree(f.Md); dfree(f.Dd); dfree(f.xd); dfree(f.Mf); dfree(f.Df); dfree(f.xf); dfree(f.dmodel);
   dfree(f.s_rhoi); dfree(f.s_T); dfree(f.s_w); dfree(f.s_lst); dfree(f.s_cnt); dfree(f.s_off);
-  dfree(f.ediag); dfree(f.nterm);
+  dfree(f.ediag); dfree(f.nterm); dfree(f.jst); dfree(f.sedge);
   if (f.e0) (void)hipEventDestroy(f.e0);
   if (f.e1) (void)hipEventDestroy(f.e1);
   if (f.e2) (void)hipEventDestroy(f.e2);
@@ -1000,8 +1065,11 @@ void run_jacobian_t(pcfd_fr& f, TM* M, TM* D) {
     hipLaunchKernelGGL(k_fr_edge_flux<NS5>, dim3(nblocks(f.nedge)), dim3(kFB), 0, f.stream, f.dmodel, f.nedge,
                        f.edges, f.edge_a, f.q, f.prm.beta, f.eflux);
     hcheck(hipGetLastError(), "k_fr_edge_flux");
+    hipLaunchKernelGGL(k_fr_jac_states<NS5>, dim3(nblocks((long long)f.nnode * (NS5 + 5))), dim3(kFB), 0, f.stream,
+                       f.dmodel, f.nnode, f.q, f.jst);
+    hcheck(hipGetLastError(), "k_fr_jac_states");
     hipLaunchKernelGGL((k_fr_jac_edge<NS5, TM>), dim3(nblocks((long long)f.nedge * (NS5 + 4))), dim3(kFB), 0,
-                       f.stream, f.dmodel, f.nedge, f.edges, f.edge_a, f.q, f.prm.beta, f.eflux,
+                       f.stream, f.dmodel, f.nedge, f.edges, f.edge_a, f.q, f.jst, f.prm.beta, f.eflux,
                        reinterpret_cast<TM*>(f.ediag));
     hcheck(hipGetLastError(), "k_fr_jac_edge");
     send(f, 6);
@@ -1020,13 +1088,13 @@ void run_jacobian_t(pcfd_fr& f, TM* M, TM* D) {
                        f.stream, f.nbnd, f.bnd, f.he_ptr, f.bcol, f.jdb);
     hcheck(hipGetLastError(), "k_fr_jac_bnd_sum");
   }
-  hipLaunchKernelGGL(k_fr_node_terms<NS5>, dim3(nblocks(f.nnode)), dim3(kFB), 0, f.stream, f.dmodel,
-                     chem_device_model(f.chem), f.nnode, f.q, f.vol, f.dt, f.prm.reactions, f.prm.beta, f.nterm);
+  hipLaunchKernelGGL(k_fr_node_terms<NS5>, dim3(nblocks(f.nrow_pad)), dim3(kFB), 0, f.stream, f.dmodel,
+                     chem_device_model(f.chem), f.nrow_pad, f.srow, f.q, f.vol, f.dt, f.prm.reactions, f.prm.beta,
+                     f.nterm);
   hcheck(hipGetLastError(), "k_fr_node_terms");
   hipLaunchKernelGGL((k_fr_jac_diag<NS5, TM>), dim3(f.nrow_pad / kLane), dim3(kLane * (NS5 + 4)), 0, f.stream,
-                     f.nrow_pad, f.srow, f.nptr, f.nslot_d, reinterpret_cast<const TM*>(f.ediag), f.bidx, f.jdb,
-                     f.nterm, f.prm.reactions,
-                     f.sbase, M, D);
+                     f.srow, f.swidth, f.sbase, f.sedge, reinterpret_cast<const TM*>(f.ediag), f.bidx, f.jdb, f.nterm,
+                     f.prm.reactions, M, D);
   hcheck(hipGetLastError(), "k_fr_jac_diag");
   f.lu_done = false;
 }
@@ -1302,13 +1370,14 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
       slots += w;
     }
     f->nslot = slots;
-    std::vector<int> scol((size_t)slots * kLane, -1);
+    std::vector<int> scol((size_t)slots * kLane, -1), sedge((size_t)slots * kLane, -1);
     std::vector<long long> eoff(2 * (size_t)ne);
     for (int i = 0; i < nn; ++i) {
       const int r = spos[i], k = r / kLane, l = r % kLane;
       for (int p = nptr[i]; p < nptr[i + 1]; ++p) {
         const long long s = (long long)sbase[k] + (p - nptr[i]);
         scol[(size_t)s * kLane + l] = nbr[p];
+        sedge[(size_t)s * kLane + l] = nslot[p];
         // row i's block for this neighbour: edge e's (n0,n1) block when i is n0
         eoff[2 * (size_t)(nslot[p] >> 1) + (nslot[p] & 1)] = s * NE2 * kLane + l;
       }
@@ -1363,6 +1432,7 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
     dput(*f, &f->swidth, swidth);
     dput(*f, &f->sbase, sbase);
     dput(*f, &f->scol, scol);
+    dput(*f, &f->sedge, sedge);
     dalloc(*f, &f->q, (size_t)f->ntot * NE);
     dalloc(*f, &f->eflux, (size_t)ne * NE);
     dalloc(*f, &f->elam, (size_t)ne);
@@ -1375,7 +1445,8 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
     dalloc(*f, &f->icount, 4);
     dalloc(*f, &f->piv, (size_t)f->nrow_pad);
     dalloc(*f, &f->ediag, 2 * (size_t)ne * NE2);
-    dalloc(*f, &f->nterm, (size_t)nn * (NE2 + ns * (ns + 1)));
+    dalloc(*f, &f->nterm, (size_t)f->nrow_pad * (NE2 + ns * (ns + 1)));
+    dalloc(*f, &f->jst, (size_t)nn * (NE + 1));
     hcheck(hipMemset(f->q, 0, sizeof(double) * (size_t)f->ntot * NE), "hipMemset");
   } catch (const std::exception& e) {
     g_fr_create_err = e.what();

@@ -15,6 +15,7 @@
 #pragma once
 
 #include <cmath>
+#include <cstddef>
 
 #ifdef __HIPCC__
 #include <hip/hip_runtime.h>
@@ -42,7 +43,7 @@ struct Model {
   double mw[kMaxS];      // kg/mol
   double R[kMaxS];       // UNIV_R / MW (Species::R, ucs/species.tcc:315)
   double lo[kMaxS][7];   // NASA-7, T <= 1000 K
-  double hi[kMaxS][7];   // NASA-7, T > 1000 K
+  double hi[kMaxS][7];   // NASA-7, T > 1000 K; follows lo
   double ref_density, ref_temperature, ref_pressure, ref_velocity;
   double vref2;          // ref_velocity^2 (ref_specific_enthalpy)
   double s_ref;          // ref_velocity^2 / ref_temperature
@@ -53,6 +54,8 @@ struct Model {
   int no_cvbc;           // noCVBC: upwind farfield, mirrored walls
 };
 
+static_assert(offsetof(Model, hi) == offsetof(Model, lo) + sizeof(Model::lo), "with_coeffs steps from lo to hi");
+
 template <int NS>
 struct State {
   static constexpr int NE = NS + 4;
@@ -60,27 +63,45 @@ struct State {
   double P, rho;  // aux
 };
 
-// Species::GetThermoCoeff (ucs/species.tcc:98-137): outside 200-6000 K the
-// pinned set is the one the range test would pick anyway
-PCFD_HD const double* coeffs(const Model& m, int s, double T) { return T > 1000.0 ? m.hi[s] : m.lo[s]; }
+// f(coefficients [species][7]) for the range T lies in.  Species::GetThermoCoeff
+// (ucs/species.tcc:98-137): outside 200-6000 K the pinned set is the one the
+// range test would pick anyway.  On the device the two tables are taken in turn,
+// each for the lanes it is for (a wavefront with none skips it): the table's
+// address is then the same in every lane and its loads are scalar.  (A pointer
+// per lane costs a mixture's properties 25 vector loads.)
+typedef const double (*CoeffTable)[7];
+template <typename F>
+PCFD_HD void with_coeffs(const Model& m, double T, F&& f) {
+  const int high = T > 1000.0 ? 1 : 0;
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll 1
+  for (int range = 0; range < 2; ++range) {
+    int k = range * (int)(sizeof(m.lo) / sizeof(m.lo[0]));
+    asm volatile("" : "+s"(k));  // or the compiler would put the lane's own flag in its place
+    if (high == range) f(m.lo + k);
+  }
+#else
+  f(high ? m.hi : m.lo);
+#endif
+}
 
 // Species::GetCp (ucs/species.tcc:43-53), J/(kg K)
-PCFD_HD double cp_species(const Model& m, int s, double T) {
-  const double* a = coeffs(m, s, T);
+PCFD_HD double cp_species(const Model& m, CoeffTable t, int s, double T) {
+  const double* a = t[s];
   const double cp_R = a[0] + T * (a[1] + T * (a[2] + T * (a[3] + T * a[4])));
   return cp_R * m.R[s];
 }
 
 // Species::GetH (ucs/species.tcc:56-70, href = 0), J/kg
-PCFD_HD double h_species(const Model& m, int s, double T) {
-  const double* a = coeffs(m, s, T);
+PCFD_HD double h_species(const Model& m, CoeffTable t, int s, double T) {
+  const double* a = t[s];
   const double h_R = a[5] + T * (a[0] + T * (a[1] / 2.0 + T * (a[2] / 3.0 + T * (a[3] / 4.0 + T * a[4] / 5.0))));
   return h_R * m.R[s];
 }
 
 // Species::GetdHdT (ucs/species.tcc:337-348)
-PCFD_HD double dhdt_species(const Model& m, int s, double T) {
-  const double* a = coeffs(m, s, T);
+PCFD_HD double dhdt_species(const Model& m, CoeffTable t, int s, double T) {
+  const double* a = t[s];
   const double r = a[0] + T * (a[1] + T * (a[2] + T * (a[3] + T * a[4])));
   return r * m.R[s];
 }
@@ -114,8 +135,10 @@ PCFD_HD void props(const Model& m, const double* rhoi, double T, double& cv, dou
   for (int i = 0; i < NS; ++i) Rd += rd[i] * m.R[i];
   Rd /= rho;
   double cpd = 0.0, cvd = 0.0, cpi[NS];
+  with_coeffs(m, Td, [&](CoeffTable t) {
 #pragma unroll
-  for (int i = 0; i < NS; ++i) cpi[i] = cp_species(m, i, Td);
+    for (int i = 0; i < NS; ++i) cpi[i] = cp_species(m, t, i, Td);
+  });
 #pragma unroll
   for (int i = 0; i < NS; ++i) cpd += cpi[i] * (rd[i] / rho);
 #pragma unroll
@@ -134,8 +157,10 @@ template <int NS>
 PCFD_HD double hmix(const Model& m, const State<NS>& s) {
   const double Td = s.q[NS + 3] * m.ref_temperature;
   double h = 0.0;
+  with_coeffs(m, Td, [&](CoeffTable t) {
 #pragma unroll
-  for (int i = 0; i < NS; ++i) h += h_species(m, i, Td) * (s.q[i] / s.rho);
+    for (int i = 0; i < NS; ++i) h += h_species(m, t, i, Td) * (s.q[i] / s.rho);
+  });
   return h / m.vref2;
 }
 
@@ -147,38 +172,53 @@ PCFD_HD double total_enthalpy(const Model& m, const State<NS>& s) {
 
 // GetTheta (ucs/compressibleFR.tcc:1640-1643), vdotn = 0
 template <int NS>
+PCFD_HD double theta_q(const double* q, const double* a) {
+  return q[NS] * a[0] + q[NS + 1] * a[1] + q[NS + 2] * a[2] + 0.0;
+}
+template <int NS>
 PCFD_HD double theta_of(const State<NS>& s, const double* a) {
-  return s.q[NS] * a[0] + s.q[NS + 1] * a[1] + s.q[NS + 2] * a[2] + 0.0;
+  return theta_q<NS>(s.q, a);
+}
+
+// What HLLCFlux takes from one side besides its native state: pressure, total
+// density, sound speed squared and total energy
+struct Side {
+  double P, rho, c2, ET;
+};
+
+template <int NS>
+PCFD_HD Side side_of(const Model& m, const State<NS>& s) {
+  Side d;
+  double cv, cp, R, g;
+  d.P = s.P;
+  d.rho = s.rho;
+  props<NS>(m, s.q, s.q[NS + 3], cv, cp, R, g, d.c2);
+  d.ET = total_enthalpy(m, s) - s.P;
+  return d;
 }
 
 // HLLCFlux (ucs/compressibleFR.tcc:300-548) with vdotn = 0, NaN components
 // zeroed as NumericalFlux does (ucs/eqnset.tcc:74-88).  Returns true when a
-// component was zeroed.
+// component was zeroed.  qL, qR: the native states of the two sides.
 template <int NS>
-PCFD_HD bool hllc(const Model& m, const State<NS>& L, const State<NS>& Rs, const double* a, double beta,
-                  double* flux) {
+PCFD_HD bool hllc_sides(const Model& m, const double* qL, const Side& dL, const double* qR, const Side& dR,
+                        const double* a, double beta, double* flux) {
   constexpr int NE = NS + 4;
-  double cvL, cpL, RL, gL, c2L, cvR, cpR, RR, gR, c2R;
-  const double uL = L.q[NS], vL = L.q[NS + 1], wL = L.q[NS + 2], TL = L.q[NS + 3], pL = L.P, rhoL = L.rho;
-  const double pgL = pL - m.Pref;
-  props<NS>(m, L.q, TL, cvL, cpL, RL, gL, c2L);
-  const double HTL = total_enthalpy(m, L), ETL = HTL - pL;
-  const double thetaL = theta_of(L, a);
-  const double uR = Rs.q[NS], vR = Rs.q[NS + 1], wR = Rs.q[NS + 2], TR = Rs.q[NS + 3], pR = Rs.P, rhoR = Rs.rho;
-  const double pgR = pR - m.Pref;
-  props<NS>(m, Rs.q, TR, cvR, cpR, RR, gR, c2R);
-  const double HTR = total_enthalpy(m, Rs), ETR = HTR - pR;
-  const double thetaR = theta_of(Rs, a);
+  const double uL = qL[NS], vL = qL[NS + 1], wL = qL[NS + 2], TL = qL[NS + 3], pL = dL.P, rhoL = dL.rho;
+  const double pgL = pL - m.Pref, c2L = dL.c2, ETL = dL.ET;
+  const double thetaL = theta_q<NS>(qL, a);
+  const double uR = qR[NS], vR = qR[NS + 1], wR = qR[NS + 2], TR = qR[NS + 3], pR = dR.P, rhoR = dR.rho;
+  const double pgR = pR - m.Pref, c2R = dR.c2, ETR = dR.ET;
+  const double thetaR = theta_q<NS>(qR, a);
   const double rho = sqrt(rhoL * rhoR);
   const double sigma = rho / (rhoL + rho);
   State<NS> roe;
 #pragma unroll
-  for (int i = 0; i < NS; ++i) roe.q[i] = L.q[i] + sigma * (Rs.q[i] - L.q[i]);
+  for (int i = 0; i < NS; ++i) roe.q[i] = qL[i] + sigma * (qR[i] - qL[i]);
   roe.q[NS] = uL + sigma * (uR - uL);
   roe.q[NS + 1] = vL + sigma * (vR - vL);
   roe.q[NS + 2] = wL + sigma * (wR - wL);
   roe.q[NS + 3] = TL + sigma * (TR - TL);
-  aux(m, roe);
   const double theta = theta_of(roe, a);
   double cv, cp, R, gt, c2;
   props<NS>(m, roe.q, roe.q[NS + 3], cv, cp, R, gt, c2);
@@ -202,7 +242,7 @@ PCFD_HD bool hllc(const Model& m, const State<NS>& L, const State<NS>& Rs, const
   bool died = false;
   if (SL >= 0.0) {
 #pragma unroll
-    for (int i = 0; i < NS; ++i) Qf[i] = L.q[i];
+    for (int i = 0; i < NS; ++i) Qf[i] = qL[i];
     Qf[NS] = rhoL * uL;
     Qf[NS + 1] = rhoL * vL;
     Qf[NS + 2] = rhoL * wL;
@@ -211,7 +251,7 @@ PCFD_HD bool hllc(const Model& m, const State<NS>& L, const State<NS>& Rs, const
     SM = thetaL;
   } else if (SR <= 0.0) {
 #pragma unroll
-    for (int i = 0; i < NS; ++i) Qf[i] = Rs.q[i];
+    for (int i = 0; i < NS; ++i) Qf[i] = qR[i];
     Qf[NS] = rhoR * uR;
     Qf[NS + 1] = rhoR * vR;
     Qf[NS + 2] = rhoR * wR;
@@ -222,7 +262,7 @@ PCFD_HD bool hllc(const Model& m, const State<NS>& L, const State<NS>& Rs, const
     pStar = pgL + rhoL * (thetaL - SL) * (thetaL - SM);
     const double omega = 1.0 / (SL - SM), const1 = SL - thetaL, const2 = pStar - pgL;
 #pragma unroll
-    for (int i = 0; i < NS; ++i) Qf[i] = omega * const1 * L.q[i];
+    for (int i = 0; i < NS; ++i) Qf[i] = omega * const1 * qL[i];
     Qf[NS] = omega * (const1 * rhoL * uL + const2 * a[0]);
     Qf[NS + 1] = omega * (const1 * rhoL * vL + const2 * a[1]);
     Qf[NS + 2] = omega * (const1 * rhoL * wL + const2 * a[2]);
@@ -231,7 +271,7 @@ PCFD_HD bool hllc(const Model& m, const State<NS>& L, const State<NS>& Rs, const
     pStar = pgR + rhoR * (thetaR - SR) * (thetaR - SM);
     const double omega = 1.0 / (SR - SM), const1 = SR - thetaR, const2 = pStar - pgR;
 #pragma unroll
-    for (int i = 0; i < NS; ++i) Qf[i] = omega * const1 * Rs.q[i];
+    for (int i = 0; i < NS; ++i) Qf[i] = omega * const1 * qR[i];
     Qf[NS] = omega * (const1 * rhoR * uR + const2 * a[0]);
     Qf[NS + 1] = omega * (const1 * rhoR * vR + const2 * a[1]);
     Qf[NS + 2] = omega * (const1 * rhoR * wR + const2 * a[2]);
@@ -266,6 +306,12 @@ PCFD_HD bool hllc(const Model& m, const State<NS>& L, const State<NS>& Rs, const
       z = true;
     }
   return z;
+}
+
+template <int NS>
+PCFD_HD bool hllc(const Model& m, const State<NS>& L, const State<NS>& Rs, const double* a, double beta,
+                  double* flux) {
+  return hllc_sides<NS>(m, L.q, side_of<NS>(m, L), Rs.q, side_of<NS>(m, Rs), a, beta, flux);
 }
 
 // MaxEigenvalue (ucs/compressibleFR.tcc:1602-1637)
@@ -661,7 +707,14 @@ PCFD_HD void temporal(const Model& m, const State<NS>& s, double vol, double dta
   props<NS>(m, s.q, T, cv, cp, R, gamma, c2);
   const double rhoDim = rho * m.ref_density, TDim = T * m.ref_temperature;
   v2 *= m.ref_velocity * m.ref_velocity;
-  double rd[NS], Yi[NS], dEtdRhoi[NS];
+  double rd[NS], Yi[NS], dEtdRhoi[NS], hs[NS], dhdt[NS];
+  with_coeffs(m, TDim, [&](CoeffTable t) {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      hs[i] = h_species(m, t, i, TDim);
+      dhdt[i] = dhdt_species(m, t, i, TDim);
+    }
+  });
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
     rd[i] = s.q[i] * m.ref_density;
@@ -689,12 +742,12 @@ PCFD_HD void temporal(const Model& m, const State<NS>& s, double vol, double dta
         if (j == i) continue;
         d -= m.R[j] * rd[j] / (rhomix * rhomix);
       }
-      dEtdRhoi[i] = hv2 + h_species(m, i, TDim) - (dPdrhomix + dPdRmix * d);
+      dEtdRhoi[i] = hv2 + hs[i] - (dPdrhomix + dPdRmix * d);
     }
     dEtdP = 0.0;
     const double dTdP = 1.0 / (rhomix * Rmix);
 #pragma unroll
-    for (int i = 0; i < NS; ++i) dEtdP += rd[i] * (dhdt_species(m, i, TDim)) * dTdP;
+    for (int i = 0; i < NS; ++i) dEtdP += rd[i] * dhdt[i] * dTdP;
     dEtdP -= 1.0;
   }
   const double ref_detdrho = m.vref2 * m.ref_density / m.ref_density;
