@@ -83,6 +83,8 @@ struct Dev {
   double* dt_next = nullptr;  // nnode: the time step being computed while the Jacobian rows read dt
   double* qjac = nullptr;   // 5 x ntot: states the Jacobian rows read when hard-set nodes are committed early
   double* qrk = nullptr;    // 5 x ntot: the state a four-stage Runge-Kutta step starts from (allocated on first use)
+  double* aos = nullptr;    // a caller's array in its own order, between a copy and a transposition (grows on use)
+  size_t aos_n = 0;         // doubles in it
   // SELL block matrix
   int* srow = nullptr;      // nrow_pad: node of each padded row (-1 = padding)
   int* swidth = nullptr;    // nchunk_s
@@ -107,11 +109,19 @@ struct Dev {
   int* icount = nullptr;
 };
 
+constexpr size_t kPin = 1 << 18;  // 2 MiB
+constexpr int kMinParts = 1024;   // at most that many partial minima
+constexpr size_t kPinAll = kPin + 8 + kMinParts;
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   hipStream_t stream2 = nullptr;  // Jacobian rows, overlapped with the edge passes (default priority)
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  hipEvent_t ev_norms = nullptr;  // the residual norms are in pin
+  // pinned host memory that kernels write to and read from: kPin values of a
+  // small caller's array, then the norms' six sums, then partial minima
+  double *pin = nullptr, *pin_dev = nullptr;
   bool overlap = true;            // PCFD_JACOBIAN_STREAM=0 turns the overlap off
   bool jac_pending = false;
   std::string err;
@@ -300,9 +310,15 @@ void launch_limiter(Ctx& c);
 void launch_gradient_limiter(Ctx& c, int nterms);  // LSQ gradient + limiter in one pass, then the clip
 void launch_residual(Ctx& c, int higher_order);  // inviscid, then viscous / noSlip edits
 void launch_viscous(Ctx& c, int higher_order);
-void launch_norms(Ctx& c, double* host_norms6);
+void launch_norms(Ctx& c);                         // sums to pin, ev_norms behind them
+void wait_norms(Ctx& c, double* host_norms6);      // their values once they are there
 void launch_timestep(Ctx& c, double cfl);
 double launch_dtmin(Ctx& c);
+// copies between a caller's arrays and the device's component arrays
+void soa_to_host(Ctx& c, const double* soa, int ld, int n, int ncomp, double* host);
+void soa_from_host(Ctx& c, double* soa, int ld, int n, int ncomp, const double* host, int stride);
+void state_to_host(Ctx& c, double gamma, double* host, int nvars);
+void launch_ones(Ctx& c, size_t n, double* v);
 void launch_jacobian(Ctx& c);
 void launch_jacobian_overlapped(Ctx& c);  // rows on stream2; jacobian_join() before the matrix is used
 void jacobian_join(Ctx& c);

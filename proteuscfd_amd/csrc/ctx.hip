@@ -47,7 +47,9 @@ void dfree(T*& p) {
 
 void free_all(Ctx& c) {
   Dev& d = c.d;
-  dfree(d.xyz); dfree(d.vol); dfree(d.vol23); dfree(d.sw); dfree(d.gwidth); dfree(d.gbase); dfree(d.gcol); dfree(d.gnrm); dfree(d.qrk);
+  dfree(d.xyz); dfree(d.vol); dfree(d.vol23); dfree(d.sw); dfree(d.gwidth); dfree(d.gbase); dfree(d.gcol); dfree(d.gnrm); dfree(d.qrk); dfree(d.aos);
+  if (c.pin) (void)hipHostFree(c.pin);
+  c.pin = c.pin_dev = nullptr;
   dfree(d.he_ptr); dfree(d.he_id); dfree(d.he_tag); dfree(d.he_node); dfree(d.seen); dfree(d.he_desc); dfree(d.rst); dfree(d.he_a); dfree(d.bnd_nodes); dfree(d.bidx);
   dfree(d.jdb); dfree(d.jhe); dfree(d.jcol); dfree(d.jqb); dfree(d.bc_type); dfree(d.twall); dfree(d.spos);
   dfree(d.qref); dfree(d.q); dfree(d.grad); dfree(d.lim); dfree(d.lim2); dfree(d.edges); dfree(d.clip_flag); dfree(d.clip_cnt);
@@ -55,7 +57,7 @@ void free_all(Ctx& c) {
   dfree(d.gslot); dfree(d.srow); dfree(d.swidth); dfree(d.swidth_lo); dfree(d.sbase); dfree(d.scol); dfree(d.Md); dfree(d.Mf); dfree(d.Dd);
   dfree(d.Df); dfree(d.bsd); dfree(d.bsf); dfree(d.xsd); dfree(d.xsf); dfree(d.psd); dfree(d.psf); dfree(d.xd); dfree(d.xf); dfree(d.red);
   dfree(d.red_out); dfree(d.icount); dfree(d.dt_next); dfree(d.qjac);
-  for (hipEvent_t* e : {&c.ev0, &c.ev1, &c.ev2, &c.ev3, &c.ev4, &c.ev5, &c.ev_fork, &c.ev_join}) {
+  for (hipEvent_t* e : {&c.ev0, &c.ev1, &c.ev2, &c.ev3, &c.ev4, &c.ev5, &c.ev_fork, &c.ev_join, &c.ev_norms}) {
     if (*e) (void)hipEventDestroy(*e);
     *e = nullptr;
   }
@@ -204,6 +206,9 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     PCFD_HIP(hipStreamCreateWithFlags(&c.stream2, hipStreamNonBlocking));
     PCFD_HIP(hipEventCreateWithFlags(&c.ev_fork, hipEventDisableTiming));
     PCFD_HIP(hipEventCreateWithFlags(&c.ev_join, hipEventDisableTiming));
+    PCFD_HIP(hipEventCreateWithFlags(&c.ev_norms, hipEventDisableTiming));
+    PCFD_HIP(hipHostMalloc((void**)&c.pin, sizeof(double) * kPinAll, hipHostMallocMapped));
+    PCFD_HIP(hipHostGetDevicePointer((void**)&c.pin_dev, c.pin, 0));
     if (const char* e = std::getenv("PCFD_JACOBIAN_STREAM")) c.overlap = std::strcmp(e, "0") != 0;
     c.nnode = nn;
     c.nbnode = nb;
@@ -541,11 +546,7 @@ int pcfd_upload_q(pcfd_ctx* ctx, const double* q, int nvars) {
       c.err = "pcfd_upload_q: need q and nvars >= 5";
       return PCFD_ERR_ARG;
     }
-    std::vector<double> s(5 * (size_t)c.ntot);
-    for (int i = 0; i < c.ntot; ++i)
-      for (int k = 0; k < 5; ++k) s[(size_t)k * c.ntot + i] = q[(size_t)i * nvars + k];
-    PCFD_HIP(hipMemcpyAsync(c.d.q, s.data(), s.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
-    PCFD_HIP(hipStreamSynchronize(c.stream));
+    soa_from_host(c, c.d.q, c.ntot, c.ntot, 5, q, nvars);
     return PCFD_OK;
   });
 }
@@ -556,25 +557,7 @@ int pcfd_download_q(pcfd_ctx* ctx, double* q, int nvars) {
       c.err = "pcfd_download_q: need q and nvars >= 5";
       return PCFD_ERR_ARG;
     }
-    std::vector<double> s(5 * (size_t)c.ntot);
-    PCFD_HIP(hipMemcpyAsync(s.data(), c.d.q, s.size() * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    PCFD_HIP(hipStreamSynchronize(c.stream));
-    const double gamma = c.have_params ? c.prm.gamma : 1.4;
-    for (int i = 0; i < c.ntot; ++i) {
-      double* Q = q + (size_t)i * nvars;
-      for (int k = 0; k < 5; ++k) Q[k] = s[(size_t)k * c.ntot + i];
-      if (nvars >= 10) {
-        double gm1 = gamma - 1.0;
-        double u = Q[1] / Q[0], v = Q[2] / Q[0], w = Q[3] / Q[0];
-        double P = gm1 * (Q[4] - 0.5 * Q[0] * (u * u + v * v + w * w));
-        double v2h = 0.5 * (u * u + v * v + w * w);
-        Q[5] = gamma * (gm1 * (Q[4] - Q[0] * v2h)) / Q[0];
-        Q[6] = P;
-        Q[7] = u;
-        Q[8] = v;
-        Q[9] = w;
-      }
-    }
+    state_to_host(c, c.have_params ? c.prm.gamma : 1.4, q, nvars);
     return PCFD_OK;
   });
 }
@@ -589,20 +572,12 @@ int pcfd_update_bcs(pcfd_ctx* ctx) {
 }
 
 static int download_soa(Ctx& c, const double* dsrc, int ncomp, double* host) {
-  std::vector<double> s((size_t)ncomp * c.nnode);
-  PCFD_HIP(hipMemcpyAsync(s.data(), dsrc, s.size() * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  PCFD_HIP(hipStreamSynchronize(c.stream));
-  for (int i = 0; i < c.nnode; ++i)
-    for (int k = 0; k < ncomp; ++k) host[(size_t)i * ncomp + k] = s[(size_t)k * c.nnode + i];
+  soa_to_host(c, dsrc, c.nnode, c.nnode, ncomp, host);
   return PCFD_OK;
 }
 
 static int upload_soa(Ctx& c, double* ddst, int ncomp, const double* host) {
-  std::vector<double> s((size_t)ncomp * c.nnode);
-  for (int i = 0; i < c.nnode; ++i)
-    for (int k = 0; k < ncomp; ++k) s[(size_t)k * c.nnode + i] = host[(size_t)i * ncomp + k];
-  PCFD_HIP(hipMemcpyAsync(ddst, s.data(), s.size() * sizeof(double), hipMemcpyHostToDevice, c.stream));
-  PCFD_HIP(hipStreamSynchronize(c.stream));
+  soa_from_host(c, ddst, c.nnode, c.nnode, ncomp, host, ncomp);
   return PCFD_OK;
 }
 
@@ -646,8 +621,9 @@ int pcfd_residual(pcfd_ctx* ctx, int iter, double* b_out, double norms[6]) {
     if (int r = need_params(c)) return r;
     int ho = (c.prm.sorder > 1 && iter > c.prm.nfirst) ? 1 : 0;
     launch_residual(c, ho);
-    launch_norms(c, norms);
-    if (b_out) return download_soa(c, c.d.b, 5, b_out);
+    launch_norms(c);
+    if (b_out) download_soa(c, c.d.b, 5, b_out);
+    if (norms) wait_norms(c, norms);
     PCFD_HIP(hipStreamSynchronize(c.stream));
     return PCFD_OK;
   });

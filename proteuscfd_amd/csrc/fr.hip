@@ -1521,10 +1521,14 @@ int pcfd_fr_upload_q(pcfd_fr* fp, const double* q, int stride) {
       f.err = "pcfd_fr_upload_q: stride must be at least ns + 4";
       return PCFD_ERR_ARG;
     }
-    std::vector<double> h((size_t)f.ntot * f.ne);
-    for (size_t i = 0; i < (size_t)f.ntot; ++i)
-      for (int k = 0; k < f.ne; ++k) h[i * f.ne + k] = q[i * stride + k];
-    hcheck(hipMemcpyAsync(f.q, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice, f.stream), "copy");
+    std::vector<double> h;
+    if (stride != f.ne) {
+      h.resize((size_t)f.ntot * f.ne);
+      for (size_t i = 0; i < (size_t)f.ntot; ++i)
+        for (int k = 0; k < f.ne; ++k) h[i * f.ne + k] = q[i * stride + k];
+      q = h.data();
+    }
+    hcheck(hipMemcpyAsync(f.q, q, sizeof(double) * (size_t)f.ntot * f.ne, hipMemcpyHostToDevice, f.stream), "copy");
     hcheck(hipStreamSynchronize(f.stream), "sync");
     return PCFD_OK;
   });
@@ -1535,6 +1539,11 @@ int pcfd_fr_download_q(pcfd_fr* fp, double* q, int stride) {
     if (!q || stride < f.ne) {
       f.err = "pcfd_fr_download_q: stride must be at least ns + 4";
       return PCFD_ERR_ARG;
+    }
+    if (stride == f.ne) {
+      hcheck(hipMemcpyAsync(q, f.q, sizeof(double) * (size_t)f.ntot * f.ne, hipMemcpyDeviceToHost, f.stream), "copy");
+      hcheck(hipStreamSynchronize(f.stream), "sync");
+      return PCFD_OK;
     }
     std::vector<double> h((size_t)f.ntot * f.ne);
     hcheck(hipMemcpyAsync(h.data(), f.q, sizeof(double) * h.size(), hipMemcpyDeviceToHost, f.stream), "copy");

@@ -822,22 +822,21 @@ __global__ void __launch_bounds__(kBlock) k_residual(int nnode, int ntot, double
   block_norm_partials(bi, red, blk);
 }
 
-// final reduction of the per-block partial sums (single block, fixed order)
+// final reduction of the per-block partial sums (a block a sum, fixed order),
+// into pinned host memory
 __global__ void __launch_bounds__(kBlock) k_reduce6(int nparts, const double* __restrict__ red,
                                                    double* __restrict__ out) {
   __shared__ double sh[kBlock];
-  for (int k = 0; k < 6; ++k) {
-    double s = 0.0;
-    for (int p = threadIdx.x; p < nparts; p += blockDim.x) s += red[k * nparts + p];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[k] = sh[0];
+  const int k = blockIdx.x;
+  double s = 0.0;
+  for (int p = threadIdx.x; p < nparts; p += blockDim.x) s += red[k * nparts + p];
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  for (int w = kBlock / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
     __syncthreads();
   }
+  if (threadIdx.x == 0) out[k] = sh[0];
 }
 
 template <int LPN>
@@ -864,16 +863,17 @@ void launch_residual(Ctx& c, int ho) {
 
 // residGlobal = sqrt(sum b^2)/(nnode*neqn), per-equation sqrt(sum b_k^2)/nnode
 // (ParallelL2Norm / StridedParallelL2Norm, ucs/parallel.h:120-182)
-void launch_norms(Ctx& c, double* host6) {
-  hipLaunchKernelGGL(k_reduce6, dim3(1), dim3(kBlock), 0, c.stream, c.nred, c.d.red, c.d.red_out);
+void launch_norms(Ctx& c) {
+  hipLaunchKernelGGL(k_reduce6, dim3(6), dim3(kBlock), 0, c.stream, c.nred, c.d.red, c.pin_dev + kPin);
   PCFD_HIP(hipGetLastError());
-  if (host6) {
-    double s[6];
-    PCFD_HIP(hipMemcpyAsync(s, c.d.red_out, sizeof(s), hipMemcpyDeviceToHost, c.stream));
-    PCFD_HIP(hipStreamSynchronize(c.stream));
-    host6[0] = std::sqrt(s[0]) / (double)((long long)c.nnode * 5);
-    for (int k = 0; k < 5; ++k) host6[1 + k] = std::sqrt(s[1 + k]) / (double)c.nnode;
-  }
+  PCFD_HIP(hipEventRecord(c.ev_norms, c.stream));
+}
+
+void wait_norms(Ctx& c, double* host6) {
+  PCFD_HIP(hipEventSynchronize(c.ev_norms));
+  const double* s = c.pin + kPin;
+  host6[0] = std::sqrt(s[0]) / (double)((long long)c.nnode * 5);
+  for (int k = 0; k < 5; ++k) host6[1 + k] = std::sqrt(s[1 + k]) / (double)c.nnode;
 }
 
 // ---------------------------------------------------------------------------
@@ -993,14 +993,13 @@ void launch_timestep(Ctx& c, double cfl) {
 }
 
 double launch_dtmin(Ctx& c) {
-  int nb = std::min(nblk(c.nnode), 1024);
-  hipLaunchKernelGGL(k_min_partial, dim3(nb), dim3(kBlock), 0, c.stream, c.nnode, c.d.dt, c.d.red);
+  const int nb = std::min(nblk(c.nnode), kMinParts);
+  hipLaunchKernelGGL(k_min_partial, dim3(nb), dim3(kBlock), 0, c.stream, c.nnode, c.d.dt, c.pin_dev + kPin + 8);
   PCFD_HIP(hipGetLastError());
-  std::vector<double> h(nb);
-  PCFD_HIP(hipMemcpyAsync(h.data(), c.d.red, sizeof(double) * nb, hipMemcpyDeviceToHost, c.stream));
   PCFD_HIP(hipStreamSynchronize(c.stream));
+  const double* h = c.pin + kPin + 8;
   double m = h[0];
-  for (double v : h) m = v < m ? v : m;
+  for (int k = 0; k < nb; ++k) m = h[k] < m ? h[k] : m;
   return m;
 }
 

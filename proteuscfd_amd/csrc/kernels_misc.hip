@@ -1,7 +1,9 @@
 // Solution update: NaN/Inf rows of the correction zeroed, then ApplyDQ
 // (ucs/solutionSpace.tcc:772-804, ucs/compressible.tcc:928-993), and the
 // explicit update (ExplicitSolve, ucs/solve.tcc:70-101).
+#include <algorithm>
 #include <stdexcept>
+#include <vector>
 
 #include "common.h"
 #include "physics.h"
@@ -174,6 +176,156 @@ void launch_apply_dq(Ctx& c, int explicit_mode, int* nzeroed) {
     PCFD_HIP(hipMemcpyAsync(nzeroed, c.d.icount, sizeof(int), hipMemcpyDeviceToHost, c.stream));
     PCFD_HIP(hipStreamSynchronize(c.stream));
   }
+}
+
+// ---- callers' arrays ---------------------------------------------------------
+// A caller's arrays hold a node's components together, the device one array a
+// component.  The reordering is the device's: it is one pass at memory speed
+// there, and the caller's array is filled by a single copy.  (On the host, with
+// its own buffer between the copy and the reordering, the gradient of 39k nodes,
+// 8.5 MB, took 1450 us to reach the caller; 650 so.)
+
+// aos[i * stride + k] = soa[k * ld + i], k < ncomp
+__global__ void __launch_bounds__(kBlock) k_to_aos(long long n, int ncomp, int ld, const double* __restrict__ soa,
+                                                  double* __restrict__ aos) {
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n * ncomp) return;
+  aos[t] = soa[t % ncomp * ld + t / ncomp];
+}
+
+__global__ void __launch_bounds__(kBlock) k_from_aos(int n, int ncomp, int ld, int stride,
+                                                    const double* __restrict__ aos, double* __restrict__ soa) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  for (int k = 0; k < ncomp; ++k) soa[(long long)k * ld + i] = aos[(long long)i * stride + k];
+}
+
+// rows of the full state: the conservative values and what follows from them,
+// in the host's arithmetic (no contracted products)
+__global__ void __launch_bounds__(kBlock) k_full_state(int ntot, double gamma, const double* __restrict__ q,
+                                                      double* __restrict__ aos) {
+#pragma clang fp contract(off)
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= ntot) return;
+  double Q[10];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) Q[k] = q[(long long)k * ntot + i];
+  const double gm1 = gamma - 1.0;
+  const double u = Q[1] / Q[0], v = Q[2] / Q[0], w = Q[3] / Q[0];
+  const double P = gm1 * (Q[4] - 0.5 * Q[0] * (u * u + v * v + w * w));
+  const double v2h = 0.5 * (u * u + v * v + w * w);
+  Q[5] = gamma * (gm1 * (Q[4] - Q[0] * v2h)) / Q[0];
+  Q[6] = P;
+  Q[7] = u;
+  Q[8] = v;
+  Q[9] = w;
+#pragma unroll
+  for (int k = 0; k < 10; ++k) aos[(long long)i * 10 + k] = Q[k];
+}
+
+__global__ void __launch_bounds__(kBlock) k_ones(size_t n, double* __restrict__ v) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) v[i] = 1.0;
+}
+
+static double* aos_space(Ctx& c, size_t n) {
+  if (c.d.aos_n < n) {
+    // the stream may still be reading the old one
+    PCFD_HIP(hipStreamSynchronize(c.stream));
+    if (c.d.aos) PCFD_HIP(hipFree(c.d.aos));
+    c.d.aos = nullptr;
+    c.d.aos_n = 0;
+    PCFD_HIP(hipMalloc((void**)&c.d.aos, sizeof(double) * n));
+    c.d.aos_n = n;
+  }
+  return c.d.aos;
+}
+
+// Where a kernel leaves or finds a caller's array of n values: up to kPin in
+// pinned host memory, which the host copies to or from itself, more in device
+// memory.  A copy engine's start costs more than the kernel's own trip over the
+// bus: 37k values went up in 137 and came down in 154 us through device memory,
+// in 26 and 30 through pinned; at 220k both took 80-100 and 130-140.
+static double* space_of(Ctx& c, size_t n) { return n <= kPin ? c.pin_dev : aos_space(c, n); }
+
+// the n rows of ncomp values a kernel has left there into the caller's rows of
+// `stride` values, the stream's work done on return
+static void rows_to_host(Ctx& c, size_t n, int ncomp, double* host, int stride) {
+  const size_t m = n * ncomp;
+  const double* src = c.pin;
+  std::vector<double> s;
+  if (m <= kPin) {
+    PCFD_HIP(hipStreamSynchronize(c.stream));
+    if (stride == ncomp) std::copy(src, src + m, host);
+  } else {
+    double* to = host;
+    if (stride != ncomp) {
+      s.resize(m);
+      src = to = s.data();
+    }
+    PCFD_HIP(hipMemcpyAsync(to, c.d.aos, sizeof(double) * m, hipMemcpyDeviceToHost, c.stream));
+    PCFD_HIP(hipStreamSynchronize(c.stream));
+  }
+  if (stride != ncomp)
+    for (size_t i = 0; i < n; ++i)
+      for (int k = 0; k < ncomp; ++k) host[i * stride + k] = src[i * ncomp + k];
+}
+
+void soa_to_host(Ctx& c, const double* soa, int ld, int n, int ncomp, double* host) {
+  const size_t m = (size_t)n * ncomp;
+  if (ncomp == 1 && m > kPin) {
+    PCFD_HIP(hipMemcpyAsync(host, soa, sizeof(double) * m, hipMemcpyDeviceToHost, c.stream));
+    PCFD_HIP(hipStreamSynchronize(c.stream));
+    return;
+  }
+  hipLaunchKernelGGL(k_to_aos, dim3((unsigned)((m + kBlock - 1) / kBlock)), dim3(kBlock), 0, c.stream, (long long)n,
+                     ncomp, ld, soa, space_of(c, m));
+  PCFD_HIP(hipGetLastError());
+  rows_to_host(c, n, ncomp, host, ncomp);
+}
+
+// rows of up to kWide values go up as they are; of wider ones only what is read
+constexpr int kWide = 10;
+
+void soa_from_host(Ctx& c, double* soa, int ld, int n, int ncomp, const double* host, int stride) {
+  std::vector<double> s;
+  if (stride > kWide) {
+    s.resize((size_t)n * ncomp);
+    for (size_t i = 0; i < (size_t)n; ++i)
+      for (int k = 0; k < ncomp; ++k) s[i * ncomp + k] = host[i * stride + k];
+    host = s.data();
+    stride = ncomp;
+  }
+  // the last row's columns past the components are not read: a caller's array
+  // may end with them
+  const size_t m = (size_t)(n - 1) * stride + ncomp;
+  double* aos = space_of(c, m);
+  if (m <= kPin) {
+    // nothing on the stream still reads the pinned rows: every use waits for its own
+    std::copy(host, host + m, c.pin);
+  } else {
+    PCFD_HIP(hipMemcpyAsync(aos, host, sizeof(double) * m, hipMemcpyHostToDevice, c.stream));
+  }
+  hipLaunchKernelGGL(k_from_aos, dim3(nblk(n)), dim3(kBlock), 0, c.stream, n, ncomp, ld, stride, aos, soa);
+  PCFD_HIP(hipGetLastError());
+  PCFD_HIP(hipStreamSynchronize(c.stream));
+}
+
+void state_to_host(Ctx& c, double gamma, double* host, int nvars) {
+  const int ncol = nvars >= 10 ? 10 : 5;
+  double* aos = space_of(c, (size_t)c.ntot * ncol);
+  if (ncol == 10)
+    hipLaunchKernelGGL(k_full_state, dim3(nblk(c.ntot)), dim3(kBlock), 0, c.stream, c.ntot, gamma, c.d.q, aos);
+  else
+    hipLaunchKernelGGL(k_to_aos, dim3((unsigned)((5LL * c.ntot + kBlock - 1) / kBlock)), dim3(kBlock), 0, c.stream,
+                       (long long)c.ntot, 5, c.ntot, c.d.q, aos);
+  PCFD_HIP(hipGetLastError());
+  rows_to_host(c, (size_t)c.ntot, ncol, host, nvars);
+}
+
+void launch_ones(Ctx& c, size_t n, double* v) {
+  hipLaunchKernelGGL(k_ones, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, c.stream, n, v);
+  PCFD_HIP(hipGetLastError());
 }
 
 }  // namespace pcfd

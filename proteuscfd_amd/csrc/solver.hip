@@ -99,9 +99,9 @@ void iterate(Ctx& c, double* resid) {
   phase_begin(c);
   launch_residual(c, ho ? 1 : 0);
   phase_end(c, 3);
-  launch_norms(c, resid);
-  c.res_nm1 = c.res;  // ucs/solutionSpace.tcc:705-706
-  c.res = resid[0];
+  // waited for at the end: the update is on its way by then, and no launch of
+  // it depends on them
+  launch_norms(c);
   if (p.nsgs > 0) {
     jacobian_join(c);
     if (!c.lu_done) {
@@ -144,6 +144,9 @@ void iterate(Ctx& c, double* resid) {
     launch_apply_dq(c, 1, nullptr);
     phase_end(c, 8);
   }
+  wait_norms(c, resid);
+  c.res_nm1 = c.res;  // ucs/solutionSpace.tcc:705-706
+  c.res = resid[0];
   c.iter++;
 }
 
@@ -166,8 +169,7 @@ int pcfd_reset_iteration(pcfd_ctx* ctx) {
     c.jac_valid = false;
     c.lu_done = false;
     // Limiter ctor fills 1.0 (ucs/limiters.tcc:39-43); PreIterate computes dt
-    std::vector<double> ones(5 * (size_t)c.nnode, 1.0);
-    PCFD_HIP(hipMemcpy(c.d.lim, ones.data(), ones.size() * sizeof(double), hipMemcpyHostToDevice));
+    launch_ones(c, 5 * (size_t)c.nnode, c.d.lim);
     c.res = c.res_nm1 = 0.0;
     c.cfl = cfl_update(c.prm, c.iter, 0.0, 0.0, c.prm.cfl_start);
     launch_timestep(c, c.cfl);
