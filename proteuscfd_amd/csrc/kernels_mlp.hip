@@ -69,22 +69,27 @@ struct MlpWeights {
   const short* W1;   // [64][16] bf16
   const short* W2;   // [64][64]
   const short* W3;   // [16][64]
+  const short* W2t;  // transposes of W2, W3
+  const short* W3t;  // [64][16]
   const float* p;    // FP32 parameters (biases read from here)
 };
 
-// per-wavefront LDS tiles
+// LDS tiles of one wavefront.  Rows are 4 values longer than their 64 or 16: a
+// fragment's 16 rows then lie in different banks (at 64 they shared 4 of them).
+constexpr int kLdH = kNh + 4, kLdX = kKin + 4;
+static_assert(kKin == kKout, "one row length for X and DY");
 struct WaveTiles {
-  float X[16][kKin];
-  float H1[16][kNh];
-  float H2[16][kNh];
-  float D1[16][kNh];  // dZ1
-  float D2[16][kNh];  // dZ2
-  float DY[16][kKout];
+  alignas(16) float X[16][kLdX];
+  alignas(16) float H1[16][kLdH];
+  alignas(16) float H2[16][kLdH];
+  alignas(16) float D1[16][kLdH];  // dZ1
+  alignas(16) float D2[16][kLdH];  // dZ2
+  alignas(16) float DY[16][kLdX];
 };
 
 __device__ __forceinline__ bf16x4 frag_rows(const float* base, int stride, int row, int k0) {
   // A operand from a row-major FP32 tile: row `row`, columns k0..k0+3
-  const float* p = base + row * stride + k0;
+  const f32x4 p = *reinterpret_cast<const f32x4*>(base + row * stride + k0);
   bf16x4 v;
   v[0] = f2bf(p[0]);
   v[1] = f2bf(p[1]);
@@ -104,73 +109,72 @@ __device__ __forceinline__ bf16x4 frag_cols(const float* base, int stride, int k
 }
 
 __device__ __forceinline__ bf16x4 wfrag(const short* W, int stride, int row, int k0) {
-  const short* p = W + row * stride + k0;
-  bf16x4 v;
-  v[0] = p[0];
-  v[1] = p[1];
-  v[2] = p[2];
-  v[3] = p[3];
-  return v;
+  return *reinterpret_cast<const bf16x4*>(W + row * stride + k0);
 }
 
-__device__ __forceinline__ bf16x4 wfrag_cols(const short* W, int stride, int k0, int col) {
-  bf16x4 v;
-  v[0] = W[(k0 + 0) * stride + col];
-  v[1] = W[(k0 + 1) * stride + col];
-  v[2] = W[(k0 + 2) * stride + col];
-  v[3] = W[(k0 + 3) * stride + col];
-  return v;
+// A wavefront's weights for forward and backward, in registers for all its tiles
+struct TrainRegs {
+  bf16x4 w1[4], w2[4][4], w3[4], w2t[4][4], w3t[4];
+  float b1[4], b2[4], b3;
+};
+
+__device__ __forceinline__ void load_train_regs(const MlpWeights& w, int r, int q, TrainRegs& R) {
+#pragma unroll
+  for (int nt = 0; nt < 4; ++nt) {
+    R.w1[nt] = wfrag(w.W1, kKin, nt * 16 + r, 4 * q);
+    R.b1[nt] = w.p[oB1 + nt * 16 + r];
+    R.b2[nt] = w.p[oB2 + nt * 16 + r];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+      R.w2[nt][kt] = wfrag(w.W2, kNh, nt * 16 + r, kt * 16 + 4 * q);
+      R.w2t[nt][kt] = wfrag(w.W2t, kNh, nt * 16 + r, kt * 16 + 4 * q);
+    }
+    R.w3[nt] = wfrag(w.W3, kNh, r, nt * 16 + 4 * q);
+    R.w3t[nt] = wfrag(w.W3t, kKout, nt * 16 + r, 4 * q);
+  }
+  R.b3 = w.p[oB3 + r];
 }
 
 // Forward pass of one 16-sample tile held in T.X; leaves H1, H2 in LDS and
 // returns Y in the D layout (lane: Y[4q+j][r]).
-__device__ __forceinline__ f32x4 tile_forward(const MlpWeights& w, WaveTiles& T, int r, int q) {
+__device__ __forceinline__ f32x4 tile_forward(const TrainRegs& R, WaveTiles& T, int r, int q) {
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  const bf16x4 ax = frag_rows(&T.X[0][0], kKin, r, 4 * q);
+  const bf16x4 ax = frag_rows(&T.X[0][0], kLdX, r, 4 * q);
 #pragma unroll
   for (int nt = 0; nt < 4; ++nt) {
-    f32x4 acc = mfma(ax, wfrag(w.W1, kKin, nt * 16 + r, 4 * q), zero);
-    const float b = w.p[oB1 + nt * 16 + r];
+    f32x4 acc = mfma(ax, R.w1[nt], zero);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) T.H1[4 * q + j][nt * 16 + r] = tanh_fast(acc[j] + b);
+    for (int j = 0; j < 4; ++j) T.H1[4 * q + j][nt * 16 + r] = tanh_fast(acc[j] + R.b1[nt]);
   }
   wave_sync();
+  bf16x4 h[4];
+#pragma unroll
+  for (int kt = 0; kt < 4; ++kt) h[kt] = frag_rows(&T.H1[0][0], kLdH, r, kt * 16 + 4 * q);
 #pragma unroll
   for (int nt = 0; nt < 4; ++nt) {
     f32x4 acc = zero;
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-      acc = mfma(frag_rows(&T.H1[0][0], kNh, r, kt * 16 + 4 * q), wfrag(w.W2, kNh, nt * 16 + r, kt * 16 + 4 * q),
-                 acc);
-    const float b = w.p[oB2 + nt * 16 + r];
+    for (int kt = 0; kt < 4; ++kt) acc = mfma(h[kt], R.w2[nt][kt], acc);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) T.H2[4 * q + j][nt * 16 + r] = tanh_fast(acc[j] + b);
+    for (int j = 0; j < 4; ++j) T.H2[4 * q + j][nt * 16 + r] = tanh_fast(acc[j] + R.b2[nt]);
   }
   wave_sync();
   f32x4 y = zero;
 #pragma unroll
-  for (int kt = 0; kt < 4; ++kt)
-    y = mfma(frag_rows(&T.H2[0][0], kNh, r, kt * 16 + 4 * q), wfrag(w.W3, kNh, r, kt * 16 + 4 * q), y);
-  const float b3 = w.p[oB3 + r];
+  for (int kt = 0; kt < 4; ++kt) y = mfma(frag_rows(&T.H2[0][0], kLdH, r, kt * 16 + 4 * q), R.w3[kt], y);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) y[j] += b3;
+  for (int j = 0; j < 4; ++j) y[j] += R.b3;
   return y;
 }
 
-__device__ __forceinline__ void load_x_tile(WaveTiles& T, const float* __restrict__ x, const int* __restrict__ idx,
-                                            int n, int s0, int lane) {
-  // 16 samples x 16 features (7 used): 4 entries per lane
+// src: the row of x that holds the tile's sample lane & 15 (below 0: past the batch)
+__device__ __forceinline__ void load_x_tile(WaveTiles& T, const float* __restrict__ x, int src, int lane) {
+  // 16 samples x 16 features (7 used): 4 entries of sample lane / 4 per lane
+  const int g = __shfl(src, lane >> 2);
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int flat = lane * 4 + e;
-    const int s = flat >> 4, f = flat & 15;
-    const int g = s0 + s;
-    float v = 0.f;
-    if (g < n && f < kNin) {
-      const long long src = idx ? (long long)idx[g] : (long long)g;
-      v = x[src * kNin + f];
-    }
-    T.X[s][f] = v;
+    const int f = (lane & 3) * 4 + e;
+    T.X[lane >> 2][f] = g >= 0 && f < kNin ? x[(long long)g * kNin + f] : 0.f;
   }
 }
 
@@ -264,16 +268,24 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_forward(MlpWeights w, int n, 
   }
 }
 
-// Loss and gradient partials of a batch: per wavefront, sum over its tiles.
-// partial[(block*kWaves + wave)*kNparam + i], lossp[block*kWaves + wave].
-__global__ void __launch_bounds__(kMlpBlock) k_mlp_grad(MlpWeights w, int n, const float* __restrict__ x,
+// Loss and gradient partials of a batch: a block is one wavefront, which sums
+// over its 16-sample tiles; partial[block * kNparam + i], lossp[block].
+// A batch of a few thousand samples gives a wavefront one tile or none, so what
+// bounds the kernel is the chain through the tile, not a rate: the weights come
+// first and at once, from rows a fragment is 8 consecutive bytes of, the
+// exchanges through LDS are free of bank conflicts, and a wavefront has its own
+// block so that all compute units share the tiles.  (Weights read where they
+// are used, the transposed ones in 2-byte pieces, rows 16-way in the same banks,
+// four wavefronts a block: 22.5 us for 8192 samples; 15.6 so.)
+__global__ void __launch_bounds__(64) k_mlp_grad(MlpWeights w, int n, const float* __restrict__ x,
                                                        const float* __restrict__ t, const int* __restrict__ idx,
                                                        float inv_count, float* __restrict__ partial,
                                                        float* __restrict__ lossp) {
-  __shared__ WaveTiles tiles[kWaves];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  __shared__ WaveTiles T;
+  const int lane = threadIdx.x;
   const int r = lane & 15, q = lane >> 4;
-  WaveTiles& T = tiles[wv];
+  TrainRegs R;
+  load_train_regs(w, r, q, R);
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   f32x4 gW1[4], gW2[4][4], gW3[4];
 #pragma unroll
@@ -285,19 +297,26 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_grad(MlpWeights w, int n, con
   }
   float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, loss = 0.f;
   const int ntile = (n + 15) / 16;
-  for (int tile = blockIdx.x * kWaves + wv; tile < ntile; tile += gridDim.x * kWaves) {
+  for (int tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
     const int s0 = tile * 16;
-    load_x_tile(T, x, idx, n, s0, lane);
+    // one read of the indices, which may lie in pinned host memory
+    const int src = s0 + r < n ? (idx ? idx[s0 + r] : s0 + r) : -1;
+    float tt[4];  // targets of this lane's output for its samples
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int g = __shfl(src, 4 * q + j);
+      tt[j] = r < kNout && g >= 0 ? t[(long long)g * kNout + r] : 0.f;
+    }
+    load_x_tile(T, x, src, lane);
     wave_sync();
-    const f32x4 yy = tile_forward(w, T, r, q);
+    const f32x4 yy = tile_forward(R, T, r, q);
     // dY = 2 (y - t) / (count) on the 5 outputs of valid samples
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int s = s0 + 4 * q + j;
       float d = 0.f;
       if (r < kNout && s < n) {
-        const long long src = idx ? (long long)idx[s] : (long long)s;
-        const float e = yy[j] - t[src * kNout + r];
+        const float e = yy[j] - tt[j];
         loss += e * e;
         d = 2.f * e * inv_count;
       }
@@ -307,7 +326,7 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_grad(MlpWeights w, int n, con
     // dW3 += dY^T H2 ; db3
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
-      gW3[kt] = mfma(frag_cols(&T.DY[0][0], kKout, 4 * q, r), frag_cols(&T.H2[0][0], kNh, 4 * q, kt * 16 + r),
+      gW3[kt] = mfma(frag_cols(&T.DY[0][0], kLdX, 4 * q, r), frag_cols(&T.H2[0][0], kLdH, 4 * q, kt * 16 + r),
                      gW3[kt]);
     if (lane < 16) {
 #pragma unroll
@@ -316,7 +335,7 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_grad(MlpWeights w, int n, con
     // dH2 = dY W3 ; dZ2 = dH2 (1 - H2^2)
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
-      f32x4 d = mfma(frag_rows(&T.DY[0][0], kKout, r, 4 * q), wfrag_cols(w.W3, kNh, 4 * q, kt * 16 + r), zero);
+      f32x4 d = mfma(frag_rows(&T.DY[0][0], kLdX, r, 4 * q), R.w3t[kt], zero);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float h = T.H2[4 * q + j][kt * 16 + r];
@@ -327,10 +346,10 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_grad(MlpWeights w, int n, con
     // dW2 += dZ2^T H1 ; db2
 #pragma unroll
     for (int ht = 0; ht < 4; ++ht) {
-      const bf16x4 a = frag_cols(&T.D2[0][0], kNh, 4 * q, ht * 16 + r);
+      const bf16x4 a = frag_cols(&T.D2[0][0], kLdH, 4 * q, ht * 16 + r);
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
-        gW2[ht][kt] = mfma(a, frag_cols(&T.H1[0][0], kNh, 4 * q, kt * 16 + r), gW2[ht][kt]);
+        gW2[ht][kt] = mfma(a, frag_cols(&T.H1[0][0], kLdH, 4 * q, kt * 16 + r), gW2[ht][kt]);
     }
 #pragma unroll
     for (int s = 0; s < 16; ++s) gb2 += T.D2[s][lane];
@@ -340,7 +359,7 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_grad(MlpWeights w, int n, con
       f32x4 d = zero;
 #pragma unroll
       for (int hk = 0; hk < 4; ++hk)
-        d = mfma(frag_rows(&T.D2[0][0], kNh, r, hk * 16 + 4 * q), wfrag_cols(w.W2, kNh, hk * 16 + 4 * q, kt * 16 + r),
+        d = mfma(frag_rows(&T.D2[0][0], kLdH, r, hk * 16 + 4 * q), R.w2t[kt][hk],
                  d);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -352,13 +371,13 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_grad(MlpWeights w, int n, con
     // dW1 += dZ1^T X ; db1
 #pragma unroll
     for (int ht = 0; ht < 4; ++ht)
-      gW1[ht] = mfma(frag_cols(&T.D1[0][0], kNh, 4 * q, ht * 16 + r), frag_cols(&T.X[0][0], kKin, 4 * q, r), gW1[ht]);
+      gW1[ht] = mfma(frag_cols(&T.D1[0][0], kLdH, 4 * q, ht * 16 + r), frag_cols(&T.X[0][0], kLdX, 4 * q, r), gW1[ht]);
 #pragma unroll
     for (int s = 0; s < 16; ++s) gb1 += T.D1[s][lane];
     wave_sync();
   }
   // write this wavefront's partial gradient
-  float* P = partial + (long long)(blockIdx.x * kWaves + wv) * kNparam;
+  float* P = partial + (long long)blockIdx.x * kNparam;
 #pragma unroll
   for (int ht = 0; ht < 4; ++ht)
 #pragma unroll
@@ -377,45 +396,48 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_grad(MlpWeights w, int n, con
   if (lane < 16) P[oB3 + lane] = lane < kNout ? gb3 : 0.f;
   // loss partial: fixed butterfly over the wavefront
   for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
-  if (lane == 0) lossp[blockIdx.x * kWaves + wv] = loss;
+  if (lane == 0) lossp[blockIdx.x] = loss;
 }
 
 // Sum of the per-wavefront partials in a fixed order, in two stages so the
 // work spreads over the chip: stage 1 sums groups of kRedGroup consecutive
-// partials (one block row per group), stage 2 sums the group totals.
+// partials (one block row per group, a group's loads all in flight), stage 2
+// sums the group totals.
 constexpr int kRedGroup = 32;
+
+template <int N>
+__device__ __forceinline__ float sum_strided(const float* __restrict__ v, int n, long long stride) {
+  float s = 0.f;
+  int p = 0;
+  for (; p + N <= n; p += N) {
+    float x[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) x[k] = v[(p + k) * stride];
+#pragma unroll
+    for (int k = 0; k < N; ++k) s += x[k];
+  }
+  for (; p < n; ++p) s += v[p * stride];
+  return s;
+}
 
 __global__ void __launch_bounds__(kMlpBlock) k_mlp_reduce1(int nparts, const float* __restrict__ partial,
                                                           const float* __restrict__ lossp, float* __restrict__ part2,
                                                           float* __restrict__ loss2) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int p0 = blockIdx.y * kRedGroup, p1 = min(nparts, p0 + kRedGroup);
-  if (i < kNparam) {
-    float s = 0.f;
-    for (int p = p0; p < p1; ++p) s += partial[(long long)p * kNparam + i];
-    part2[(long long)blockIdx.y * kNparam + i] = s;
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    float s = 0.f;
-    for (int p = p0; p < p1; ++p) s += lossp[p];
-    loss2[blockIdx.y] = s;
-  }
+  if (i < kNparam)
+    part2[(long long)blockIdx.y * kNparam + i] =
+        sum_strided<16>(partial + (long long)p0 * kNparam + i, p1 - p0, kNparam);
+  else if (i == kNparam)
+    loss2[blockIdx.y] = sum_strided<16>(lossp + p0, p1 - p0, 1);
 }
 
 __global__ void __launch_bounds__(kMlpBlock) k_mlp_reduce2(int ngroup, const float* __restrict__ part2,
                                                           const float* __restrict__ loss2, float* __restrict__ grad,
                                                           float* __restrict__ loss) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < kNparam) {
-    float s = 0.f;
-    for (int b = 0; b < ngroup; ++b) s += part2[(long long)b * kNparam + i];
-    grad[i] = s;
-  }
-  if (i == 0) {
-    float s = 0.f;
-    for (int b = 0; b < ngroup; ++b) s += loss2[b];
-    *loss = s;
-  }
+  if (i < kNparam) grad[i] = sum_strided<8>(part2 + i, ngroup, kNparam);
+  else if (i == kNparam) *loss = sum_strided<8>(loss2, ngroup, 1);
 }
 
 // padded entries of the layout stay exactly zero
@@ -426,16 +448,43 @@ __device__ __forceinline__ bool live_param(int i) {
   return true;
 }
 
-__global__ void __launch_bounds__(kMlpBlock) k_mlp_adam(float* __restrict__ p, float* __restrict__ m,
-                                                       float* __restrict__ v, const float* __restrict__ g, float lr,
-                                                       float b1, float b2, float eps, float c1, float c2,
-                                                       short* __restrict__ W1, short* __restrict__ W2,
-                                                       short* __restrict__ W3) {
+// the BF16 weights the kernels read, W2 and W3 in both orders
+struct MlpBf16 {
+  short *W1 = nullptr, *W2 = nullptr, *W3 = nullptr, *W2t = nullptr, *W3t = nullptr;
+};
+
+__device__ __forceinline__ void store_bf16(int i, float v, const MlpBf16& W) {
+  const short b = f2bf(v);
+  if (i < oB1) {
+    W.W1[i - oW1] = b;
+  } else if (i >= oW2 && i < oB2) {
+    const int j = i - oW2;
+    W.W2[j] = b;
+    W.W2t[j % kNh * kNh + j / kNh] = b;
+  } else if (i >= oW3 && i < oB3) {
+    const int j = i - oW3;
+    W.W3[j] = b;
+    W.W3t[j % kNh * kKout + j / kNh] = b;
+  }
+}
+
+// A training step's second stage of the sums and its Adam update: a thread has
+// its parameter's gradient and needs no other's.  (Two launches took 5.2 and
+// 3.7 us of a step, one takes 3.4.)
+constexpr int kAdamBlock = 64;  // kNparam + 1 threads over as many compute units as that gives
+
+__global__ void __launch_bounds__(kAdamBlock) k_mlp_adam(float* __restrict__ p, float* __restrict__ m,
+                                                        float* __restrict__ v, int ngroup,
+                                                        const float* __restrict__ part2,
+                                                        const float* __restrict__ loss2, float* __restrict__ loss,
+                                                        float lr, float b1, float b2, float eps, float c1, float c2,
+                                                        MlpBf16 W) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == kNparam) *loss = sum_strided<8>(loss2, ngroup, 1);
   if (i >= kNparam) return;
   float pi = p[i];
   if (live_param(i)) {
-    const float gi = g[i];
+    const float gi = sum_strided<8>(part2 + i, ngroup, kNparam);
     const float mi = b1 * m[i] + (1.f - b1) * gi;
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
     m[i] = mi;
@@ -445,18 +494,12 @@ __global__ void __launch_bounds__(kMlpBlock) k_mlp_adam(float* __restrict__ p, f
     pi = 0.f;
   }
   p[i] = pi;
-  if (i < oB1) W1[i - oW1] = f2bf(pi);
-  else if (i >= oW2 && i < oB2) W2[i - oW2] = f2bf(pi);
-  else if (i >= oW3 && i < oB3) W3[i - oW3] = f2bf(pi);
+  store_bf16(i, pi, W);
 }
 
-__global__ void k_mlp_to_bf16(const float* __restrict__ p, short* __restrict__ W1, short* __restrict__ W2,
-                              short* __restrict__ W3) {
+__global__ void k_mlp_to_bf16(const float* __restrict__ p, MlpBf16 W) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= kNparam) return;
-  if (i < oB1) W1[i - oW1] = f2bf(p[i]);
-  else if (i >= oW2 && i < oB2) W2[i - oW2] = f2bf(p[i]);
-  else if (i >= oW3 && i < oB3) W3[i - oW3] = f2bf(p[i]);
+  if (i < kNparam) store_bf16(i, p[i], W);
 }
 
 }  // namespace pcfd
@@ -471,7 +514,7 @@ struct pcfd_mlp {
   float* v = nullptr;
   float* g = nullptr;  // gradient
   float* loss = nullptr;
-  short *W1 = nullptr, *W2 = nullptr, *W3 = nullptr;
+  MlpBf16 W;
   float* partial = nullptr;
   float* lossp = nullptr;
   float* part2 = nullptr;  // group totals of the partials
@@ -502,26 +545,33 @@ int guarded_mlp(pcfd_mlp* c, F&& f) {
   }
 }
 
-MlpWeights weights(const pcfd_mlp& c) { return MlpWeights{c.W1, c.W2, c.W3, c.p}; }
+MlpWeights weights(const pcfd_mlp& c) { return MlpWeights{c.W.W1, c.W.W2, c.W.W3, c.W.W2t, c.W.W3t, c.p}; }
 
 void refresh_bf16(pcfd_mlp& c) {
-  hipLaunchKernelGGL(k_mlp_to_bf16, dim3((kNparam + 255) / 256), dim3(256), 0, c.stream, c.p, c.W1, c.W2, c.W3);
+  hipLaunchKernelGGL(k_mlp_to_bf16, dim3((kNparam + 255) / 256), dim3(256), 0, c.stream, c.p, c.W);
   mcheck(hipGetLastError(), "k_mlp_to_bf16");
 }
 
-// loss/gradient of n samples (device arrays, optional index list)
-void grad_device(pcfd_mlp& c, int n, const float* x, const float* t, const int* idx) {
+// group sums of loss and gradient of n samples (device arrays, optional index
+// list); returns the number of groups
+int grad_groups(pcfd_mlp& c, int n, const float* x, const float* t, const int* idx) {
   const int ntile = (n + 15) / 16;
-  const int grid = std::max(1, std::min(c.grid, (ntile + kWaves - 1) / kWaves));
-  hipLaunchKernelGGL(k_mlp_grad, dim3(grid), dim3(kMlpBlock), 0, c.stream, weights(c), n, x, t, idx,
+  const int nparts = std::max(1, std::min(c.grid, ntile));
+  hipLaunchKernelGGL(k_mlp_grad, dim3(nparts), dim3(64), 0, c.stream, weights(c), n, x, t, idx,
                      1.0f / (float)((long long)n * kNout), c.partial, c.lossp);
   mcheck(hipGetLastError(), "k_mlp_grad");
-  const int nparts = grid * kWaves, ngroup = (nparts + kRedGroup - 1) / kRedGroup;
-  hipLaunchKernelGGL(k_mlp_reduce1, dim3((kNparam + kMlpBlock - 1) / kMlpBlock, ngroup), dim3(kMlpBlock), 0,
-                     c.stream, nparts, c.partial, c.lossp, c.part2, c.loss2);
+  const int ngroup = (nparts + kRedGroup - 1) / kRedGroup;
+  hipLaunchKernelGGL(k_mlp_reduce1, dim3(kNparam / kMlpBlock + 1, ngroup), dim3(kMlpBlock), 0, c.stream, nparts,
+                     c.partial, c.lossp, c.part2, c.loss2);
   mcheck(hipGetLastError(), "k_mlp_reduce1");
-  hipLaunchKernelGGL(k_mlp_reduce2, dim3((kNparam + kMlpBlock - 1) / kMlpBlock), dim3(kMlpBlock), 0, c.stream,
-                     ngroup, c.part2, c.loss2, c.g, c.loss);
+  return ngroup;
+}
+
+// loss and gradient of n samples
+void grad_device(pcfd_mlp& c, int n, const float* x, const float* t, const int* idx) {
+  const int ngroup = grad_groups(c, n, x, t, idx);
+  hipLaunchKernelGGL(k_mlp_reduce2, dim3(kNparam / kMlpBlock + 1), dim3(kMlpBlock), 0, c.stream, ngroup, c.part2,
+                     c.loss2, c.g, c.loss);
   mcheck(hipGetLastError(), "k_mlp_reduce2");
 }
 
@@ -536,6 +586,27 @@ struct DBuf {
   template <typename T>
   T* as() const {
     return (T*)p;
+  }
+};
+
+struct PinBuf {
+  void* p = nullptr;
+  explicit PinBuf(size_t bytes) { mcheck(hipHostMalloc(&p, bytes, hipHostMallocMapped), "hipHostMalloc"); }
+  ~PinBuf() {
+    if (p) (void)hipHostFree(p);
+  }
+  PinBuf(const PinBuf&) = delete;
+  PinBuf& operator=(const PinBuf&) = delete;
+};
+
+struct EventPair {
+  hipEvent_t e[2] = {nullptr, nullptr};
+  EventPair() {
+    for (hipEvent_t& v : e) mcheck(hipEventCreateWithFlags(&v, hipEventDisableTiming), "hipEventCreate");
+  }
+  ~EventPair() {
+    for (hipEvent_t v : e)
+      if (v) (void)hipEventDestroy(v);
   }
 };
 
@@ -566,19 +637,21 @@ int pcfd_mlp_create(unsigned long long seed, pcfd_mlp** out) {
     mcheck(hipEventCreate(&c->e0), "hipEventCreate");
     mcheck(hipEventCreate(&c->e1), "hipEventCreate");
     c->scratch = pcfd::scratch_on_current_device();
-    c->grid = 256;
+    c->grid = 1024;
     const size_t P = sizeof(float) * kNparam;
     mcheck(hipMalloc((void**)&c->p, P), "hipMalloc");
     mcheck(hipMalloc((void**)&c->m, P), "hipMalloc");
     mcheck(hipMalloc((void**)&c->v, P), "hipMalloc");
     mcheck(hipMalloc((void**)&c->g, P), "hipMalloc");
     mcheck(hipMalloc((void**)&c->loss, sizeof(float)), "hipMalloc");
-    mcheck(hipMalloc((void**)&c->W1, sizeof(short) * kNh * kKin), "hipMalloc");
-    mcheck(hipMalloc((void**)&c->W2, sizeof(short) * kNh * kNh), "hipMalloc");
-    mcheck(hipMalloc((void**)&c->W3, sizeof(short) * kKout * kNh), "hipMalloc");
-    mcheck(hipMalloc((void**)&c->partial, sizeof(float) * (size_t)c->grid * kWaves * kNparam), "hipMalloc");
-    mcheck(hipMalloc((void**)&c->lossp, sizeof(float) * (size_t)c->grid * kWaves), "hipMalloc");
-    const size_t ngroup = ((size_t)c->grid * kWaves + kRedGroup - 1) / kRedGroup;
+    mcheck(hipMalloc((void**)&c->W.W1, sizeof(short) * kNh * kKin), "hipMalloc");
+    mcheck(hipMalloc((void**)&c->W.W2, sizeof(short) * kNh * kNh), "hipMalloc");
+    mcheck(hipMalloc((void**)&c->W.W3, sizeof(short) * kKout * kNh), "hipMalloc");
+    mcheck(hipMalloc((void**)&c->W.W2t, sizeof(short) * kNh * kNh), "hipMalloc");
+    mcheck(hipMalloc((void**)&c->W.W3t, sizeof(short) * kKout * kNh), "hipMalloc");
+    mcheck(hipMalloc((void**)&c->partial, sizeof(float) * (size_t)c->grid * kNparam), "hipMalloc");
+    mcheck(hipMalloc((void**)&c->lossp, sizeof(float) * (size_t)c->grid), "hipMalloc");
+    const size_t ngroup = ((size_t)c->grid + kRedGroup - 1) / kRedGroup;
     mcheck(hipMalloc((void**)&c->part2, sizeof(float) * ngroup * kNparam), "hipMalloc");
     mcheck(hipMalloc((void**)&c->loss2, sizeof(float) * ngroup), "hipMalloc");
     // Glorot-uniform weights, zero biases (host-side, reproducible)
@@ -614,7 +687,7 @@ int pcfd_mlp_destroy(pcfd_mlp* c) {
   float* fs[] = {c->p, c->m, c->v, c->g, c->loss, c->partial, c->lossp, c->part2, c->loss2};
   for (float* f : fs)
     if (f) (void)hipFree(f);
-  short* ss[] = {c->W1, c->W2, c->W3};
+  short* ss[] = {c->W.W1, c->W.W2, c->W.W3, c->W.W2t, c->W.W3t};
   for (short* s : ss)
     if (s) (void)hipFree(s);
   if (c->e0) (void)hipEventDestroy(c->e0);
@@ -732,38 +805,51 @@ int pcfd_mlp_train(pcfd_mlp* c, int n, const float* x, const float* t, int steps
       return PCFD_ERR_ARG;
     }
     DBuf dx(sizeof(float) * (size_t)n * kNin), dt(sizeof(float) * (size_t)n * kNout),
-        didx(sizeof(int) * (size_t)batch);
+        dloss(sizeof(float) * (size_t)steps);
+    // Two index lists in pinned memory, which the gradient kernel reads once,
+    // from there: while a step runs the host draws the next one's.  (With one
+    // list, a copy and a wait for each step the device sat idle while the host
+    // drew: 90 us a step of 8192 samples, 45 of them busy; 33 so.)
+    PinBuf hidx(sizeof(int) * 2 * (size_t)batch);
+    int* didx = nullptr;
+    mcheck(hipHostGetDevicePointer((void**)&didx, hidx.p, 0), "hipHostGetDevicePointer");
+    EventPair done;
+    struct Drain {  // the kernels read the lists: none is freed before they end
+      hipStream_t s;
+      ~Drain() { (void)hipStreamSynchronize(s); }
+    } drain{m.stream};
     mcheck(hipMemcpyAsync(dx.p, x, sizeof(float) * (size_t)n * kNin, hipMemcpyHostToDevice, m.stream), "copy");
     mcheck(hipMemcpyAsync(dt.p, t, sizeof(float) * (size_t)n * kNout, hipMemcpyHostToDevice, m.stream), "copy");
-    std::vector<int> hidx((size_t)batch);
-    std::vector<float> hist;
     uint64_t s = seed;
+    const uint64_t recip = ~0ull / (uint64_t)n;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     mcheck(hipEventRecord(m.e0, m.stream), "hipEventRecord");
     for (int it = 0; it < steps; ++it) {
+      const size_t at = (size_t)(it & 1) * batch;
+      int* list = (int*)hidx.p + at;
+      if (it >= 2) mcheck(hipEventSynchronize(done.e[it & 1]), "hipEventSynchronize");
       for (int k = 0; k < batch; ++k) {
         s = mix(s);
-        hidx[k] = (int)(s % (uint64_t)n);
+        // s % n by the reciprocal: the quotient is at most one too small
+        uint64_t rem = s - (uint64_t)(((unsigned __int128)s * recip) >> 64) * (uint64_t)n;
+        if (rem >= (uint64_t)n) rem -= (uint64_t)n;
+        list[k] = (int)rem;
       }
-      mcheck(hipMemcpyAsync(didx.p, hidx.data(), sizeof(int) * (size_t)batch, hipMemcpyHostToDevice, m.stream),
-             "copy");
-      grad_device(m, batch, dx.as<float>(), dt.as<float>(), didx.as<int>());
+      const int ngroup = grad_groups(m, batch, dx.as<float>(), dt.as<float>(), didx + at);
+      mcheck(hipEventRecord(done.e[it & 1], m.stream), "hipEventRecord");
       ++m.adam_t;
       // cosine decay of the step size over the run
       const float lr_t = 0.5f * lr * (1.f + std::cos(3.14159265f * (float)it / (float)std::max(1, steps)));
       const float c1 = 1.f - std::pow(b1, (float)m.adam_t), c2 = 1.f - std::pow(b2, (float)m.adam_t);
-      hipLaunchKernelGGL(k_mlp_adam, dim3((kNparam + kMlpBlock - 1) / kMlpBlock), dim3(kMlpBlock), 0, m.stream,
-                         m.p, m.m, m.v, m.g, lr_t, b1, b2, eps, c1, c2, m.W1, m.W2, m.W3);
+      hipLaunchKernelGGL(k_mlp_adam, dim3(kNparam / kAdamBlock + 1), dim3(kAdamBlock), 0, m.stream, m.p, m.m, m.v,
+                         ngroup, m.part2, m.loss2, dloss.as<float>() + it, lr_t, b1, b2, eps, c1, c2, m.W);
       mcheck(hipGetLastError(), "k_mlp_adam");
-      if (loss_history) {
-        float l = 0.f;
-        mcheck(hipMemcpyAsync(&l, m.loss, sizeof(float), hipMemcpyDeviceToHost, m.stream), "copy");
-        mcheck(hipStreamSynchronize(m.stream), "hipStreamSynchronize");
-        loss_history[it] = l / (float)((long long)batch * kNout);
-      } else {
-        // the host-side index buffer is reused: wait for the copy
-        mcheck(hipStreamSynchronize(m.stream), "hipStreamSynchronize");
-      }
+    }
+    if (loss_history && steps > 0) {
+      mcheck(hipMemcpyAsync(loss_history, dloss.p, sizeof(float) * (size_t)steps, hipMemcpyDeviceToHost, m.stream),
+             "copy");
+      mcheck(hipStreamSynchronize(m.stream), "hipStreamSynchronize");
+      for (int it = 0; it < steps; ++it) loss_history[it] /= (float)((long long)batch * kNout);
     }
     mcheck(hipEventRecord(m.e1, m.stream), "hipEventRecord");
     mcheck(hipEventSynchronize(m.e1), "hipEventSynchronize");
