@@ -719,6 +719,10 @@ __global__ void __launch_bounds__(64) k_fr_prepare(int nrow_pad, TM* __restrict_
 // is 64 consecutive rows' entry), the nine components meet in LDS, and wave
 // 0 solves the diagonal blocks.  Per component the arithmetic is the
 // reference's matrix-vector product row and subtraction, in its order.
+// A group's block entries are loaded before the barrier that its x wait at,
+// and the next group's x while the group is worked on: the slots' loads do not
+// wait for each other (22.4 -> 17.2 us a pass at 5.9k nodes in FP64, 64.3 ->
+// 55.5 at 185k in FP32).
 template <int NS, typename TM>
 __global__ void __launch_bounds__(64 * (NS + 4)) k_fr_sgs_color(int chunk0, const int* __restrict__ srow,
                                                               const int* __restrict__ swidth,
@@ -744,23 +748,38 @@ __global__ void __launch_bounds__(64 * (NS + 4)) k_fr_sgs_color(int chunk0, cons
   const TM* mb = Moff + (long long)sbase[chunk] * NE2 * kLane + (long long)(rr * NE) * kLane + lane;
   // every wave runs the chunk's w slots (the barriers need all of them);
   // a row's padding slots (j < 0) contribute nothing
+  int jn[SB];
+  TM xn[SB];
+#pragma unroll
+  for (int t = 0; t < SB; ++t) jn[t] = (i >= 0 && t < w) ? scol[cb + (long long)t * kLane] : -1;
+#pragma unroll
+  for (int t = 0; t < SB; ++t) xn[t] = jn[t] >= 0 ? x[(long long)jn[t] * NE + rr] : (TM)0;
   for (int s0 = 0; s0 < w; s0 += SB) {
     TM* xg = &xs[(s0 / SB) & 1][0][0][0];
+    TM blk[SB][NE];
     int jj[SB];
 #pragma unroll
     for (int t = 0; t < SB; ++t) {
-      jj[t] = (i >= 0 && s0 + t < w) ? scol[cb + (long long)(s0 + t) * kLane] : -1;
-      xg[(t * NE + rr) * 64 + lane] = jj[t] >= 0 ? x[(long long)jj[t] * NE + rr] : (TM)0;
+      jj[t] = jn[t];
+#pragma unroll
+      for (int c = 0; c < NE; ++c)
+        blk[t][c] = jj[t] >= 0 ? mb[((long long)(s0 + t) * NE2 + c) * kLane] : (TM)0;
     }
+#pragma unroll
+    for (int t = 0; t < SB; ++t)
+      jn[t] = (i >= 0 && s0 + SB + t < w) ? scol[cb + (long long)(s0 + SB + t) * kLane] : -1;
+#pragma unroll
+    for (int t = 0; t < SB; ++t) xg[(t * NE + rr) * 64 + lane] = xn[t];
     __syncthreads();
+#pragma unroll
+    for (int t = 0; t < SB; ++t) xn[t] = jn[t] >= 0 ? x[(long long)jn[t] * NE + rr] : (TM)0;
 #pragma unroll
     for (int t = 0; t < SB; ++t) {
       if (jj[t] >= 0) {
-        const TM* blk = mb + (long long)(s0 + t) * NE2 * kLane;
         const TM* xb = xg + t * NE * 64;
-        TM v = blk[0] * xb[lane];
+        TM v = blk[t][0] * xb[lane];
 #pragma unroll
-        for (int c = 1; c < NE; ++c) v += blk[(long long)c * kLane] * xb[c * 64 + lane];
+        for (int c = 1; c < NE; ++c) v += blk[t][c] * xb[c * 64 + lane];
         rhs -= v;
       }
     }
