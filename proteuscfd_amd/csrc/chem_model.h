@@ -25,51 +25,84 @@ struct ChemDev {
   double net[PCFD_CHEM_MAXR][PCFD_CHEM_MAXS], nu[PCFD_CHEM_MAXR];
 };
 
+// Powers come in two forms.
+//
+// LibPow calls pow for every exponent, as the reference does.  The finite-rate
+// solver keeps it: its source Jacobian differences two sources 1e-8 apart, so a
+// last bit of a power is a part in 1e8 of an entry, and of 200 solves of the
+// reacting bump from random states two answered the other form's last bits with
+// more than 2e-7 of a value in their result.
+//
+// ProductPow, for the calls that return rates, sources and Jacobians: the small
+// whole exponents that mass action is made of are products -- 1 and x are pow's
+// results, x*x is rounded once, the cube's second rounding is corrected -- and the
+// halves that Arrhenius rates use come from sqrt(T), each corrected by what its
+// roundings left out, so that all are within a hair of half a unit.  (A pow is
+// some 200 instructions; with them source and Jacobian of 400k five-species cells
+// took 1.58 ms, with products, rate constants shared by the columns and whole-line
+// stores 0.24 ms.)
+//
 // isWholeNumber (ucs/macros.h:24-30); integer exponents go through pow of
-// the promoted integer like the reference's pow(Type, Int).  The small whole
-// exponents that mass action is made of are products: 1 and x are pow's
-// results, x*x is rounded once, the cube's second rounding is corrected.  (A
-// pow is some 200 instructions; with them source and Jacobian of 400k
-// five-species cells took 1.58 ms, with products, rate constants shared by the
-// columns and whole-line stores 0.24 ms.)
-__device__ __forceinline__ double powr(double x, double e) {
-  const int up = (int)(e + 0.5), flat = (int)e;
-  if (up == flat) e = (double)flat;
-  if (e == 0.0) return 1.0;
-  if (e == 1.0) return x;
-  if (e == 2.0) return x * x;
-  if (e == -1.0) return 1.0 / x;
-  if (e == 3.0) {
-    const double x2 = x * x, r = x2 * x;
-    const double c = __builtin_fma(x2, x, __builtin_fma(x, x, -x2) * x);
-    return __builtin_isinf(x2) || __builtin_isnan(c) ? r : c;
+// the promoted integer like the reference's pow(Type, Int)
+struct LibPow {
+  static __device__ __forceinline__ double conc(double x, double e) {
+    const int up = (int)(e + 0.5), flat = (int)e;
+    return pow(x, up == flat ? (double)flat : e);
   }
-  return pow(x, e);
-}
+  static __device__ __forceinline__ double temp(double T, double n) { return pow(T, n); }
+};
 
+struct ProductPow {
+  static __device__ __forceinline__ double conc(double x, double e) {
+    const int up = (int)(e + 0.5), flat = (int)e;
+    if (up == flat) e = (double)flat;
+    if (e == 0.0) return 1.0;
+    if (e == 1.0) return x;
+    if (e == 2.0) return x * x;
+    if (e == -1.0) return 1.0 / x;
+    if (e == 3.0) {
+      const double x2 = x * x, r = x2 * x;
+      const double c = __builtin_fma(x2, x, __builtin_fma(x, x, -x2) * x);
+      return __builtin_isinf(x2) || __builtin_isnan(c) ? r : c;
+    }
+    return pow(x, e);
+  }
+  static __device__ __forceinline__ double temp(double T, double n) {
+    if (n == 0.0) return 1.0;
+    if (n == 1.0) return T;
+    if (n == -1.0) return 1.0 / T;
+    // the corrections' products must neither overflow nor vanish
+    const bool plain = T > 1.0e-100 && T < 1.0e100;
+    if (plain && (fabs(n) == 0.5 || fabs(n) == 1.5)) {
+      const double s = sqrt(T), ds = __builtin_fma(-s, s, T) * (0.5 / s);  // sqrt(T) = s + ds
+      if (n == 0.5) return s;
+      double p = s, dp = ds;  // T^|n| = p + dp
+      if (fabs(n) == 1.5) {
+        p = T * s;
+        dp = __builtin_fma(T, s, -p) + T * ds;
+        if (n == 1.5) return p + dp;
+      }
+      const double y = 1.0 / p;
+      return __builtin_fma(y, __builtin_fma(-p, y, 1.0) - dp * y, y);
+    }
+    return pow(T, n);
+  }
+};
+
+template <typename P>
 __device__ __forceinline__ double kf_of(const ChemDev& m, int r, double T) {
   const double A = m.A[r], EA = m.EA[r], n = m.n[r];
-  // pow(T, n) in the reference: whole and half exponents up to 3/2 as products
-  // and quotients of T and sqrt(T), at most three roundings
-  double Tn;
-  if (n == 0.0) Tn = 1.0;
-  else if (n == 1.0) Tn = T;
-  else if (n == -1.0) Tn = 1.0 / T;
-  else if (fabs(n) == 0.5 || fabs(n) == 1.5) {
-    Tn = sqrt(T);
-    if (fabs(n) == 1.5) Tn *= T;
-    if (n < 0.0) Tn = 1.0 / Tn;
-  } else Tn = pow(T, n);
   switch (m.type[r]) {
     case 0: return (A * exp(-EA / (kUnivR * T)));
-    case 1: return (A * Tn * exp(-EA / (kUnivR * T)));
-    case 2: return (A * Tn * exp(-EA / T));
-    case 3: return (A * Tn);
+    case 1: return (A * P::temp(T, n) * exp(-EA / (kUnivR * T)));
+    case 2: return (A * P::temp(T, n) * exp(-EA / T));
+    case 3: return (A * P::temp(T, n));
   }
   return -999.0;
 }
 
 // GetEquilibriumReactionRate (ucs/reaction.tcc:628-679); lnT = log(T)
+template <typename P>
 __device__ __forceinline__ double kc_of(const ChemDev& m, int r, double T, double lnT) {
   double d[7] = {0, 0, 0, 0, 0, 0, 0};
   const bool high = T > 1000.0;  // GetThermoCoeff: pinned ranges pick the same set
@@ -84,7 +117,7 @@ __device__ __forceinline__ double kc_of(const ChemDev& m, int r, double T, doubl
       exp(d[0] * (lnT - 1.0) + T * (d[1] / 2.0 + T * (d[2] / 6.0 + T * (d[3] / 12.0 + d[4] / 20.0 * T))) -
           d[5] / T + d[6]);
   double Kc = Kp;
-  if (!(fabs(m.nu[r]) < 1.0e-15)) Kc *= powr(101325.0 / (kUnivR * T), m.nu[r]);
+  if (!(fabs(m.nu[r]) < 1.0e-15)) Kc *= P::conc(101325.0 / (kUnivR * T), m.nu[r]);
   return Kc;
 }
 
@@ -107,7 +140,7 @@ __device__ __forceinline__ double pick(const double* v, int k) {
 }
 
 // GetMassProductionRates for one state: rhoi (kg/m^3), T (K) -> wdot (kg/m^3/s)
-template <int NS>
+template <int NS, typename P = ProductPow>
 __device__ inline void wdot_of(const ChemDev& m, const double* rhoi, double T, double* wdot) {
   constexpr int MS = NS > 0 ? NS : PCFD_CHEM_MAXS;
   const int ns = nspecies_of<NS>(m);
@@ -120,13 +153,13 @@ __device__ inline void wdot_of(const ChemDev& m, const double* rhoi, double T, d
   }
   const double lnT = log(T);
   for (int r = 0; r < m.nr; ++r) {
-    const double Kf = kf_of(m, r, T);
-    const double Kb = Kf / kc_of(m, r, T, lnT);
+    const double Kf = kf_of<P>(m, r, T);
+    const double Kb = Kf / kc_of<P>(m, r, T, lnT);
     double pf = 1.0, pd = 1.0;
     for (int k = 0; k < m.nloc[r]; ++k) {
       const double x = pick<NS>(X, m.loc[r][k]);
-      pf *= powr(x, m.nup[r][k]);
-      pd *= powr(x, m.nupp[r][k]);
+      pf *= P::conc(x, m.nup[r][k]);
+      pd *= P::conc(x, m.nupp[r][k]);
     }
     double Mc = 1.0;
     if (m.tb[r]) {
@@ -152,7 +185,7 @@ __device__ inline void wdot_of(const ChemDev& m, const double* rhoi, double T, d
 }
 
 // SourceTerm (ucs/compressibleFR.tcc:1276-1312) on the FR state
-template <int NS>
+template <int NS, typename P = ProductPow>
 __device__ inline void source_of(const ChemDev& m, const double* Q, double vol, double* src) {
   constexpr int MS = NS > 0 ? NS : PCFD_CHEM_MAXS;
   const int ns = nspecies_of<NS>(m);
@@ -163,7 +196,7 @@ __device__ inline void source_of(const ChemDev& m, const double* Q, double vol, 
     if (i >= ns) break;
     rhoi[i] = Q[i] * m.ref_density;
   }
-  wdot_of<NS>(m, rhoi, T, w);
+  wdot_of<NS, P>(m, rhoi, T, w);
 #pragma unroll
   for (int i = 0; i < MS; ++i) {
     if (i >= ns) break;
@@ -179,7 +212,7 @@ __device__ inline void source_of(const ChemDev& m, const double* Q, double vol, 
 // reaction and shared; every copy's products and sums, in their order, are
 // wdot_of's, so w[(1 + c) * ns + i] equals wdot_of of copy c bit for bit
 // and w[i] that of the state.  w [(ns + 1) * ns].
-template <int NS>
+template <int NS, typename P = ProductPow>
 __device__ inline void wdot_rho_columns(const ChemDev& m, const double* rhoi, const double* rhop, double T,
                                         double* w) {
   constexpr int MS = NS > 0 ? NS : PCFD_CHEM_MAXS;
@@ -198,8 +231,8 @@ __device__ inline void wdot_rho_columns(const ChemDev& m, const double* rhoi, co
   }
   const double lnT = log(T);
   for (int r = 0; r < m.nr; ++r) {
-    const double Kf = kf_of(m, r, T);
-    const double Kb = Kf / kc_of(m, r, T, lnT);
+    const double Kf = kf_of<P>(m, r, T);
+    const double Kb = Kf / kc_of<P>(m, r, T, lnT);
     // copy s has species s - 1 raised (0: the state itself)
     double pf[MS + 1], pd[MS + 1], Mc[MS + 1];
 #pragma unroll
@@ -219,7 +252,7 @@ __device__ inline void wdot_rho_columns(const ChemDev& m, const double* rhoi, co
       const int l = m.loc[r][k];
       const double x = pick<NS>(X, l), xp = pick<NS>(Xp, l);
       const double eu = m.nup[r][k], ed = m.nupp[r][k];
-      const double fu = powr(x, eu), fup = powr(xp, eu), fd = powr(x, ed), fdp = powr(xp, ed);
+      const double fu = P::conc(x, eu), fup = P::conc(xp, eu), fd = P::conc(x, ed), fdp = P::conc(xp, ed);
       const double w1 = m.eff[r][k] - 1.0;
 #pragma unroll
       for (int s = 0; s <= MS; ++s) {
@@ -251,7 +284,7 @@ __device__ inline void wdot_rho_columns(const ChemDev& m, const double* rhoi, co
 // (the species columns of the forward-difference source Jacobian):
 // src[i] is the state's, src[(1 + c) * ns + i] copy c's, each bit for bit
 // what source_of gives.  src [(ns + 1) * ns].
-template <int NS>
+template <int NS, typename P = ProductPow>
 __device__ inline void source_rho_columns(const ChemDev& m, const double* Q, double h, double vol, double* src) {
   constexpr int MS = NS > 0 ? NS : PCFD_CHEM_MAXS;
   const int ns = nspecies_of<NS>(m);
@@ -263,7 +296,7 @@ __device__ inline void source_rho_columns(const ChemDev& m, const double* Q, dou
     rhoi[i] = Q[i] * m.ref_density;
     rhop[i] = (Q[i] + h) * m.ref_density;
   }
-  wdot_rho_columns<NS>(m, rhoi, rhop, T, src);
+  wdot_rho_columns<NS, P>(m, rhoi, rhop, T, src);
 #pragma unroll
   for (int k = 0; k < (MS + 1) * MS; ++k) {
     if (k >= (ns + 1) * ns) break;

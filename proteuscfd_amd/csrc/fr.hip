@@ -286,7 +286,7 @@ __global__ void __launch_bounds__(kFB) k_fr_residual(const Model* __restrict__ m
       double Q[NE];
 #pragma unroll
       for (int k = 0; k < NE; ++k) Q[k] = q[(long long)i * NE + k];
-      source_of<NS>(*cm, Q, vol[i], S);
+      source_of<NS, LibPow>(*cm, Q, vol[i], S);
     } else {
 #pragma unroll
       for (int k = 0; k < NS; ++k) S[k] = 0.0;
@@ -565,7 +565,7 @@ __global__ void __launch_bounds__(kFB) k_fr_node_terms(const Model* __restrict__
   const double h = kFrH;
   // the state and its species columns (Q[c] + h) share the T-only rate
   // constants: the same values as NS + 1 separate source evaluations
-  source_rho_columns<NS>(*cm, Q, h, v, sc);
+  source_rho_columns<NS, LibPow>(*cm, Q, h, v, sc);
   const double* s0 = sc;
 #pragma unroll
   for (int c = 0; c < NS; ++c)
@@ -573,7 +573,7 @@ __global__ void __launch_bounds__(kFB) k_fr_node_terms(const Model* __restrict__
     for (int j = 0; j < NS; ++j) o[(long long)(NE2 + j * (NS + 1) + c) * kLane] = (sc[(1 + c) * NS + j] - s0[j]) / h;
   // the T column
   Q[NS + 3] += h;
-  source_of<NS>(*cm, Q, v, s1);
+  source_of<NS, LibPow>(*cm, Q, v, s1);
 #pragma unroll
   for (int j = 0; j < NS; ++j) o[(long long)(NE2 + j * (NS + 1) + NS) * kLane] = (s1[j] - s0[j]) / h;
 }
