@@ -111,7 +111,7 @@ struct Dev {
 
 constexpr size_t kPin = 1 << 18;  // 2 MiB
 constexpr int kMinParts = 1024;   // at most that many partial minima
-constexpr size_t kPinAll = kPin + 8 + kMinParts;
+constexpr size_t kPinHead = 8 + kMinParts;
 
 struct Ctx {
   int device = 0;
@@ -119,9 +119,11 @@ struct Ctx {
   hipStream_t stream2 = nullptr;  // Jacobian rows, overlapped with the edge passes (default priority)
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   hipEvent_t ev_norms = nullptr;  // the residual norms are in pin
-  // pinned host memory that kernels write to and read from: kPin values of a
-  // small caller's array, then the norms' six sums, then partial minima
+  // pinned host memory that kernels write to and read from: the norms' six sums,
+  // partial minima from 8, a small caller's array of up to pin_n values from
+  // kPinHead (kPin of them, or a mesh's widest array where that is smaller)
   double *pin = nullptr, *pin_dev = nullptr;
+  size_t pin_n = 0;
   bool overlap = true;            // PCFD_JACOBIAN_STREAM=0 turns the overlap off
   bool jac_pending = false;
   std::string err;

@@ -207,13 +207,14 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     PCFD_HIP(hipEventCreateWithFlags(&c.ev_fork, hipEventDisableTiming));
     PCFD_HIP(hipEventCreateWithFlags(&c.ev_join, hipEventDisableTiming));
     PCFD_HIP(hipEventCreateWithFlags(&c.ev_norms, hipEventDisableTiming));
-    PCFD_HIP(hipHostMalloc((void**)&c.pin, sizeof(double) * kPinAll, hipHostMallocMapped));
-    PCFD_HIP(hipHostGetDevicePointer((void**)&c.pin_dev, c.pin, 0));
     if (const char* e = std::getenv("PCFD_JACOBIAN_STREAM")) c.overlap = std::strcmp(e, "0") != 0;
     c.nnode = nn;
     c.nbnode = nb;
     c.nedge = ne;
     c.ntot = nn + nb;
+    c.pin_n = std::min(kPin, 27 * (size_t)c.ntot);
+    PCFD_HIP(hipHostMalloc((void**)&c.pin, sizeof(double) * (kPinHead + c.pin_n), hipHostMallocMapped));
+    PCFD_HIP(hipHostGetDevicePointer((void**)&c.pin_dev, c.pin, 0));
     c.ntag = nt;
     c.nnz = 2 * ne;
     // ---- node adjacency in edge order, with the edge id: a node's slots

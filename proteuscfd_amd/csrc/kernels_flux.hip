@@ -864,14 +864,14 @@ void launch_residual(Ctx& c, int ho) {
 // residGlobal = sqrt(sum b^2)/(nnode*neqn), per-equation sqrt(sum b_k^2)/nnode
 // (ParallelL2Norm / StridedParallelL2Norm, ucs/parallel.h:120-182)
 void launch_norms(Ctx& c) {
-  hipLaunchKernelGGL(k_reduce6, dim3(6), dim3(kBlock), 0, c.stream, c.nred, c.d.red, c.pin_dev + kPin);
+  hipLaunchKernelGGL(k_reduce6, dim3(6), dim3(kBlock), 0, c.stream, c.nred, c.d.red, c.pin_dev);
   PCFD_HIP(hipGetLastError());
   PCFD_HIP(hipEventRecord(c.ev_norms, c.stream));
 }
 
 void wait_norms(Ctx& c, double* host6) {
   PCFD_HIP(hipEventSynchronize(c.ev_norms));
-  const double* s = c.pin + kPin;
+  const double* s = c.pin;
   host6[0] = std::sqrt(s[0]) / (double)((long long)c.nnode * 5);
   for (int k = 0; k < 5; ++k) host6[1 + k] = std::sqrt(s[1 + k]) / (double)c.nnode;
 }
@@ -994,10 +994,10 @@ void launch_timestep(Ctx& c, double cfl) {
 
 double launch_dtmin(Ctx& c) {
   const int nb = std::min(nblk(c.nnode), kMinParts);
-  hipLaunchKernelGGL(k_min_partial, dim3(nb), dim3(kBlock), 0, c.stream, c.nnode, c.d.dt, c.pin_dev + kPin + 8);
+  hipLaunchKernelGGL(k_min_partial, dim3(nb), dim3(kBlock), 0, c.stream, c.nnode, c.d.dt, c.pin_dev + 8);
   PCFD_HIP(hipGetLastError());
   PCFD_HIP(hipStreamSynchronize(c.stream));
-  const double* h = c.pin + kPin + 8;
+  const double* h = c.pin + 8;
   double m = h[0];
   for (int k = 0; k < nb; ++k) m = h[k] < m ? h[k] : m;
   return m;

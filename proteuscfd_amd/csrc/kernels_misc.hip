@@ -241,20 +241,20 @@ static double* aos_space(Ctx& c, size_t n) {
   return c.d.aos;
 }
 
-// Where a kernel leaves or finds a caller's array of n values: up to kPin in
+// Where a kernel leaves or finds a caller's array of n values: up to pin_n in
 // pinned host memory, which the host copies to or from itself, more in device
 // memory.  A copy engine's start costs more than the kernel's own trip over the
 // bus: 37k values went up in 137 and came down in 154 us through device memory,
 // in 26 and 30 through pinned; at 220k both took 80-100 and 130-140.
-static double* space_of(Ctx& c, size_t n) { return n <= kPin ? c.pin_dev : aos_space(c, n); }
+static double* space_of(Ctx& c, size_t n) { return n <= c.pin_n ? c.pin_dev + kPinHead : aos_space(c, n); }
 
 // the n rows of ncomp values a kernel has left there into the caller's rows of
 // `stride` values, the stream's work done on return
 static void rows_to_host(Ctx& c, size_t n, int ncomp, double* host, int stride) {
   const size_t m = n * ncomp;
-  const double* src = c.pin;
+  const double* src = c.pin + kPinHead;
   std::vector<double> s;
-  if (m <= kPin) {
+  if (m <= c.pin_n) {
     PCFD_HIP(hipStreamSynchronize(c.stream));
     if (stride == ncomp) std::copy(src, src + m, host);
   } else {
@@ -273,7 +273,7 @@ static void rows_to_host(Ctx& c, size_t n, int ncomp, double* host, int stride) 
 
 void soa_to_host(Ctx& c, const double* soa, int ld, int n, int ncomp, double* host) {
   const size_t m = (size_t)n * ncomp;
-  if (ncomp == 1 && m > kPin) {
+  if (ncomp == 1 && m > c.pin_n) {
     PCFD_HIP(hipMemcpyAsync(host, soa, sizeof(double) * m, hipMemcpyDeviceToHost, c.stream));
     PCFD_HIP(hipStreamSynchronize(c.stream));
     return;
@@ -300,9 +300,9 @@ void soa_from_host(Ctx& c, double* soa, int ld, int n, int ncomp, const double* 
   // may end with them
   const size_t m = (size_t)(n - 1) * stride + ncomp;
   double* aos = space_of(c, m);
-  if (m <= kPin) {
+  if (m <= c.pin_n) {
     // nothing on the stream still reads the pinned rows: every use waits for its own
-    std::copy(host, host + m, c.pin);
+    std::copy(host, host + m, c.pin + kPinHead);
   } else {
     PCFD_HIP(hipMemcpyAsync(aos, host, sizeof(double) * m, hipMemcpyHostToDevice, c.stream));
   }
