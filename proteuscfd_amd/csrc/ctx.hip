@@ -8,6 +8,7 @@
 
 #include "../../include/pcfd_mesh.h"
 #include "common.h"
+#include "fill.h"
 
 using namespace pcfd;
 
@@ -35,8 +36,9 @@ void dput(Ctx& c, T** p, const std::vector<T>& h) {
 // zero-filled: the padding rows of a row-order vector stay zero
 template <typename T>
 void dzero(Ctx& c, T** p, size_t n) {
+  static_assert(sizeof(T) % 4 == 0, "launch_zero writes words");
   dalloc(c, p, n);
-  PCFD_HIP(hipMemset(*p, 0, std::max<size_t>(n, 1) * sizeof(T)));
+  launch_zero(c.stream, *p, n * (sizeof(T) / 4));
 }
 
 template <typename T>
@@ -438,7 +440,7 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     dput(c, &d.twall, twall);
     dput(c, &d.spos, spos);
     dalloc(c, &d.q, 5 * (size_t)c.ntot);
-    dalloc(c, &d.grad, 27 * (size_t)nn);
+    dzero(c, &d.grad, 27 * (size_t)nn);
     dalloc(c, &d.lim, 5 * (size_t)nn);
     dalloc(c, &d.lim2, 5 * (size_t)nn);
     {
@@ -461,7 +463,6 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     dalloc(c, &d.red, 6 * (size_t)std::max(nblk(4LL * nn), 1024));
     dalloc(c, &d.red_out, 8);
     dalloc(c, &d.icount, 4);
-    PCFD_HIP(hipMemset(d.grad, 0, 27 * sizeof(double) * (size_t)nn));
     launch_lsq_moments(c);
     PCFD_HIP(hipStreamSynchronize(c.stream));
   } catch (const std::exception& e) {

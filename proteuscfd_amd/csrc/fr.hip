@@ -35,6 +35,7 @@
 #include "../../include/pcfd_fr.h"
 #include "../../include/pcfd_mesh.h"
 #include "chem_model.h"
+#include "fill.h"
 #include "fr_physics.h"
 
 namespace pcfd {
@@ -1466,7 +1467,7 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
     dalloc(*f, &f->ediag, 2 * (size_t)ne * NE2);
     dalloc(*f, &f->nterm, (size_t)f->nrow_pad * (NE2 + ns * (ns + 1)));
     dalloc(*f, &f->jst, (size_t)nn * (NE + 1));
-    hcheck(hipMemset(f->q, 0, sizeof(double) * (size_t)f->ntot * NE), "hipMemset");
+    launch_zero(f->stream, f->q, 2 * (size_t)f->ntot * NE);
   } catch (const std::exception& e) {
     g_fr_create_err = e.what();
     free_all(*f);

@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "common.h"
+#include "fill.h"
 #include "physics.h"
 #include "scan.h"
 
@@ -67,6 +68,18 @@ __global__ void __launch_bounds__(kBlock) k_explicit(int nnode, int ntot, double
 }
 
 __global__ void k_zero_int(int* p) { *p = 0; }
+
+__global__ void __launch_bounds__(kBlock) k_zero_words(size_t n, unsigned* __restrict__ p) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
+void launch_zero(hipStream_t stream, void* p, size_t n) {
+  if (n == 0) return;
+  hipLaunchKernelGGL(k_zero_words, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream, n,
+                     (unsigned*)p);
+  PCFD_HIP(hipGetLastError());
+}
 
 // One stage of the four-stage Runge-Kutta extension: Q = Q0 + a dt/vol b
 // through ApplyDQ; a row whose correction is NaN/Inf keeps Q0 (counted).

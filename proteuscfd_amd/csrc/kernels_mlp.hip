@@ -28,6 +28,7 @@
 
 #include "../../include/pcfd_chem.h"
 #include "chem_model.h"
+#include "fill.h"
 #include "scan.h"
 
 namespace pcfd {
@@ -669,8 +670,8 @@ int pcfd_mlp_create(unsigned long long seed, pcfd_mlp** out) {
     for (int o = 0; o < kNout; ++o)
       for (int k = 0; k < kNh; ++k) h[oW3 + o * kNh + k] = uni(a3);
     mcheck(hipMemcpy(c->p, h.data(), P, hipMemcpyHostToDevice), "hipMemcpy");
-    mcheck(hipMemset(c->m, 0, P), "hipMemset");
-    mcheck(hipMemset(c->v, 0, P), "hipMemset");
+    launch_zero(c->stream, c->m, kNparam);
+    launch_zero(c->stream, c->v, kNparam);
     refresh_bf16(*c);
     mcheck(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
   } catch (const std::exception& e) {
