@@ -53,7 +53,10 @@ struct Dev {
   int* he_tag = nullptr;    // nbnode
   int* he_node = nullptr;   // nbnode: node i of each half-edge, in he_id's order; ~i where a half-edge resets it
   int4* he_desc = nullptr;  // nbnode, in he_id's order: half-edge id, face tag, BC type, wall-normal neighbour or -1
-  int* rst = nullptr;       // nrst: the boundary nodes that a half-edge resets (index into bnd_nodes)
+  int4* rst = nullptr;      // runs of half-edges of the nodes that a half-edge resets, by level: node, first and
+                            // past-the-last list position, 1 where the node's list begins
+  int* he_src = nullptr;    // nbnode: the half-edge that leaves the wall-normal neighbour in the state this one
+                            // reads (list position), or -1: as it stands in q
   double* seen = nullptr;   // 5 x nbnode: the node state each half-edge of such a node sees
   double* he_a = nullptr;   // 4 x nbnode
   int* bnd_nodes = nullptr; // nodes with >= 1 half-edge
@@ -130,7 +133,7 @@ struct Ctx {
   int nnode = 0, nbnode = 0, nedge = 0, ntot = 0, ntag = 0, nnz = 0, nbnd = 0;
   int nchunk_g = 0, nchunk_s = 0, nrow_pad = 0;
   long long nslot_g = 0, nslot_s = 0;
-  int nrst = 0;           // boundary nodes that a hard-set half-edge resets
+  std::vector<int> rst_level;  // [levels+1] ranges of Dev::rst; empty where no half-edge resets its node
   int max_swidth = 0;     // slots of the widest SELL row
   long long nblocks = 0;  // nnode + 2*nedge (reference count)
   int ncolor = 0;

@@ -52,7 +52,7 @@ void free_all(Ctx& c) {
   dfree(d.xyz); dfree(d.vol); dfree(d.vol23); dfree(d.sw); dfree(d.gwidth); dfree(d.gbase); dfree(d.gcol); dfree(d.gnrm); dfree(d.qrk); dfree(d.aos);
   if (c.pin) (void)hipHostFree(c.pin);
   c.pin = c.pin_dev = nullptr;
-  dfree(d.he_ptr); dfree(d.he_id); dfree(d.he_tag); dfree(d.he_node); dfree(d.seen); dfree(d.he_desc); dfree(d.rst); dfree(d.he_a); dfree(d.bnd_nodes); dfree(d.bidx);
+  dfree(d.he_ptr); dfree(d.he_id); dfree(d.he_tag); dfree(d.he_node); dfree(d.seen); dfree(d.he_desc); dfree(d.rst); dfree(d.he_src); dfree(d.he_a); dfree(d.bnd_nodes); dfree(d.bidx);
   dfree(d.jdb); dfree(d.jhe); dfree(d.jcol); dfree(d.jqb); dfree(d.bc_type); dfree(d.twall); dfree(d.spos);
   dfree(d.qref); dfree(d.q); dfree(d.grad); dfree(d.lim); dfree(d.lim2); dfree(d.edges); dfree(d.clip_flag); dfree(d.clip_cnt);
   dfree(d.clip_off); dfree(d.clip_list); dfree(d.b); dfree(d.dt);
@@ -91,6 +91,56 @@ void fetch(std::vector<double>& h, const T* src, size_t n) {
   PCFD_HIP(hipMemcpy(t.data(), src, n * sizeof(T), hipMemcpyDeviceToHost));
   h.resize(n);
   for (size_t k = 0; k < n; ++k) h[k] = (double)t[k];
+}
+
+// The walk through the half-edges of the nodes that a half-edge resets
+// (he_node < 0), cut into runs that can go side by side: a node's half-edges
+// keep their order, and one that reads a wall-normal neighbour which earlier
+// half-edges have reset goes a level after the run of the last of them.
+// he_src: list position of that half-edge, -1 where there is none; rst: the runs
+// by level, level[l] .. level[l+1].
+void plan_resets(const pcfd_mesh_desc* m, const std::vector<int>& he_ptr, const std::vector<int>& he_node,
+                 const std::vector<int>& he_nrm, const std::vector<double>& twall, std::vector<int>& he_src,
+                 std::vector<int4>& rst, std::vector<int>& level) {
+  struct Node {
+    int p = 0, run = -1;
+    bool reset = false;
+  };
+  std::vector<Node> nodes(m->nnode);
+  std::vector<int4> runs;
+  std::vector<int> lev;
+  he_src.assign(m->nbnode, -1);
+  int nlev = 0;
+  for (int h = 0; h < m->nbnode; ++h) {
+    const int i = m->bedges[2 * h], tag = m->bfactag[h], type = m->bc_type[tag], nn = he_nrm[h];
+    if (he_node[he_ptr[i]] >= 0) continue;
+    Node& s = nodes[i];
+    const int p = he_ptr[i] + s.p++;
+    int at = 0;
+    if (type == 4 /* noSlip */ && twall[tag] < 0.0 && nn >= 0 && nodes[nn].reset) {
+      he_src[p] = he_ptr[nn] + nodes[nn].p - 1;
+      at = lev[nodes[nn].run] + 1;
+    }
+    if (s.run < 0 || lev[s.run] < at) {
+      s.run = (int)runs.size();
+      runs.push_back(int4{i, p, p, p == he_ptr[i] ? 1 : 0});
+      lev.push_back(at);
+      nlev = std::max(nlev, at + 1);
+    }
+    runs[s.run].z = p + 1;
+    s.reset |= type == 1 /* dirichlet */ || type == 7 /* sonicInflow */ || type == 4;
+  }
+  rst.clear();
+  level.clear();
+  if (runs.empty()) return;
+  level.push_back(0);
+  for (int l = 0; l < nlev; ++l) {
+    for (size_t k = 0; k < runs.size(); ++k)
+      if (lev[k] == l) rst.push_back(runs[k]);
+    // neighbouring threads take neighbouring nodes
+    std::sort(rst.begin() + level.back(), rst.end(), [](const int4& a, const int4& b) { return a.y < b.y; });
+    level.push_back((int)rst.size());
+  }
 }
 
 int need_params(Ctx& c) {
@@ -151,7 +201,7 @@ void sub_end(Ctx& c, int k) {
 void ensure_matrix_alloc(Ctx& c) { ensure_matrix(c); }
 void ensure_overlap_buffers(Ctx& c) {
   if (!c.d.dt_next) dalloc(c, &c.d.dt_next, (size_t)c.nnode);
-  if (c.nrst > 0 && !c.d.qjac) dalloc(c, &c.d.qjac, 5 * (size_t)c.ntot);
+  if (!c.rst_level.empty() && !c.d.qjac) dalloc(c, &c.d.qjac, 5 * (size_t)c.ntot);
 }
 }  // namespace pcfd
 
@@ -285,7 +335,7 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
       for (int h = 0; h < nb; ++h) he_id[hfill[m->bedges[2 * h]]++] = h;
     }
     // boundary nodes; hard-set BC types reset the state of their node
-    std::vector<int> bnd, rst, bidx(nn, -1), he_node(nb);
+    std::vector<int> bnd, bidx(nn, -1), he_node(nb);
     for (int i = 0; i < nn; ++i)
       if (he_ptr[i + 1] > he_ptr[i]) {
         bool resets = false;
@@ -294,12 +344,10 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
           resets |= ty == 1 /* dirichlet */ || ty == 7 /* sonicInflow */ || ty == 4 /* noSlip */;
         }
         for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) he_node[p] = resets ? ~i : i;
-        if (resets) rst.push_back((int)bnd.size());
         bidx[i] = (int)bnd.size();
         bnd.push_back(i);
       }
     c.nbnd = (int)bnd.size();
-    c.nrst = (int)rst.size();
     std::vector<int> he_tag(m->bfactag, m->bfactag + nb);
     std::vector<double> he_a(4 * (size_t)nb);
     for (int h = 0; h < nb; ++h)
@@ -428,8 +476,14 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
       }
       dput(c, &d.he_desc, desc);
     }
-    dput(c, &d.rst, rst);
-    if (c.nrst > 0) dalloc(c, &d.seen, 5 * (size_t)nb);
+    {
+      std::vector<int> he_src;
+      std::vector<int4> rst;
+      plan_resets(m, he_ptr, he_node, he_nrm, twall, he_src, rst, c.rst_level);
+      dput(c, &d.he_src, he_src);
+      dput(c, &d.rst, rst);
+      if (!rst.empty()) dalloc(c, &d.seen, 5 * (size_t)nb);
+    }
     dput(c, &d.he_a, he_a);
     dput(c, &d.bnd_nodes, bnd);
     dput(c, &d.bidx, bidx);

@@ -69,19 +69,21 @@ void launch_lsq_moments(Ctx& c) {
 // on the 36k-node plate, 29 us on the 5.7k-node wedge; now 41, 28 + 11 and 7 + 8
 // us, beside the Jacobian rows in the first two.)
 //
-// JAC: the Jacobian's re-evaluation, which keeps the interior states for its
-// rows to read; the reset states go to Qb, and q's interior part is committed
-// later.
-template <bool JAC>
-__global__ void __launch_bounds__(kBndBlock) k_bnd_resets(BndArgs A, double* __restrict__ Qb) {
+// An adiabatic wall reads the state its wall-normal neighbour has at that point
+// of the walk, and the neighbour may itself be reset: by half-edges that come
+// before (the state they leave is `seen` at he_src) or after (q holds it, which
+// this kernel does not write).  Half-edges that read another node's reset are
+// walked in a later launch than that reset (`seg`, by level; meshes without such
+// neighbours have one).
+__global__ void __launch_bounds__(kBndBlock) k_bnd_resets(BndArgs A, const int4* __restrict__ seg, int nseg) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= A.nrst) return;
-  const int bt = A.rst[t], i = A.bnd_nodes[bt];
-  double QL[5], Q0[5];
+  if (t >= nseg) return;
+  const int4 sg = seg[t];
+  const int i = sg.x, p1 = sg.z;
+  double QL[5];
 #pragma unroll
-  for (int k = 0; k < 5; ++k) Q0[k] = QL[k] = A.q[k * A.ntot + i];
-  const int p1 = A.he_ptr[i + 1];
-  for (int p0 = A.he_ptr[i]; p0 < p1; p0 += 4) {
+  for (int k = 0; k < 5; ++k) QL[k] = sg.w ? A.q[k * A.ntot + i] : A.seen[k * A.nbnode + sg.y - 1];
+  for (int p0 = sg.y; p0 < p1; p0 += 4) {
     // four descriptors at a time, so that their loads overlap
     int4 d[4];
 #pragma unroll
@@ -92,17 +94,12 @@ __global__ void __launch_bounds__(kBndBlock) k_bnd_resets(BndArgs A, double* __r
       if (p >= p1) break;
       const int tag = d[u].y, type = d[u].z, nn = d[u].w, ph = A.nnode + d[u].x;
       if (type == BC_NOSLIP) {
-        // hard-set wall node (adiabatic walls read the wall-normal neighbour
-        // as it stands before this update)
         const double tw = A.twall[tag];
         if (!(tw < 0.0 && nn < 0)) {
           double nQ[5] = {0, 0, 0, 0, 0}, QR[5];
 #pragma unroll
           for (int k = 0; k < 5; ++k) QR[k] = A.q[k * A.ntot + ph];
-          if (tw < 0.0) {
-#pragma unroll
-            for (int k = 0; k < 5; ++k) nQ[k] = A.q[k * A.ntot + nn];
-          }
+          if (tw < 0.0) wall_normal_state(A, p, nn, nQ);
           noslip_state(QL, QR, tw, nQ, A.gamma);
 #pragma unroll
           for (int k = 0; k < 5; ++k) A.q[k * A.ntot + ph] = QR[k];
@@ -118,21 +115,22 @@ __global__ void __launch_bounds__(kBndBlock) k_bnd_resets(BndArgs A, double* __r
       for (int k = 0; k < 5; ++k) A.seen[k * A.nbnode + p] = QL[k];
     }
   }
-#pragma unroll
-  for (int k = 0; k < 5; ++k) {
-    if (JAC) Qb[(long long)bt * 5 + k] = QL[k];
-    else if (QL[k] != Q0[k]) A.q[k * A.ntot + i] = QL[k];
-  }
 }
 
 __global__ void __launch_bounds__(kBndBlock) k_update_bcs(BndArgs A) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= A.nbnode) return;
+  const int node = A.he_node[p];
+  double QL[5], QR[5], Qr[5];
+  bnd_seen(A, p, QL);
+  if (node < 0 && (p + 1 == A.nbnode || A.he_node[p + 1] != node)) {
+    // the node's last half-edge: its walk is over (no thread here reads q there)
+#pragma unroll
+    for (int k = 0; k < 5; ++k) A.q[k * A.ntot + ~node] = QL[k];
+  }
   const int4 d = A.he_desc[p];
   const int h = d.x, tag = d.y, type = d.z, ph = A.nnode + h;
   if (type == BC_NOSLIP || is_dirichlet(type)) return;  // set by k_bnd_resets
-  double QL[5], QR[5], Qr[5];
-  bnd_seen(A, p, QL);
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
     QR[k] = A.q[k * A.ntot + ph];
@@ -146,20 +144,21 @@ __global__ void __launch_bounds__(kBndBlock) k_update_bcs(BndArgs A) {
 }
 
 BndArgs bnd_args(Ctx& c) {
-  return BndArgs{c.nbnd, c.nnode, c.ntot, c.ntag, c.nbnode, c.nrst, c.d.bnd_nodes, c.d.rst, c.d.he_ptr,
-                 c.d.he_node, c.d.he_desc, c.d.he_a, c.d.qref, c.d.twall, c.prm.gamma, c.d.q, c.d.seen};
+  return BndArgs{c.nbnd, c.nnode, c.ntot, c.ntag, c.nbnode, c.d.bnd_nodes, c.d.he_ptr, c.d.he_node, c.d.he_src,
+                 c.d.he_desc, c.d.he_a, c.d.qref, c.d.twall, c.prm.gamma, c.d.q, c.d.seen};
 }
 
-void launch_bnd_resets(Ctx& c, hipStream_t s, double* Qb) {
-  if (c.nrst == 0) return;
-  hipLaunchKernelGGL(Qb ? k_bnd_resets<true> : k_bnd_resets<false>, dim3(nblk(c.nrst, kBndBlock)), dim3(kBndBlock), 0,
-                     s, bnd_args(c), Qb);
-  PCFD_HIP(hipGetLastError());
+void launch_bnd_resets(Ctx& c, hipStream_t s) {
+  for (size_t l = 0; l + 1 < c.rst_level.size(); ++l) {
+    const int s0 = c.rst_level[l], n = c.rst_level[l + 1] - s0;
+    hipLaunchKernelGGL(k_bnd_resets, dim3(nblk(n, kBndBlock)), dim3(kBndBlock), 0, s, bnd_args(c), c.d.rst + s0, n);
+    PCFD_HIP(hipGetLastError());
+  }
 }
 
 void launch_update_bcs(Ctx& c) {
   if (c.nbnd == 0) return;
-  launch_bnd_resets(c, c.stream, nullptr);
+  launch_bnd_resets(c, c.stream);
   hipLaunchKernelGGL(k_update_bcs, dim3(nblk(c.nbnode, kBndBlock)), dim3(kBndBlock), 0, c.stream, bnd_args(c));
   PCFD_HIP(hipGetLastError());
 }

@@ -142,10 +142,7 @@ __global__ void __launch_bounds__(kBndBlock) k_jac_bnd_cols(BndArgs B, int sym2d
       const int nn = d.w;
       live = !(tw < 0.0 && nn < 0);
       double nQ[5] = {0, 0, 0, 0, 0};
-      if (tw < 0.0 && live) {
-#pragma unroll
-        for (int k = 0; k < 5; ++k) nQ[k] = B.q[k * B.ntot + nn];
-      }
+      if (tw < 0.0 && live) wall_normal_state(B, p, nn, nQ);
       noslip_state(QPL, QPR, tw, nQ, B.gamma);
     } else {
       double Qr[5];
@@ -164,16 +161,17 @@ __global__ void __launch_bounds__(kBndBlock) k_jac_bnd_cols(BndArgs B, int sym2d
   for (int rr = 0; rr < 5; ++rr) col[t * 5 + rr] = Dc[rr];
 }
 
-// ... and the states of the nodes that no half-edge resets, as they stand, to Qb
+// ... and the nodes' states after the re-evaluation to Qb
 __global__ void __launch_bounds__(kBlock) k_jac_bnd_sum(BndArgs B, const double* __restrict__ col,
                                                        double* __restrict__ Db, double* __restrict__ Qb) {
   const long long t25 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t25 >= 25LL * B.nbnd) return;
   const int t = (int)(t25 / 25), k = (int)(t25 % 25);  // k = column * 5 + row, as col stores them
   const int i = B.bnd_nodes[t];
-  if (k < 5 && B.he_node[B.he_ptr[i]] >= 0) Qb[5LL * t + k] = B.q[k * B.ntot + i];
+  const int p1 = B.he_ptr[i + 1];
+  if (k < 5) Qb[5LL * t + k] = B.he_node[p1 - 1] < 0 ? B.seen[k * B.nbnode + p1 - 1] : B.q[k * B.ntot + i];
   double s = 0.0;
-  for (int p = B.he_ptr[i]; p < B.he_ptr[i + 1]; ++p) s += col[25LL * p + k];
+  for (int p = B.he_ptr[i]; p < p1; ++p) s += col[25LL * p + k];
   Db[25LL * t + (k % 5) * 5 + k / 5] = s;
 }
 
@@ -376,7 +374,7 @@ __global__ void __launch_bounds__(kBlock) k_jacobian(JacArgs A, const int* __res
 // Dirichlet / sonic-inflow and noSlip overwrites of boundary node states,
 // deferred until all rows have read the pre-update states (the reference
 // applies them inside Bkernel_NumJac after Kernel_NumJac has run): the
-// states k_jac_boundary ended with are copied into q.
+// states the boundary part ended with are copied into q.
 __global__ void __launch_bounds__(kBlock) k_commit_hardset(int nbnd, int ntot, const int* __restrict__ bnd_nodes,
                                                           const double* __restrict__ Qb, double* __restrict__ q) {
   int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -456,7 +454,7 @@ static JacArgs jac_args(Ctx& c) {
 
 static void jac_boundary(Ctx& c, const JacArgs& A, hipStream_t s) {
   if (c.nbnd == 0) return;
-  launch_bnd_resets(c, s, c.d.jqb);
+  launch_bnd_resets(c, s);
   const BndArgs B = bnd_args(c);
   hipLaunchKernelGGL(A.flux_alg ? k_jac_bnd_base<true> : k_jac_bnd_base<false>, dim3(nblk(c.nbnode, kBndBlock)),
                      dim3(kBndBlock), 0, s, B, A.sym2d, A.bcentred, c.d.jhe);
@@ -528,7 +526,7 @@ void launch_jacobian(Ctx& c) {
 void launch_jacobian_overlapped(Ctx& c) {
   JacArgs A = jac_args(c);
   jac_boundary(c, A, c.stream);
-  if (c.nrst > 0) {
+  if (!c.rst_level.empty()) {
     PCFD_HIP(hipMemcpyAsync(c.d.qjac, c.d.q, sizeof(double) * 5 * (size_t)c.ntot, hipMemcpyDeviceToDevice,
                             c.stream));
     A.q = c.d.qjac;

@@ -20,7 +20,6 @@ def rel(a, b):
 # BC types of face tags 1..6 and wall temperatures (< 0 adiabatic) of tags 3 and 5
 MIXES = {
     "noslip both": ([BC_FARFIELD, BC_SONIC_OUTFLOW, BC_NOSLIP, BC_SYMMETRY, BC_NOSLIP, BC_FARFIELD], -1.0, 1.1),
-    # (an adiabatic wall next to another hard-set wall copies a neighbour that the walk may have reset already)
     "floor adiabatic": ([BC_FARFIELD, BC_FARFIELD, BC_SYMMETRY, BC_IMPERMEABLE, BC_NOSLIP, BC_SYMMETRY], 0.9, -1.0),
     "resets in between": ([BC_SONIC_INFLOW, BC_SONIC_OUTFLOW, BC_IMPERMEABLE, BC_DIRICHLET, BC_NOSLIP, BC_FARFIELD],
                           1.0, 1.0),
@@ -31,12 +30,38 @@ MIXES = {
 @pytest.mark.parametrize("centred", [0, 1])
 @pytest.mark.parametrize("mix", list(MIXES))
 def test_mixed_half_edges(mix, centred):
-    from proteuscfd_amd import gpu
     types, tw3, tw5 = MIXES[mix]
+    check(mix, types, {3: tw3, 5: tw5}, centred)
+
+
+# Adiabatic walls whose wall-normal neighbour another half-edge resets: before (its new state is read, as in the
+# walk in half-edge order) or after (its old one), in chains, and each the other's across a channel one cell wide.
+# BC types of face tags 1..6, wall temperatures, cells across
+RESET_NEIGHBOURS = {
+    "inflow beside": ([BC_SONIC_INFLOW, BC_SONIC_OUTFLOW, BC_SYMMETRY, BC_SYMMETRY, BC_NOSLIP, BC_FARFIELD], {5: -1.0}, 4),
+    "set walls beside": ([BC_DIRICHLET, BC_SONIC_OUTFLOW, BC_NOSLIP, BC_NOSLIP, BC_NOSLIP, BC_SONIC_INFLOW],
+                         {3: 1.1, 4: -1.0, 5: -1.0}, 4),
+    "all adiabatic": ([BC_NOSLIP, BC_NOSLIP, BC_NOSLIP, BC_NOSLIP, BC_NOSLIP, BC_NOSLIP], {}, 3),
+    "thin channel": ([BC_SONIC_INFLOW, BC_SONIC_OUTFLOW, BC_NOSLIP, BC_NOSLIP, BC_NOSLIP, BC_FARFIELD],
+                     {3: -1.0, 4: -1.0, 5: 0.9}, 1),
+}
+
+
+@pytest.mark.parametrize("centred", [0, 1])
+@pytest.mark.parametrize("mix", list(RESET_NEIGHBOURS))
+def test_adiabatic_wall_beside_a_reset_node(mix, centred):
+    types, tw, ny = RESET_NEIGHBOURS[mix]
+    check(mix, types, tw, centred, ny)
+
+
+def check(mix, types, tw, centred, ny=4):
+    from proteuscfd_amd import gpu
     p = Params(sorder=1, cfl=5.0, nsgs=2, viscous=1, reynolds=1.0e3, mach_ref=0.3, jac_boundary_type=centred)
-    case = cases.plate_case(nx=5, ny=4, nz=6, nlayers=2, first_h=0.05, growth=1.2, params=p)
+    case = cases.plate_case(nx=5, ny=ny, nz=6, nlayers=2, first_h=0.05, growth=1.2, params=p)
     case.bc_type[1:7] = types
-    case.twall[3], case.twall[5] = tw3, tw5
+    case.twall[1:7] = -1.0
+    for tag, t in tw.items():
+        case.twall[tag] = t
     # distinct reference states, so that it shows which reset a half-edge saw
     for t in range(1, 7):
         case.qref[t, :5] *= 1.0 + 0.01 * t
