@@ -28,10 +28,11 @@ struct ChemDev {
 // Powers come in two forms.
 //
 // LibPow calls pow for every exponent, as the reference does.  The finite-rate
-// solver keeps it: its source Jacobian differences two sources 1e-8 apart, so a
-// last bit of a power is a part in 1e8 of an entry, and of 200 solves of the
-// reacting bump from random states two answered the other form's last bits with
-// more than 2e-7 of a value in their result.
+// solver keeps it, in the surrogate's exact fallback too: its source Jacobian
+// differences two sources 1e-8 apart, so a last bit of a power is a part in 1e8
+// of an entry, and of 200 solves of the reacting bump from random states two
+// answered the other form's last bits with more than 2e-7 of a value in their
+// result.
 //
 // ProductPow, for the calls that return rates, sources and Jacobians: the small
 // whole exponents that mass action is made of are products -- 1 and x are pow's

@@ -37,14 +37,11 @@
 #include "chem_model.h"
 #include "fill.h"
 #include "fr_physics.h"
+#include "wdot_list.h"
 
 namespace pcfd {
 const ChemDev* chem_device_model(const pcfd_chem* c);
 int chem_nspecies(const pcfd_chem* c);
-// the production-rate surrogate with exact fallback (kernels_mlp.hip): runs on
-// the surrogate's stream and returns with it synchronised
-int surrogate_launch(pcfd_chem* chem, pcfd_mlp& m, const pcfd_surrogate_desc* d, int n, const double* rhoi,
-                     const double* T, double* wdot, int* lst, int* cnt, int* off, int* nfallback, double* ms);
 }  // namespace pcfd
 
 using namespace pcfd;
@@ -1034,7 +1031,7 @@ void run_residual(pcfd_fr& f, double* norms) {
     int nf = 0;
     double ms = 0.0;
     const int rc = surrogate_launch(const_cast<pcfd_chem*>(f.chem), *f.mlp, &f.sdesc, f.nnode, f.s_rhoi, f.s_T,
-                                    f.s_w, f.s_lst, f.s_cnt, f.s_off, &nf, &ms);
+                                    f.s_w, f.s_lst, f.s_cnt, f.s_off, k_wdot_list<LibPow>, &nf, &ms);
     if (rc != PCFD_OK) throw std::runtime_error("surrogate production rates failed");
     f.s_last_fallback = nf;
     f.s_fallback_total += nf;

@@ -30,6 +30,7 @@
 #include "chem_model.h"
 #include "fill.h"
 #include "scan.h"
+#include "wdot_list.h"
 
 namespace pcfd {
 
@@ -992,31 +993,6 @@ __global__ void __launch_bounds__(kMlpBlock) k_surrogate(MlpWeights w, MlpWeight
   }
 }
 
-// Exact rates of the fallback cells: entry t of the compacted list lives in
-// the pass p with off[p] <= t < off[p+1] (binary search).
-__global__ void __launch_bounds__(kChemBlock) k_wdot_list(const ChemDev* __restrict__ md, int npass,
-                                                         const int* __restrict__ lst, const int* __restrict__ off,
-                                                         const double* __restrict__ rhoi,
-                                                         const double* __restrict__ T, double* __restrict__ wdot) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= off[npass]) return;
-  int lo = 0, hi = npass;  // off[lo] <= t < off[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (off[mid] <= t) lo = mid;
-    else hi = mid;
-  }
-  const int c = lst[(long long)lo * 64 + (t - off[lo])];
-  const ChemDev& m = *md;
-  // the surrogate is built for five species
-  double r[kNout], w[kNout];
-#pragma unroll
-  for (int k = 0; k < kNout; ++k) r[k] = rhoi[(long long)c * kNout + k];
-  wdot_of<kNout>(m, r, T[c], w);
-#pragma unroll
-  for (int k = 0; k < kNout; ++k) wdot[(long long)c * kNout + k] = w[k];
-}
-
 const ChemDev* chem_device_model(const pcfd_chem* c);
 int chem_nspecies(const pcfd_chem* c);
 const double* chem_mw(const pcfd_chem* c);
@@ -1051,12 +1027,6 @@ int* scratch_on_current_device() {
   return g_scratch_ptr[dev];
 }
 
-// Surrogate pass + fixed-order scan of the per-pass fallback counts + exact
-// rates of the fallback list, on the mlp's stream; lst/cnt/off hold at least
-// npass*64, npass and npass+1 ints.
-int surrogate_launch(pcfd_chem* chem, pcfd_mlp& m, const pcfd_surrogate_desc* d, int n, const double* rhoi,
-                     const double* T, double* wdot, int* lst, int* cnt, int* off, int* nfallback, double* ms);
-
 }  // namespace pcfd
 
 extern "C" {
@@ -1079,8 +1049,8 @@ int pcfd_chem_surrogate_wdot_device(pcfd_chem* chem, pcfd_mlp* mlp, const pcfd_s
     // fallback list: 64 slots per pass, per-pass counts, their offsets
     DBuf dlst(sizeof(int) * (size_t)npass * 64), dcnt(sizeof(int) * (size_t)npass),
         doff(sizeof(int) * ((size_t)npass + 1));
-    return surrogate_launch(chem, m, d, n, rhoi, T, wdot, dlst.as<int>(), dcnt.as<int>(), doff.as<int>(), nfallback,
-                            ms);
+    return surrogate_launch(chem, m, d, n, rhoi, T, wdot, dlst.as<int>(), dcnt.as<int>(), doff.as<int>(),
+                            k_wdot_list<ProductPow>, nfallback, ms);
   });
 }
 
@@ -1108,7 +1078,8 @@ int pcfd_chem_surrogate_wdot_device_noalloc(pcfd_chem* chem, pcfd_mlp* mlp, cons
     int* const lst = base;
     int* const cnt = base + (size_t)kNoAllocPasses * 64;
     int* const off = cnt + kNoAllocPasses;
-    return surrogate_launch(chem, m, d, n, rhoi, T, wdot, lst, cnt, off, nfallback, ms);
+    return surrogate_launch(chem, m, d, n, rhoi, T, wdot, lst, cnt, off, k_wdot_list<ProductPow>, nfallback,
+                            ms);
   });
 }
 
@@ -1117,7 +1088,8 @@ int pcfd_chem_surrogate_wdot_device_noalloc(pcfd_chem* chem, pcfd_mlp* mlp, cons
 namespace pcfd {
 
 int surrogate_launch(pcfd_chem* chem, pcfd_mlp& m, const pcfd_surrogate_desc* d, int n, const double* rhoi,
-                     const double* T, double* wdot, int* lst, int* cnt, int* off, int* nfallback, double* ms) {
+                     const double* T, double* wdot, int* lst, int* cnt, int* off, WdotList exact, int* nfallback,
+                     double* ms) {
   SurrogateDev sd{};
   sd.lnT_mid = (float)d->lnT_mid;
   sd.ilnT_half = (float)(1.0 / d->lnT_half);
@@ -1169,7 +1141,7 @@ int surrogate_launch(pcfd_chem* chem, pcfd_mlp& m, const pcfd_surrogate_desc* d,
                        rhoi, T, wdot, lst, cnt);
   mcheck(hipGetLastError(), "k_surrogate");
   launch_scan_counts(m.stream, npass, cnt, off);
-  hipLaunchKernelGGL(k_wdot_list, dim3((n + kChemBlock - 1) / kChemBlock), dim3(kChemBlock), 0, m.stream,
+  hipLaunchKernelGGL(exact, dim3((n + kChemBlock - 1) / kChemBlock), dim3(kChemBlock), 0, m.stream,
                      chem_device_model(chem), npass, lst, off, rhoi, T, wdot);
   mcheck(hipGetLastError(), "k_wdot_list");
   mcheck(hipEventRecord(m.e1, m.stream), "hipEventRecord");

@@ -295,10 +295,7 @@ def test_fr_surrogate_rates_in_the_loop():
     on the reacting bump (3000 K, partly dissociated), 5 steps each.  With
     err_tol 1e-12 every node goes back to the exact rates: the steps agree
     with exact chemistry to 1e-8 in the residual history and 1e-6 in the
-    field (the fallback's exact rates come from the dimensional states, the
-    residual's own from the non-dimensional ones, so the source differs in
-    the last bits, and the reacting Newton steps amplify that as they do
-    between host and device).  With err_tol 0.5 and the rate floors at
+    field (to the bit: test_gpu_fr_fallback.py).  With err_tol 0.5 and the rate floors at
     rho / t_ref, the network keeps some nodes (about 8 %): the run stays
     finite, the stats add up, and the field moves by less than 5e-2 per
     variable from exact chemistry in the 5 steps.  The source Jacobian
