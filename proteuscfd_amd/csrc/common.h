@@ -109,7 +109,7 @@ struct Dev {
   // reductions
   double* red = nullptr;    // partial sums
   double* red_out = nullptr;
-  int* icount = nullptr;
+  int* icount = nullptr;    // [0] zeroed rows of an update, [1] a diagonal block holds a NaN or infinity
 };
 
 constexpr size_t kPin = 1 << 18;  // 2 MiB

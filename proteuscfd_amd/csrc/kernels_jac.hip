@@ -35,6 +35,7 @@ struct JacArgs {
   int flux_alg;            // 1: algebraic flux (generic form only)
   int centred;             // 1: centred differences, jacobianFieldType 1 (generic form only)
   int bcentred;            // 1: centred boundary differences, jacobianBoundaryType 1
+  int* nonfinite;          // cleared by the rows, set by k_prepare_sgs
 };
 
 // One-sided differences with h = 1e-8 (ucs/jacobian.tcc:268): the quotient
@@ -196,6 +197,7 @@ __global__ void __launch_bounds__(kBlock) k_jacobian(JacArgs A, const int* __res
   const int r = ((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * 12 + lane64 / 5;
   const int c = lane64 % 5;
   if (r >= A.nrow_pad) return;
+  if (r == 0 && c == 0) *A.nonfinite = 0;
   const int i = A.srow[r];
   if (i < 0) return;
   const int chunk = r >> 6, lane = r & 63;
@@ -449,7 +451,7 @@ static JacArgs jac_args(Ctx& c) {
                  c.d.gnrm, c.nslot_g * kW, c.d.vol, c.d.dt, c.d.q, c.d.srow, c.d.sbase, c.d.xyz,
                  ViscParams{p.gamma, p.re_tilde, p.prandtl, p.prandtl_t, p.sutherland_s, p.symmetry2d},
                  p.flux_type == PCFD_FLUX_ALGEBRAIC ? 1 : 0, p.jac_field_type == 1 ? 1 : 0,
-                 p.jac_boundary_type == 1 ? 1 : 0};
+                 p.jac_boundary_type == 1 ? 1 : 0, c.d.icount + 1};
 }
 
 static void jac_boundary(Ctx& c, const JacArgs& A, hipStream_t s) {
@@ -561,15 +563,24 @@ void jacobian_join(Ctx& c) {
 // the same elimination (rows swapped physically: compile-time register
 // indices, no scratch) applied to the unit columns, so a row update is one
 // 5x5 product.  The elimination runs in FP64 for both storage types.
+//
+// A block that holds a NaN or an infinity is reported: an off-diagonal block
+// holds one only where a diagonal block does (its column's, which sums it, or
+// where that node's rows are hard-set its own row's, which has the same flux),
+// and the first sweep then takes nothing for granted (k_sgs_color).
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_prepare_sgs(int nrow_pad, const int* __restrict__ srow,
-                                                       T* __restrict__ Dg) {
+                                                       T* __restrict__ Dg, int* __restrict__ nonfinite) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= nrow_pad || srow[r] < 0) return;
   T* a = Dg + (long long)(r >> 6) * 25 * kW + (r & 63);
   double A[25];
 #pragma unroll
   for (int k = 0; k < 25; ++k) A[k] = (double)a[k * kW];
+  double z = 0.0;
+#pragma unroll
+  for (int k = 0; k < 25; ++k) z += 0.0 * A[k];
+  if (z != 0.0) atomicOr(nonfinite, 1);  // NaN
   int p[5] = {0, 1, 2, 3, 4};
   int row = 0;  // persists across columns, like the reference's
 #pragma unroll
@@ -633,10 +644,10 @@ __global__ void __launch_bounds__(kBlock) k_prepare_sgs(int nrow_pad, const int*
 void launch_prepare_sgs(Ctx& c) {
   if (c.prm.precision == PCFD_CHOSEN_FP32)
     hipLaunchKernelGGL(k_prepare_sgs<float>, dim3(nblk(c.nrow_pad)), dim3(kBlock), 0, c.stream, c.nrow_pad, c.d.srow,
-                       c.d.Df);
+                       c.d.Df, c.d.icount + 1);
   else
     hipLaunchKernelGGL(k_prepare_sgs<double>, dim3(nblk(c.nrow_pad)), dim3(kBlock), 0, c.stream, c.nrow_pad,
-                       c.d.srow, c.d.Dd);
+                       c.d.srow, c.d.Dd, c.d.icount + 1);
   PCFD_HIP(hipGetLastError());
 }
 

@@ -49,7 +49,10 @@ __device__ __forceinline__ T mload(const T* p) {
 // only the blocks whose neighbours have moved since (the lower-colour run
 // forwards, the higher-colour run backwards) and takes the other half's sum
 // from `ps`, where it leaves its own: every off-diagonal block is read once
-// per symmetric sweep instead of twice.
+// per symmetric sweep instead of twice.  In the first forward sweep the
+// higher-colour neighbours are zero and their blocks are left out, unless the
+// matrix holds NaNs or infinities (`nonfinite` given and set): those times zero
+// are NaN, and the rows that have them are the rows an update leaves out.
 //
 // LPR lanes share a row and take alternate slots; their partial sums are
 // combined with a fixed exchange (all lanes end with the same value) before
@@ -73,7 +76,8 @@ __global__ void __launch_bounds__(kBlock) k_sgs_color(int row0, int nrows, int b
                                                      const int* __restrict__ sbase, const int* __restrict__ scol,
                                                      const T* __restrict__ Moff, const T* __restrict__ Dg,
                                                      const T* __restrict__ bs, T* __restrict__ ps,
-                                                     T* __restrict__ x, T* __restrict__ xnode) {
+                                                     T* __restrict__ x, T* __restrict__ xnode,
+                                                     const int* __restrict__ nonfinite) {
   constexpr int RPW = 64 / LPR;  // rows per wavefront
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const int l64 = threadIdx.x & 63;
@@ -107,6 +111,16 @@ __global__ void __launch_bounds__(kBlock) k_sgs_color(int row0, int nrows, int b
         v += mload<NT>(blk + (rr * 5 + 3) * kW) * x3;
         v += mload<NT>(blk + (rr * 5 + 4) * kW) * x4;
         acc[rr] += v;
+      }
+    }
+    if (nonfinite && __builtin_expect(*nonfinite != 0, 0)) {
+      const int wu = swidth[chunk];
+      for (int s = wl + sub; s < wu && scol[cb + (long long)s * kW] >= 0; s += LPR) {
+        const T* blk = mb + (long long)s * 25 * kW;
+#pragma unroll 1
+        for (int k = 0; k < 5; ++k)
+#pragma unroll
+          for (int rr = 0; rr < 5; ++rr) acc[rr] += blk[(rr * 5 + k) * kW] * (T)0;
       }
     }
   }
@@ -193,13 +207,13 @@ static int lanes_per_row(int nrows) { return nrows <= 4096 ? 8 : nrows <= 12288 
 
 template <typename T, bool NT>
 static void sgs_pass(Ctx& c, int row0, int nrows, bool backward, bool use_ps, bool save_ps, const T* Moff,
-                     const T* Dg, const T* bs, T* ps, T* x, T* xnode) {
+                     const T* Dg, const T* bs, T* ps, T* x, T* xnode, const int* nonfinite) {
   const int lpr = lanes_per_row(nrows);
   auto kern = lpr == 1 ? k_sgs_color<T, 1, NT>
               : lpr == 2 ? k_sgs_color<T, 2, NT> : lpr == 4 ? k_sgs_color<T, 4, NT> : k_sgs_color<T, 8, NT>;
   hipLaunchKernelGGL(kern, dim3(nblk((long long)nrows * lpr)), dim3(kBlock), 0, c.stream, row0, nrows, (int)backward,
                      (int)use_ps, (int)save_ps, c.d.srow, c.d.swidth, c.d.swidth_lo, c.d.sbase, c.d.scol, Moff, Dg,
-                     bs, ps, x, xnode);
+                     bs, ps, x, xnode, nonfinite);
   PCFD_HIP(hipGetLastError());
 }
 
@@ -241,7 +255,8 @@ static void sgs_impl(Ctx& c, int nsgs, const T* Moff, const T* Dg, T* bs, T* ps,
         const int nrows = (c.color_chunk[col + 1] - c.color_chunk[col]) * kW;
         (streamed ? sgs_pass<T, true> : sgs_pass<T, false>)(c, row0, nrows, dir == 1, inner && !first_pass,
                                                             inner && !last_pass, Moff, Dg, bs, ps, x,
-                                                            last_pass ? xnode : nullptr);
+                                                            last_pass ? xnode : nullptr,
+                                                            first_pass ? c.d.icount + 1 : nullptr);
       }
     }
     sub_end(c, 9);
