@@ -41,6 +41,15 @@ void dzero(Ctx& c, T** p, size_t n) {
   launch_zero(c.stream, *p, n * (sizeof(T) / 4));
 }
 
+// two host arrays in one device array: q points at the second
+template <typename T>
+void dput2(Ctx& c, T** p, T** q, const std::vector<T>& a, const std::vector<T>& b) {
+  std::vector<T> h(a);
+  h.insert(h.end(), b.begin(), b.end());
+  dput(c, p, h);
+  *q = *p + a.size();
+}
+
 template <typename T>
 void dfree(T*& p) {
   if (p) (void)hipFree(p);
@@ -52,12 +61,12 @@ void free_all(Ctx& c) {
   dfree(d.xyz); dfree(d.vol); dfree(d.vol23); dfree(d.sw); dfree(d.gwidth); dfree(d.gbase); dfree(d.gcol); dfree(d.gnrm); dfree(d.qrk); dfree(d.aos);
   if (c.pin) (void)hipHostFree(c.pin);
   c.pin = c.pin_dev = nullptr;
-  dfree(d.he_ptr); dfree(d.he_id); dfree(d.he_tag); dfree(d.he_node); dfree(d.seen); dfree(d.he_desc); dfree(d.rst); dfree(d.he_src); dfree(d.he_a); dfree(d.bnd_nodes); dfree(d.bidx);
-  dfree(d.jdb); dfree(d.jhe); dfree(d.jcol); dfree(d.jqb); dfree(d.bc_type); dfree(d.twall); dfree(d.spos);
+  dfree(d.he_ptr); dfree(d.he_id); dfree(d.he_tag); dfree(d.he_node); dfree(d.seen); dfree(d.he_desc); dfree(d.rst); dfree(d.he_a); dfree(d.bnd_nodes); dfree(d.bidx);
+  dfree(d.jdb); dfree(d.jhe); dfree(d.jqb); dfree(d.bc_type); dfree(d.twall); dfree(d.spos);
   dfree(d.qref); dfree(d.q); dfree(d.grad); dfree(d.lim); dfree(d.lim2); dfree(d.edges); dfree(d.clip_flag); dfree(d.clip_cnt);
   dfree(d.clip_off); dfree(d.clip_list); dfree(d.b); dfree(d.dt);
-  dfree(d.gslot); dfree(d.srow); dfree(d.swidth); dfree(d.swidth_lo); dfree(d.sbase); dfree(d.scol); dfree(d.Md); dfree(d.Mf); dfree(d.Dd);
-  dfree(d.Df); dfree(d.bsd); dfree(d.bsf); dfree(d.xsd); dfree(d.xsf); dfree(d.psd); dfree(d.psf); dfree(d.xd); dfree(d.xf); dfree(d.red);
+  dfree(d.srow); dfree(d.swidth); dfree(d.sbase); dfree(d.scol); dfree(d.Md); dfree(d.Mf); dfree(d.Dd);
+  dfree(d.Df); dfree(d.xsd); dfree(d.xsf); dfree(d.red);
   dfree(d.red_out); dfree(d.icount); dfree(d.dt_next); dfree(d.qjac);
   for (hipEvent_t* e : {&c.ev0, &c.ev1, &c.ev2, &c.ev3, &c.ev4, &c.ev5, &c.ev_fork, &c.ev_join, &c.ev_norms}) {
     if (*e) (void)hipEventDestroy(*e);
@@ -151,24 +160,32 @@ int need_params(Ctx& c) {
   return PCFD_OK;
 }
 
+// the sweeps' vectors, in one array: the correction in row order (its padding
+// zero), the right-hand side, the partial sums, the correction in node order
+template <typename T>
+void sgs_vectors(Ctx& c, T** xs, T** bs, T** ps, T** x) {
+  if (*xs) return;
+  const size_t n = 5 * (size_t)c.nrow_pad;
+  dzero(c, xs, 3 * n + 5 * (size_t)c.nnode);
+  *bs = *xs + n;
+  *ps = *bs + n;
+  *x = *ps + n;
+}
+
 void ensure_matrix(Ctx& c) {
-  if (!c.d.jhe) dalloc(c, &c.d.jhe, 10 * (size_t)c.nbnode);
-  if (!c.d.jcol) dalloc(c, &c.d.jcol, 25 * (size_t)c.nbnode);
+  if (!c.d.jhe) {
+    dalloc(c, &c.d.jhe, 35 * (size_t)c.nbnode);
+    c.d.jcol = c.d.jhe + 10 * (size_t)c.nbnode;
+  }
   const size_t off = (size_t)c.nslot_s * kW * 25, dg = (size_t)c.nchunk_s * kW * 25;
   if (c.prm.precision == PCFD_CHOSEN_FP32) {
     if (!c.d.Mf) dalloc(c, &c.d.Mf, off);
     if (!c.d.Df) dalloc(c, &c.d.Df, dg);
-    if (!c.d.bsf) dalloc(c, &c.d.bsf, 5 * (size_t)c.nrow_pad);
-    if (!c.d.xf) dalloc(c, &c.d.xf, 5 * (size_t)c.nnode);
-    if (!c.d.xsf) dzero(c, &c.d.xsf, 5 * (size_t)c.nrow_pad);
-    if (!c.d.psf) dalloc(c, &c.d.psf, 5 * (size_t)c.nrow_pad);
+    sgs_vectors(c, &c.d.xsf, &c.d.bsf, &c.d.psf, &c.d.xf);
   } else {
     if (!c.d.Md) dalloc(c, &c.d.Md, off);
     if (!c.d.Dd) dalloc(c, &c.d.Dd, dg);
-    if (!c.d.bsd) dalloc(c, &c.d.bsd, 5 * (size_t)c.nrow_pad);
-    if (!c.d.xd) dalloc(c, &c.d.xd, 5 * (size_t)c.nnode);
-    if (!c.d.xsd) dzero(c, &c.d.xsd, 5 * (size_t)c.nrow_pad);
-    if (!c.d.psd) dalloc(c, &c.d.psd, 5 * (size_t)c.nrow_pad);
+    sgs_vectors(c, &c.d.xsd, &c.d.bsd, &c.d.psd, &c.d.xd);
   }
 }
 
@@ -462,12 +479,11 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     dalloc(c, &d.sw, 6 * (size_t)nn);
     dput(c, &d.gwidth, gwidth);
     dput(c, &d.gbase, gbase);
-    dput(c, &d.gcol, gcol);
+    dput2(c, &d.gcol, &d.gslot, gcol, gslot);
     dput(c, &d.gnrm, gnrm);
     dput(c, &d.he_ptr, he_ptr);
     dput(c, &d.he_id, he_id);
     dput(c, &d.he_tag, he_tag);
-    dput(c, &d.he_node, he_node);
     {
       std::vector<int4> desc(nb);
       for (int p = 0; p < nb; ++p) {
@@ -480,9 +496,11 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
       std::vector<int> he_src;
       std::vector<int4> rst;
       plan_resets(m, he_ptr, he_node, he_nrm, twall, he_src, rst, c.rst_level);
-      dput(c, &d.he_src, he_src);
-      dput(c, &d.rst, rst);
-      if (!rst.empty()) dalloc(c, &d.seen, 5 * (size_t)nb);
+      dput2(c, &d.he_node, &d.he_src, he_node, he_src);
+      if (!rst.empty()) {
+        dput(c, &d.rst, rst);
+        dalloc(c, &d.seen, 5 * (size_t)nb);
+      }
     }
     dput(c, &d.he_a, he_a);
     dput(c, &d.bnd_nodes, bnd);
@@ -509,9 +527,7 @@ int pcfd_create(const pcfd_mesh_desc* m, pcfd_ctx** out) {
     dalloc(c, &d.b, 5 * (size_t)nn);
     dalloc(c, &d.dt, (size_t)nn);
     dput(c, &d.srow, srow);
-    dput(c, &d.gslot, gslot);
-    dput(c, &d.swidth, swidth);
-    dput(c, &d.swidth_lo, swidth_lo);
+    dput2(c, &d.swidth, &d.swidth_lo, swidth, swidth_lo);
     dput(c, &d.sbase, sbase);
     dput(c, &d.scol, scol);
     dalloc(c, &d.red, 6 * (size_t)std::max(nblk(4LL * nn), 1024));
