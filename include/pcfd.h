@@ -144,7 +144,7 @@ int pcfd_set_timestep(pcfd_ctx* ctx, const double* dt);
 int pcfd_jacobian(pcfd_ctx* ctx);
 /* Download Jacobian blocks for an arbitrary block-CRS pattern (ia[nnode+1],
  * ja[nblocks]); M[blk*25 + r*5 + c].  Valid after pcfd_jacobian and before
- * pcfd_prepare_sgs (which factorises the diagonal blocks in place). */
+ * pcfd_prepare_sgs (which inverts the diagonal blocks in place). */
 int pcfd_download_jacobian(pcfd_ctx* ctx, const int* ia, const int* ja, double* M);
 int pcfd_prepare_sgs(pcfd_ctx* ctx);
 /* nSgs symmetric multicolour sweeps from x0 = 0 on b; x_out[node*5+k].

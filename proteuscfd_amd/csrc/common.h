@@ -194,12 +194,17 @@ __device__ __forceinline__ long long gbase_of(const Gell& g, int i) {
 // Lanes per node of the edge passes.  A node's neighbours are a serial chain
 // of gathers and fluxes, so a mesh that leaves the chip idle takes four lanes
 // a node and a larger one two (us at 1 / 2 / 4 lanes): second-order residual
-// 50 / 36 / 31 (729 nodes), 78 / 60 / 64 (74k), 164 / 138 / 166 (275k); residual
-// with viscous fluxes 95 / 79 / 75 (36k), 406 / 381 / 486 (416k); time step 22 /
-// 14 / 11 (9k), 94 / 73 / 85 (416k).  The gradient's 27 sums cost more to combine:
-// 20 / 15 / 13 (9k), 27 / 23 / 28 (74k), 56 / 60 / 81 (275k).
+// 50 / 36 / 31 (729 nodes), 78 / 60 / 64 (74k), 164 / 138 / 166 (275k), 697 / 620 / -
+// (1.5M); time step 22 / 14 / 11 (9k), 94 / 73 / 85 (416k).
+//
+// The gradient, whose 27 sums cost more to combine, and the viscous pass, which
+// gathers 24 values a neighbour, gain from a second lane only up to the 768
+// workgroups that are resident at once, three a compute unit.  Gradient 20 / 15 /
+// 13 (9k), 24.7 / 21.3 (97k), 25.9 / 27.9 (111k), 56 / 60 / 81 (275k); with the
+// limiter 59.7 / 57.8 (97k), 61.6 / 64.3 (111k); viscous 38 / - / 29 (36k), 52.7 /
+// 41.4 (93k), 53.3 / 56.6 (108k), 333 / 365 (840k), 558 / 624 (1.5M).
 inline int lanes_per_node(int nnode) { return nnode <= 49152 ? 4 : 2; }
-inline int gradient_lanes(int nnode) { return nnode <= 49152 ? 4 : nnode <= 131072 ? 2 : 1; }
+inline int wide_lanes(int nnode) { return nnode <= 49152 ? 4 : nnode <= 98304 ? 2 : 1; }
 
 // LPN (1, 2 or 4) adjacent lanes share a node and take alternate neighbours;
 // these move values among them with DPP quad permutes (no LDS).

@@ -484,7 +484,7 @@ void launch_gradient(Ctx& c, int nterms) {
     return;
   }
   const LimArgs none{0, 0.0, 0.0, nullptr, nullptr};
-  const int lpn = gradient_lanes(c.nnode);
+  const int lpn = wide_lanes(c.nnode);
   auto kern = gradient_kernel<false>(nterms, lpn);
   hipLaunchKernelGGL(kern, dim3(nblk((long long)c.nnode * lpn)), dim3(kBlock), 0, c.stream, c.nnode, c.ntot, gell(c),
                      c.d.xyz,
@@ -709,7 +709,7 @@ void launch_limiter(Ctx& c) {
 void launch_gradient_limiter(Ctx& c, int nterms) {
   const pcfd_params& p = c.prm;
   const LimArgs L{p.limiter, p.venkat_K * p.venkat_K * p.venkat_K, p.chi, c.d.vol, c.d.lim2};
-  const int lpn = gradient_lanes(c.nnode);
+  const int lpn = wide_lanes(c.nnode);
   auto kern = gradient_kernel<true>(nterms, lpn);
   hipLaunchKernelGGL(kern, dim3(nblk((long long)c.nnode * lpn)), dim3(kBlock), 0, c.stream, c.nnode, c.ntot, gell(c),
                      c.d.xyz,

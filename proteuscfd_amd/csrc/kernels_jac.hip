@@ -1,4 +1,4 @@
-// First-order finite-difference block Jacobian and diagonal LU.
+// First-order finite-difference block Jacobian and the inverses of its diagonal.
 //
 // Reference: ComputeSpatialJacobian (ucs/jacobian.tcc:129-210) scatters per
 // edge A[R][L] += -dF/dQL and A[L][R] += dF/dQR (Kernel_NumJac :253-304),
@@ -7,11 +7,11 @@
 // off-diagonal blocks onto the diagonal (Kernel_Diag_NumJac :436-456), and
 // ContributeTemporalTerms adds vol/dt (:213-250).
 //
-// Here one thread owns one block row of the SELL matrix (threads run in
-// SELL row order, so 64 lanes write 64 consecutive addresses): it writes
-// the row's off-diagonal blocks and accumulates its own diagonal (boundary
-// part first, then edges in ascending neighbour order, then the temporal
-// term), so every block has a single writer.  Storage type T is double
+// Here five lanes own one block row of the SELL matrix, a column each (12
+// rows a wavefront, in SELL row order): they write the row's off-diagonal
+// blocks and accumulate its diagonal (boundary part first, then edges in
+// ascending neighbour order, then the temporal term), so every entry has a
+// single writer.  Storage type T is double
 // (plain) or float (chosen form); the differences are always taken in FP64.
 #include <stdexcept>
 

@@ -147,11 +147,11 @@ void launch_viscous(Ctx& c, int higher_order) {
   const pcfd_params& p = c.prm;
   if (!p.viscous && !c.has_noslip) return;
   const ViscParams vp{p.gamma, p.re_tilde, p.prandtl, p.prandtl_t, p.sutherland_s, p.symmetry2d};
-  const int lpn = p.viscous ? lanes_per_node(c.nnode) : 1;
+  const int lpn = p.viscous ? wide_lanes(c.nnode) : 1;
   const int nb = nblk((long long)c.nnode * lpn);
   const Gell g{c.d.gwidth, c.d.gbase, c.d.gcol, c.d.gnrm, c.nslot_g * kW};
   if (p.viscous)
-    hipLaunchKernelGGL((lpn == 4 ? k_viscous<true, 4> : k_viscous<true, 2>), dim3(nb), dim3(kBlock), 0, c.stream,
+    hipLaunchKernelGGL((lpn == 4 ? k_viscous<true, 4> : lpn == 2 ? k_viscous<true, 2> : k_viscous<true, 1>), dim3(nb), dim3(kBlock), 0, c.stream,
                        c.nnode, c.ntot, c.ntag, higher_order, vp, g, c.d.xyz, c.d.q, c.d.grad, c.d.he_ptr, c.d.he_id, c.d.he_tag, c.d.he_a, c.nbnode,
                        c.d.bc_type, c.d.twall, c.d.b, c.d.red);
   else

@@ -1,5 +1,5 @@
 """The edge passes on both sides of every lanes-per-node rule (four lanes up to
-49,152 nodes, two above; the gradient one above 131,072), phase by phase
+49,152 nodes, two above; gradient and viscous pass one above 98,304), phase by phase
 against the oracle, and the fused gradient-limiter pass of the timed
 iterations against the separate passes, NaN states included."""
 import numpy as np
@@ -17,7 +17,7 @@ def rel(a, b):
 
 
 @pytest.mark.parametrize("kind,size", [("bump", 3), ("bump", 37), ("bump", 51), ("plate", (21, 9, 24)),
-                                       ("plate", (60, 20, 45))])
+                                       ("plate", (60, 20, 45)), ("plate", (70, 27, 54))])
 def test_edge_passes(kind, size):
     from proteuscfd_amd import gpu
     if kind == "bump":

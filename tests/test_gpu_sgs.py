@@ -38,12 +38,17 @@ def pattern(m):
     return ia, c[o].astype(np.int32)
 
 
-# rows a colour: 1 (a lone node), a ragged chunk, and about 1.6k, 6k, 60k and 140k
-@pytest.mark.parametrize("n", [1, 2, 131, 5000, 20001, 180001, 420005])
-@pytest.mark.parametrize("precision", [0, 1])
+# rows a colour: 1 (a lone node), a ragged chunk, and about 1.6k, 6k, 60k and 140k; for each storage type the
+# largest matrix does not fit the 256 MiB cache and is streamed
+SIZES = [(p, n) for p in (0, 1) for n in (1, 2, 131, 5000, 20001, 180001, 420005)] + [(1, 900001)]
+STREAMED = {(0, 420005), (1, 900001)}
+
+
+@pytest.mark.parametrize("precision,n", SIZES)
 def test_colour_passes(n, precision):
     from proteuscfd_amd import gpu
     m = ribbon(n)
+    assert (2 * m.nedge * 25 * (4 if precision else 8) > 256 * 2**20) == ((precision, n) in STREAMED)
     q0 = qinf(1.4, 0.5)
     case = Case("ribbon", m, np.array([0, BC_FARFIELD], dtype=np.int32), np.tile(q0, (2, 1)), q0, Params(nsgs=3))
     print(f"[sgs] n={n} precision={precision}", flush=True)
