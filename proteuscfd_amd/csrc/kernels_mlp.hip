@@ -527,6 +527,11 @@ struct pcfd_mlp {
   long long adam_t = 0;
   float last_ms = 0.f;
   std::string err;
+  // training: pinned memory for the index lists and the losses (grown on use, at
+  // most kPinKeep: a call that wants more has its own), a list's last reader
+  void* pin = nullptr;
+  size_t pin_bytes = 0;
+  hipEvent_t drawn[2] = {nullptr, nullptr};
 };
 
 namespace {
@@ -593,7 +598,9 @@ struct DBuf {
 
 struct PinBuf {
   void* p = nullptr;
-  explicit PinBuf(size_t bytes) { mcheck(hipHostMalloc(&p, bytes, hipHostMallocMapped), "hipHostMalloc"); }
+  explicit PinBuf(size_t bytes) {
+    if (bytes) mcheck(hipHostMalloc(&p, bytes, hipHostMallocMapped), "hipHostMalloc");
+  }
   ~PinBuf() {
     if (p) (void)hipHostFree(p);
   }
@@ -601,16 +608,19 @@ struct PinBuf {
   PinBuf& operator=(const PinBuf&) = delete;
 };
 
-struct EventPair {
-  hipEvent_t e[2] = {nullptr, nullptr};
-  EventPair() {
-    for (hipEvent_t& v : e) mcheck(hipEventCreateWithFlags(&v, hipEventDisableTiming), "hipEventCreate");
+// the handle's pinned memory, at least `bytes` (no kernel is reading it: every
+// call drains the stream)
+constexpr size_t kPinKeep = 1 << 20;
+void* pin_space(pcfd_mlp& m, size_t bytes) {
+  if (m.pin_bytes < bytes) {
+    if (m.pin) mcheck(hipHostFree(m.pin), "hipHostFree");
+    m.pin = nullptr;
+    m.pin_bytes = 0;
+    mcheck(hipHostMalloc(&m.pin, bytes, hipHostMallocMapped), "hipHostMalloc");
+    m.pin_bytes = bytes;
   }
-  ~EventPair() {
-    for (hipEvent_t v : e)
-      if (v) (void)hipEventDestroy(v);
-  }
-};
+  return m.pin;
+}
 
 // splitmix64: the batch index stream of training
 uint64_t mix(uint64_t z) {
@@ -638,6 +648,7 @@ int pcfd_mlp_create(unsigned long long seed, pcfd_mlp** out) {
     mcheck(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
     mcheck(hipEventCreate(&c->e0), "hipEventCreate");
     mcheck(hipEventCreate(&c->e1), "hipEventCreate");
+    for (hipEvent_t& e : c->drawn) mcheck(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
     c->scratch = pcfd::scratch_on_current_device();
     c->grid = 1024;
     const size_t P = sizeof(float) * kNparam;
@@ -694,6 +705,9 @@ int pcfd_mlp_destroy(pcfd_mlp* c) {
     if (s) (void)hipFree(s);
   if (c->e0) (void)hipEventDestroy(c->e0);
   if (c->e1) (void)hipEventDestroy(c->e1);
+  for (hipEvent_t e : c->drawn)
+    if (e) (void)hipEventDestroy(e);
+  if (c->pin) (void)hipHostFree(c->pin);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return PCFD_OK;
@@ -806,17 +820,22 @@ int pcfd_mlp_train(pcfd_mlp* c, int n, const float* x, const float* t, int steps
       m.err = "pcfd_mlp_train: invalid arguments";
       return PCFD_ERR_ARG;
     }
-    DBuf dx(sizeof(float) * (size_t)n * kNin), dt(sizeof(float) * (size_t)n * kNout),
-        dloss(sizeof(float) * (size_t)steps);
+    DBuf dx(sizeof(float) * (size_t)n * kNin), dt(sizeof(float) * (size_t)n * kNout);
     // Two index lists in pinned memory, which the gradient kernel reads once,
     // from there: while a step runs the host draws the next one's.  (With one
     // list, a copy and a wait for each step the device sat idle while the host
-    // drew: 90 us a step of 8192 samples, 45 of them busy; 33 so.)
-    PinBuf hidx(sizeof(int) * 2 * (size_t)batch);
+    // drew: 90 us a step of 8192 samples, 45 of them busy; 33 so.)  The steps'
+    // losses go behind the lists.  The memory stays with the network for calls of
+    // a few steps: one step of 64 samples takes 77-94 us, 142 with pinned memory and
+    // events of its own.
+    const size_t bytes = sizeof(int) * 2 * (size_t)batch + sizeof(float) * (size_t)steps;
+    PinBuf own(bytes > kPinKeep ? bytes : 0);
+    int* const hidx = (int*)(own.p ? own.p : pin_space(m, bytes));
+    const float* const hloss = (const float*)(hidx + 2 * (size_t)batch);
     int* didx = nullptr;
-    mcheck(hipHostGetDevicePointer((void**)&didx, hidx.p, 0), "hipHostGetDevicePointer");
-    EventPair done;
-    struct Drain {  // the kernels read the lists: none is freed before they end
+    mcheck(hipHostGetDevicePointer((void**)&didx, hidx, 0), "hipHostGetDevicePointer");
+    float* const dloss = (float*)(didx + 2 * (size_t)batch);
+    struct Drain {  // the kernels read the lists: none is freed or drawn anew before they end
       hipStream_t s;
       ~Drain() { (void)hipStreamSynchronize(s); }
     } drain{m.stream};
@@ -828,8 +847,8 @@ int pcfd_mlp_train(pcfd_mlp* c, int n, const float* x, const float* t, int steps
     mcheck(hipEventRecord(m.e0, m.stream), "hipEventRecord");
     for (int it = 0; it < steps; ++it) {
       const size_t at = (size_t)(it & 1) * batch;
-      int* list = (int*)hidx.p + at;
-      if (it >= 2) mcheck(hipEventSynchronize(done.e[it & 1]), "hipEventSynchronize");
+      int* list = hidx + at;
+      if (it >= 2) mcheck(hipEventSynchronize(m.drawn[it & 1]), "hipEventSynchronize");
       for (int k = 0; k < batch; ++k) {
         s = mix(s);
         // s % n by the reciprocal: the quotient is at most one too small
@@ -838,23 +857,19 @@ int pcfd_mlp_train(pcfd_mlp* c, int n, const float* x, const float* t, int steps
         list[k] = (int)rem;
       }
       const int ngroup = grad_groups(m, batch, dx.as<float>(), dt.as<float>(), didx + at);
-      mcheck(hipEventRecord(done.e[it & 1], m.stream), "hipEventRecord");
+      mcheck(hipEventRecord(m.drawn[it & 1], m.stream), "hipEventRecord");
       ++m.adam_t;
       // cosine decay of the step size over the run
       const float lr_t = 0.5f * lr * (1.f + std::cos(3.14159265f * (float)it / (float)std::max(1, steps)));
       const float c1 = 1.f - std::pow(b1, (float)m.adam_t), c2 = 1.f - std::pow(b2, (float)m.adam_t);
       hipLaunchKernelGGL(k_mlp_adam, dim3(kNparam / kAdamBlock + 1), dim3(kAdamBlock), 0, m.stream, m.p, m.m, m.v,
-                         ngroup, m.part2, m.loss2, dloss.as<float>() + it, lr_t, b1, b2, eps, c1, c2, m.W);
+                         ngroup, m.part2, m.loss2, dloss + it, lr_t, b1, b2, eps, c1, c2, m.W);
       mcheck(hipGetLastError(), "k_mlp_adam");
-    }
-    if (loss_history && steps > 0) {
-      mcheck(hipMemcpyAsync(loss_history, dloss.p, sizeof(float) * (size_t)steps, hipMemcpyDeviceToHost, m.stream),
-             "copy");
-      mcheck(hipStreamSynchronize(m.stream), "hipStreamSynchronize");
-      for (int it = 0; it < steps; ++it) loss_history[it] /= (float)((long long)batch * kNout);
     }
     mcheck(hipEventRecord(m.e1, m.stream), "hipEventRecord");
     mcheck(hipEventSynchronize(m.e1), "hipEventSynchronize");
+    if (loss_history)
+      for (int it = 0; it < steps; ++it) loss_history[it] = hloss[it] / (float)((long long)batch * kNout);
     mcheck(hipEventElapsedTime(&m.last_ms, m.e0, m.e1), "hipEventElapsedTime");
     return PCFD_OK;
   });

@@ -64,3 +64,27 @@ def test_training_draws_its_batches_in_order(batch):
         # BF16 roundings that go the other way, as above
         assert abs(hist[it] - lo) <= 2.0**-9 * lo, it
     net.close()
+
+
+def test_calls_share_a_network():
+    """Calls of growing and shrinking batches on one network, among them one whose index lists it does not keep
+    (above 1 MiB): every step's loss is its own batch's."""
+    from proteuscfd_amd import gpu
+
+    n, steps = 140001, 3
+    net = gpu.MLP(seed=0)
+    p = R.init(9).astype(np.float32)
+    x, t = samples(n, 4)
+    net.params = p
+    for k, batch in enumerate([1, 300, 140000, 17]):
+        print(f"[mlp batches] shared batch={batch}", flush=True)
+        hist = net.train(x, t, steps=steps, batch=batch, lr=1e-9, seed=70 + k)
+        s = 70 + k
+        for it in range(steps):
+            idx = []
+            for _ in range(batch):
+                s = mix(s)
+                idx.append(s % n)
+            lo, _ = R.loss_grad(p, x[idx], t[idx])
+            assert abs(hist[it] - lo) <= 2.0**-9 * lo, (batch, it)
+    net.close()
