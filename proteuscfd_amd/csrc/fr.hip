@@ -93,26 +93,21 @@ __device__ __forceinline__ void store_state(double* __restrict__ q, long long i,
 // registers takes 0.094 ms (the same bits).
 constexpr int kBB = 64;  // threads per block of the half-edge kernels: one wavefront, up to 512 registers
 
-__device__ __forceinline__ bool resets_node(int type) { return type == fr::kSonicInflow || type == fr::kDirichlet; }
+__host__ __device__ __forceinline__ bool resets_node(int type) { return type == fr::kSonicInflow || type == fr::kDirichlet; }
 
-// the node state half-edge p of node i sees
+// the node state half-edge p of node i sees: the reference state of tag
+// he_seen[p], or the node's own
 template <int NS>
 __device__ __forceinline__ void load_seen(const double* __restrict__ q, const double* __restrict__ qref, int i, int p,
-                                          const int* __restrict__ he_ptr, const int* __restrict__ he_id,
-                                          const int* __restrict__ he_tag, const int* __restrict__ bc_type,
-                                          State<NS>& L, const Model& m) {
-  int t = -1;
-  for (int k = he_ptr[i]; k < p; ++k) {
-    const int tag = he_tag[he_id[k]];
-    if (resets_node(bc_type[tag])) t = tag;
-  }
+                                          const int* __restrict__ he_seen, State<NS>& L, const Model& m) {
+  const int t = he_seen[p];
   if (t >= 0) load_state<NS>(qref, t, L, m);
   else load_state<NS>(q, i, L, m);
 }
 
 template <int NS>
 __global__ void __launch_bounds__(kBB) k_fr_bcs(const Model* __restrict__ mp, int nbe, const int* __restrict__ he_node,
-                                               const int* __restrict__ he_ptr, const int* __restrict__ he_id,
+                                               const int* __restrict__ he_seen, const int* __restrict__ he_id,
                                                const int* __restrict__ he_tag, const double* __restrict__ he_a,
                                                const int* __restrict__ bc_type, const double* __restrict__ qref,
                                                int nnode, double beta, double* __restrict__ q) {
@@ -121,7 +116,7 @@ __global__ void __launch_bounds__(kBB) k_fr_bcs(const Model* __restrict__ mp, in
   const Model& m = *mp;
   const int i = he_node[p], h = he_id[p], tag = he_tag[h];
   State<NS> L, R, Qr;
-  load_seen<NS>(q, qref, i, p, he_ptr, he_id, he_tag, bc_type, L, m);
+  load_seen<NS>(q, qref, i, p, he_seen, L, m);
   load_state<NS>(q, (long long)nnode + h, R, m);
   load_state<NS>(qref, tag, Qr, m);
   double a[4];
@@ -130,25 +125,17 @@ __global__ void __launch_bounds__(kBB) k_fr_bcs(const Model* __restrict__ mp, in
   if (fr::bc_state<NS>(m, bc_type[tag], L, R, Qr, a, beta)) store_state<NS>(q, (long long)nnode + h, R);
 }
 
-// boundary nodes with a Dirichlet / sonic-inflow half-edge take the reference
-// state of the last one
+// the nodes with a Dirichlet / sonic-inflow half-edge (rst: node, tag of the
+// last one) take its reference state
 template <int NS>
-__global__ void __launch_bounds__(kFB) k_fr_hardset(int nbnd, const int* __restrict__ bnd,
-                                                   const int* __restrict__ he_ptr, const int* __restrict__ he_id,
-                                                   const int* __restrict__ he_tag, const int* __restrict__ bc_type,
+__global__ void __launch_bounds__(kFB) k_fr_hardset(int nrst, const int2* __restrict__ rst,
                                                    const double* __restrict__ qref, double* __restrict__ q) {
   constexpr int NE = NS + 4;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nbnd) return;
-  const int i = bnd[t];
-  int last = -1;
-  for (int k = he_ptr[i]; k < he_ptr[i + 1]; ++k) {
-    const int tag = he_tag[he_id[k]];
-    if (resets_node(bc_type[tag])) last = tag;
-  }
-  if (last < 0) return;
+  if (t >= nrst) return;
+  const int2 r = rst[t];
 #pragma unroll
-  for (int k = 0; k < NE; ++k) q[(long long)i * NE + k] = qref[(long long)last * NE + k];
+  for (int k = 0; k < NE; ++k) q[(long long)r.x * NE + k] = qref[(long long)r.y * NE + k];
 }
 
 // ---- edge passes -----------------------------------------------------------
@@ -450,7 +437,7 @@ __global__ void __launch_bounds__(kFB) k_fr_jac_edge(const Model* __restrict__ m
 template <int NS>
 __global__ void __launch_bounds__(kBB) k_fr_jac_bnd_base(const Model* __restrict__ mp, int nbe,
                                                         const int* __restrict__ he_node,
-                                                        const int* __restrict__ he_ptr,
+                                                        const int* __restrict__ he_seen,
                                                         const int* __restrict__ he_id, const int* __restrict__ he_tag,
                                                         const double* __restrict__ he_a,
                                                         const int* __restrict__ bc_type,
@@ -462,7 +449,7 @@ __global__ void __launch_bounds__(kBB) k_fr_jac_bnd_base(const Model* __restrict
   const Model& m = *mp;
   const int i = he_node[p], h = he_id[p], tag = he_tag[h];
   State<NS> L, R, Qr;
-  load_seen<NS>(q, qref, i, p, he_ptr, he_id, he_tag, bc_type, L, m);
+  load_seen<NS>(q, qref, i, p, he_seen, L, m);
   load_state<NS>(q, (long long)nnode + h, R, m);
   load_state<NS>(qref, tag, Qr, m);
   double a[4];
@@ -884,7 +871,7 @@ struct pcfd_fr {
   std::string err;
   const pcfd_chem* chem = nullptr;
   int ns = 0, ne = 0, nnode = 0, nbnode = 0, nedge = 0, ntot = 0, ntag = 0, nbnd = 0;
-  bool has_hardset = false;  // a half-edge resets its node's state (Dirichlet, sonic inflow)
+  int nrst = 0;  // nodes whose state a half-edge resets (Dirichlet, sonic inflow)
   int ncolor = 0, nchunk = 0, nrow_pad = 0;
   long long nslot = 0;
   std::vector<int> color_chunk, h_nptr, h_nslot, h_edges, h_srow, h_spos, h_sbase;
@@ -901,9 +888,10 @@ struct pcfd_fr {
   // device arrays
   double *q = nullptr, *qref = nullptr, *vol = nullptr, *edge_a = nullptr, *he_a = nullptr, *eflux = nullptr,
          *elam = nullptr, *b = nullptr, *dt = nullptr, *jdb = nullptr, *bhe = nullptr, *bcol = nullptr, *red = nullptr, *aux = nullptr;
-  int *edges = nullptr, *nptr = nullptr, *nslot_d = nullptr, *he_ptr = nullptr, *he_id = nullptr, *he_tag = nullptr, *he_node = nullptr,
+  int *edges = nullptr, *nptr = nullptr, *nslot_d = nullptr, *he_ptr = nullptr, *he_id = nullptr, *he_tag = nullptr, *he_node = nullptr, *he_seen = nullptr,
       *bc_type = nullptr, *bnd = nullptr, *bidx = nullptr, *srow = nullptr, *swidth = nullptr, *sbase = nullptr,
       *scol = nullptr, *sedge = nullptr, *icount = nullptr;
+  int2* rst = nullptr;
   long long* piv = nullptr;
   double *ediag = nullptr, *nterm = nullptr;  // Jacobian diagonal parts: per edge side, per row
   fr::Side* jst = nullptr;                    // and the nodes' plain and raised states' properties
@@ -942,7 +930,7 @@ void dfree(T*& p) {
 void free_all(pcfd_fr& f) {
   dfree(f.q); dfree(f.qref); dfree(f.vol); dfree(f.edge_a); dfree(f.he_a); dfree(f.eflux); dfree(f.elam);
   dfree(f.b); dfree(f.dt); dfree(f.jdb); dfree(f.bhe); dfree(f.bcol); dfree(f.red); dfree(f.aux); dfree(f.edges); dfree(f.nptr);
-  dfree(f.nslot_d); dfree(f.he_ptr); dfree(f.he_id); dfree(f.he_tag); dfree(f.he_node); dfree(f.bc_type); dfree(f.bnd);
+  dfree(f.nslot_d); dfree(f.he_ptr); dfree(f.he_id); dfree(f.he_tag); dfree(f.he_node); dfree(f.he_seen); dfree(f.rst); dfree(f.bc_type); dfree(f.bnd);
   dfree(f.bidx); dfree(f.srow); dfree(f.swidth); dfree(f.sbase); dfree(f.scol); dfree(f.icount);
   dfree(f.piv); dfree(f.Md); dfree(f.Dd); dfree(f.xd); dfree(f.Mf); dfree(f.Df); dfree(f.xf); dfree(f.dmodel);
   dfree(f.s_rhoi); dfree(f.s_T); dfree(f.s_w); dfree(f.s_lst); dfree(f.s_cnt); dfree(f.s_off);
@@ -999,16 +987,15 @@ void send(pcfd_fr& f, int k) {
 constexpr int NS5 = 5;
 
 void run_hardset(pcfd_fr& f) {
-  if (!f.has_hardset) return;
-  hipLaunchKernelGGL(k_fr_hardset<NS5>, dim3(nblocks(f.nbnd)), dim3(kFB), 0, f.stream, f.nbnd, f.bnd, f.he_ptr,
-                     f.he_id, f.he_tag, f.bc_type, f.qref, f.q);
+  if (f.nrst == 0) return;
+  hipLaunchKernelGGL(k_fr_hardset<NS5>, dim3(nblocks(f.nrst)), dim3(kFB), 0, f.stream, f.nrst, f.rst, f.qref, f.q);
   hcheck(hipGetLastError(), "k_fr_hardset");
 }
 
 void run_bcs(pcfd_fr& f) {
   if (f.nbnd == 0) return;
   hipLaunchKernelGGL(k_fr_bcs<NS5>, dim3(nblocks(f.nbnode, kBB)), dim3(kBB), 0, f.stream, f.dmodel, f.nbnode,
-                     f.he_node, f.he_ptr, f.he_id, f.he_tag, f.he_a, f.bc_type, f.qref, f.nnode, f.prm.beta, f.q);
+                     f.he_node, f.he_seen, f.he_id, f.he_tag, f.he_a, f.bc_type, f.qref, f.nnode, f.prm.beta, f.q);
   hcheck(hipGetLastError(), "k_fr_bcs");
   run_hardset(f);
 }
@@ -1093,7 +1080,7 @@ void run_jacobian_t(pcfd_fr& f, TM* M, TM* D) {
   }
   if (f.nbnd > 0) {
     hipLaunchKernelGGL(k_fr_jac_bnd_base<NS5>, dim3(nblocks(f.nbnode, kBB)), dim3(kBB), 0, f.stream, f.dmodel,
-                       f.nbnode, f.he_node, f.he_ptr, f.he_id, f.he_tag, f.he_a, f.bc_type, f.qref, f.nnode,
+                       f.nbnode, f.he_node, f.he_seen, f.he_id, f.he_tag, f.he_a, f.bc_type, f.qref, f.nnode,
                        f.prm.beta, f.q, f.bhe);
     hcheck(hipGetLastError(), "k_fr_jac_bnd_base");
     run_hardset(f);
@@ -1344,14 +1331,21 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
         bnd.push_back(i);
       }
     f->nbnd = (int)bnd.size();
-    // node of each half-edge in list order
-    std::vector<int> he_node(nb);
-    for (int i = 0; i < nn; ++i)
-      for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) he_node[p] = i;
-    for (int h = 0; h < nb; ++h) {
-      const int ty = m->bc_type[m->bfactag[h]];
-      if (ty == fr::kSonicInflow || ty == fr::kDirichlet) f->has_hardset = true;
+    // in list order, each half-edge's node and the tag of the last half-edge
+    // before it that resets the node (-1: none); the nodes that are reset
+    std::vector<int> he_node(nb), he_seen(nb);
+    std::vector<int2> rst;
+    for (int i : bnd) {
+      int t = -1;
+      for (int p = he_ptr[i]; p < he_ptr[i + 1]; ++p) {
+        const int tag = m->bfactag[he_id[p]];
+        he_node[p] = i;
+        he_seen[p] = t;
+        if (resets_node(m->bc_type[tag])) t = tag;
+      }
+      if (t >= 0) rst.push_back(int2{i, t});
     }
+    f->nrst = (int)rst.size();
     // colouring and the SELL layout of the block matrix
     std::vector<int> colour(nn);
     const int ncol = pcfd_color_nodes(nn, ne, m->edges, colour.data());
@@ -1439,6 +1433,8 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
     dput(*f, &f->he_id, he_id);
     dput(*f, &f->he_tag, he_tag);
     dput(*f, &f->he_node, he_node);
+    dput(*f, &f->he_seen, he_seen);
+    dput(*f, &f->rst, rst);
     dput(*f, &f->bc_type, bct);
     dput(*f, &f->qref, qr);
     dput(*f, &f->bnd, bnd);
