@@ -44,9 +44,15 @@ void dzero(Ctx& c, T** p, size_t n) {
 // two host arrays in one device array: q points at the second
 template <typename T>
 void dput2(Ctx& c, T** p, T** q, const std::vector<T>& a, const std::vector<T>& b) {
-  std::vector<T> h(a);
-  h.insert(h.end(), b.begin(), b.end());
-  dput(c, p, h);
+  if (a.size() + b.size() <= (1 << 16)) {  // one copy
+    std::vector<T> h(a);
+    h.insert(h.end(), b.begin(), b.end());
+    dput(c, p, h);
+  } else {
+    dalloc(c, p, a.size() + b.size());
+    if (!a.empty()) PCFD_HIP(hipMemcpy(*p, a.data(), a.size() * sizeof(T), hipMemcpyHostToDevice));
+    if (!b.empty()) PCFD_HIP(hipMemcpy(*p + a.size(), b.data(), b.size() * sizeof(T), hipMemcpyHostToDevice));
+  }
   *q = *p + a.size();
 }
 
@@ -62,7 +68,7 @@ void free_all(Ctx& c) {
   if (c.pin) (void)hipHostFree(c.pin);
   c.pin = c.pin_dev = nullptr;
   dfree(d.he_ptr); dfree(d.he_id); dfree(d.he_tag); dfree(d.he_node); dfree(d.seen); dfree(d.he_desc); dfree(d.rst); dfree(d.he_a); dfree(d.bnd_nodes); dfree(d.bidx);
-  dfree(d.jdb); dfree(d.jhe); dfree(d.jqb); dfree(d.bc_type); dfree(d.twall); dfree(d.spos);
+  dfree(d.jdb); dfree(d.jqb); dfree(d.bc_type); dfree(d.twall); dfree(d.spos);
   dfree(d.qref); dfree(d.q); dfree(d.grad); dfree(d.lim); dfree(d.lim2); dfree(d.edges); dfree(d.clip_flag); dfree(d.clip_cnt);
   dfree(d.clip_off); dfree(d.clip_list); dfree(d.b); dfree(d.dt);
   dfree(d.srow); dfree(d.swidth); dfree(d.sbase); dfree(d.scol); dfree(d.Md); dfree(d.Mf); dfree(d.Dd);
@@ -173,11 +179,11 @@ void sgs_vectors(Ctx& c, T** xs, T** bs, T** ps, T** x) {
 }
 
 void ensure_matrix(Ctx& c) {
-  if (!c.d.jhe) {
-    dalloc(c, &c.d.jhe, 35 * (size_t)c.nbnode);
-    c.d.jcol = c.d.jhe + 10 * (size_t)c.nbnode;
-  }
-  const size_t off = (size_t)c.nslot_s * kW * 25, dg = (size_t)c.nchunk_s * kW * 25;
+  // the off-diagonal blocks' array first holds the boundary part's records and
+  // columns, 35 doubles a half-edge
+  const size_t s = c.prm.precision == PCFD_CHOSEN_FP32 ? 2 : 1;
+  const size_t off = std::max((size_t)c.nslot_s * kW * 25, 35 * s * (size_t)c.nbnode);
+  const size_t dg = (size_t)c.nchunk_s * kW * 25;
   if (c.prm.precision == PCFD_CHOSEN_FP32) {
     if (!c.d.Mf) dalloc(c, &c.d.Mf, off);
     if (!c.d.Df) dalloc(c, &c.d.Df, dg);

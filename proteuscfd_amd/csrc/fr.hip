@@ -887,14 +887,17 @@ struct pcfd_fr {
   long long bytes = 0;
   // device arrays
   double *q = nullptr, *qref = nullptr, *vol = nullptr, *edge_a = nullptr, *he_a = nullptr, *eflux = nullptr,
-         *elam = nullptr, *b = nullptr, *dt = nullptr, *jdb = nullptr, *bhe = nullptr, *bcol = nullptr, *red = nullptr, *aux = nullptr;
+         *elam = nullptr, *b = nullptr, *dt = nullptr, *jdb = nullptr, *red = nullptr, *aux = nullptr;
   int *edges = nullptr, *nptr = nullptr, *nslot_d = nullptr, *he_ptr = nullptr, *he_id = nullptr, *he_tag = nullptr, *he_node = nullptr, *he_seen = nullptr,
       *bc_type = nullptr, *bnd = nullptr, *bidx = nullptr, *srow = nullptr, *swidth = nullptr, *sbase = nullptr,
       *scol = nullptr, *sedge = nullptr, *icount = nullptr;
   int2* rst = nullptr;
   long long* piv = nullptr;
   double *ediag = nullptr, *nterm = nullptr;  // Jacobian diagonal parts: per edge side, per row
-  fr::Side* jst = nullptr;                    // and the nodes' plain and raised states' properties
+  // one after the other in nterm before the row terms: the properties of the
+  // nodes' plain and raised states; the half-edges' columns and records
+  fr::Side* jst = nullptr;
+  double *bcol = nullptr, *bhe = nullptr;
   double *Md = nullptr, *Dd = nullptr, *xd = nullptr;
   float *Mf = nullptr, *Df = nullptr, *xf = nullptr;
   // production-rate surrogate in the residual (null: exact rates)
@@ -921,6 +924,21 @@ void dput(pcfd_fr& f, T** p, const std::vector<T>& h) {
   if (!h.empty()) hcheck(hipMemcpy(*p, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice), "hipMemcpy");
 }
 
+// two host arrays in one device array: q points at the second
+template <typename T>
+void dput2(pcfd_fr& f, T** p, T** q, const std::vector<T>& a, const std::vector<T>& b) {
+  if (a.size() + b.size() <= (1 << 16)) {  // one copy
+    std::vector<T> h(a);
+    h.insert(h.end(), b.begin(), b.end());
+    dput(f, p, h);
+  } else {
+    dalloc(f, p, a.size() + b.size());
+    if (!a.empty()) hcheck(hipMemcpy(*p, a.data(), sizeof(T) * a.size(), hipMemcpyHostToDevice), "hipMemcpy");
+    if (!b.empty()) hcheck(hipMemcpy(*p + a.size(), b.data(), sizeof(T) * b.size(), hipMemcpyHostToDevice), "hipMemcpy");
+  }
+  *q = *p + a.size();
+}
+
 template <typename T>
 void dfree(T*& p) {
   if (p) (void)hipFree(p);
@@ -929,12 +947,12 @@ void dfree(T*& p) {
 
 void free_all(pcfd_fr& f) {
   dfree(f.q); dfree(f.qref); dfree(f.vol); dfree(f.edge_a); dfree(f.he_a); dfree(f.eflux); dfree(f.elam);
-  dfree(f.b); dfree(f.dt); dfree(f.jdb); dfree(f.bhe); dfree(f.bcol); dfree(f.red); dfree(f.aux); dfree(f.edges); dfree(f.nptr);
-  dfree(f.nslot_d); dfree(f.he_ptr); dfree(f.he_id); dfree(f.he_tag); dfree(f.he_node); dfree(f.he_seen); dfree(f.rst); dfree(f.bc_type); dfree(f.bnd);
+  dfree(f.b); dfree(f.dt); dfree(f.jdb); dfree(f.red); dfree(f.aux); dfree(f.edges); dfree(f.nptr);
+  dfree(f.nslot_d); dfree(f.he_ptr); dfree(f.he_id); dfree(f.he_tag); dfree(f.he_node); dfree(f.rst); dfree(f.bc_type); dfree(f.bnd);
   dfree(f.bidx); dfree(f.srow); dfree(f.swidth); dfree(f.sbase); dfree(f.scol); dfree(f.icount);
   dfree(f.piv); dfree(f.Md); dfree(f.Dd); dfree(f.xd); dfree(f.Mf); dfree(f.Df); dfree(f.xf); dfree(f.dmodel);
   dfree(f.s_rhoi); dfree(f.s_T); dfree(f.s_w); dfree(f.s_lst); dfree(f.s_cnt); dfree(f.s_off);
-  dfree(f.ediag); dfree(f.nterm); dfree(f.jst); dfree(f.sedge);
+  dfree(f.ediag); dfree(f.nterm);
   if (f.e0) (void)hipEventDestroy(f.e0);
   if (f.e1) (void)hipEventDestroy(f.e1);
   if (f.e2) (void)hipEventDestroy(f.e2);
@@ -1432,9 +1450,8 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
     dput(*f, &f->he_ptr, he_ptr);
     dput(*f, &f->he_id, he_id);
     dput(*f, &f->he_tag, he_tag);
-    dput(*f, &f->he_node, he_node);
-    dput(*f, &f->he_seen, he_seen);
-    dput(*f, &f->rst, rst);
+    dput2(*f, &f->he_node, &f->he_seen, he_node, he_seen);
+    if (f->nrst > 0) dput(*f, &f->rst, rst);
     dput(*f, &f->bc_type, bct);
     dput(*f, &f->qref, qr);
     dput(*f, &f->bnd, bnd);
@@ -1444,22 +1461,23 @@ int pcfd_fr_create(const pcfd_mesh_desc* m, pcfd_chem* chem, const double* qref,
     dput(*f, &f->srow, srow);
     dput(*f, &f->swidth, swidth);
     dput(*f, &f->sbase, sbase);
-    dput(*f, &f->scol, scol);
-    dput(*f, &f->sedge, sedge);
+    dput2(*f, &f->scol, &f->sedge, scol, sedge);
     dalloc(*f, &f->q, (size_t)f->ntot * NE);
     dalloc(*f, &f->eflux, (size_t)ne * NE);
     dalloc(*f, &f->elam, (size_t)ne);
     dalloc(*f, &f->b, (size_t)nn * NE);
     dalloc(*f, &f->dt, (size_t)nn);
     dalloc(*f, &f->jdb, (size_t)std::max(f->nbnd, 1) * NE2);
-    dalloc(*f, &f->bhe, (size_t)std::max(nb, 1) * 3 * NE);
-    dalloc(*f, &f->bcol, (size_t)std::max(nb, 1) * NE2);
     dalloc(*f, &f->red, (size_t)(NE + 1) * std::max(nblocks(nn), 256));
     dalloc(*f, &f->icount, 4);
     dalloc(*f, &f->piv, (size_t)f->nrow_pad);
     dalloc(*f, &f->ediag, 2 * (size_t)ne * NE2);
-    dalloc(*f, &f->nterm, (size_t)f->nrow_pad * (NE2 + ns * (ns + 1)));
-    dalloc(*f, &f->jst, (size_t)nn * (NE + 1));
+    static_assert(sizeof(fr::Side) == 4 * sizeof(double), "Side");
+    dalloc(*f, &f->nterm, std::max({(size_t)f->nrow_pad * (NE2 + ns * (ns + 1)), (size_t)nn * (NE + 1) * 4,
+                                    (size_t)nb * (NE2 + 3 * NE)}));
+    f->jst = reinterpret_cast<fr::Side*>(f->nterm);
+    f->bcol = f->nterm;
+    f->bhe = f->bcol + (size_t)nb * NE2;
     launch_zero(f->stream, f->q, 2 * (size_t)f->ntot * NE);
   } catch (const std::exception& e) {
     g_fr_create_err = e.what();

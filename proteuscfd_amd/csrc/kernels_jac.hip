@@ -458,13 +458,17 @@ static void jac_boundary(Ctx& c, const JacArgs& A, hipStream_t s) {
   if (c.nbnd == 0) return;
   launch_bnd_resets(c, s);
   const BndArgs B = bnd_args(c);
+  // per half-edge, until the rows fill the array: boundary state and unperturbed
+  // flux (10), the columns of the diagonal's boundary part (25)
+  double* const jhe = c.prm.precision == PCFD_CHOSEN_FP32 ? reinterpret_cast<double*>(c.d.Mf) : c.d.Md;
+  double* const jcol = jhe + 10 * (size_t)c.nbnode;
   hipLaunchKernelGGL(A.flux_alg ? k_jac_bnd_base<true> : k_jac_bnd_base<false>, dim3(nblk(c.nbnode, kBndBlock)),
-                     dim3(kBndBlock), 0, s, B, A.sym2d, A.bcentred, c.d.jhe);
+                     dim3(kBndBlock), 0, s, B, A.sym2d, A.bcentred, jhe);
   PCFD_HIP(hipGetLastError());
   hipLaunchKernelGGL(A.flux_alg ? k_jac_bnd_cols<true> : k_jac_bnd_cols<false>, dim3(nblk(5LL * c.nbnode, kBndBlock)),
-                     dim3(kBndBlock), 0, s, B, A.sym2d, A.bcentred, c.d.jhe, c.d.jcol);
+                     dim3(kBndBlock), 0, s, B, A.sym2d, A.bcentred, jhe, jcol);
   PCFD_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_jac_bnd_sum, dim3(nblk(25LL * c.nbnd)), dim3(kBlock), 0, s, B, c.d.jcol, c.d.jdb, c.d.jqb);
+  hipLaunchKernelGGL(k_jac_bnd_sum, dim3(nblk(25LL * c.nbnd)), dim3(kBlock), 0, s, B, jcol, c.d.jdb, c.d.jqb);
   PCFD_HIP(hipGetLastError());
 }
 
