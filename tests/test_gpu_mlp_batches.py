@@ -88,3 +88,24 @@ def test_calls_share_a_network():
             lo, _ = R.loss_grad(p, x[idx], t[idx])
             assert abs(hist[it] - lo) <= 2.0**-9 * lo, (batch, it)
     net.close()
+
+
+@pytest.mark.parametrize("steps", [1, 4095, 4096, 4097])
+def test_long_calls_keep_every_loss(steps):
+    """A step size that moves no weight: the losses of one call are those of calls of at most 1,000 steps that
+    draw on from where the one before stopped, to the bit, on both sides of the 4,096 losses a network keeps."""
+    from proteuscfd_amd import gpu
+
+    n, batch = 97, 3
+    net = gpu.MLP(seed=0)
+    net.params = R.init(5).astype(np.float32)
+    x, t = samples(n, 6)
+    whole = net.train(x, t, steps=steps, batch=batch, lr=1e-30, seed=8)
+    s, parts = 8, []
+    for k in range(0, steps, 1000):
+        m = min(1000, steps - k)
+        parts.append(net.train(x, t, steps=m, batch=batch, lr=1e-30, seed=s))
+        for _ in range(m * batch):
+            s = mix(s)
+    assert np.all(whole > 0) and np.array_equal(whole, np.concatenate(parts))
+    net.close()
